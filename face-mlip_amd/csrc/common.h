@@ -65,6 +65,46 @@ __device__ __forceinline__ v4f mfma_16x16x4(float a, float b, v4f c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
+// fp32 products on the bf16 matrix cores. x = h + m + l with h = bf16(x), m = bf16(x - h),
+// l = bf16(x - h - m), each rounded to nearest: the three limbs hold 24 bits of x, and
+// x w = xh wh + (xh wm + xm wh) + (xm wm + xh wl + xl wh) up to 2^-25 of |x w| at most, below one fp32
+// rounding. Six v_mfma_f32_32x32x16_bf16 do the work of sixteen 16x16x4 fp32 products of the same
+// shape in 192 cycles instead of 512 (register-only loops: 1300-1580 / 6 = 217-263 against 110-137
+// TFLOP/s), and with fp32 accumulation over fewer, longer dot products their sums are closer to
+// 64 bits (relative error of a K = 160 / 512 / 1024 sum 1.7e-7 / 3.4e-7 / 4.9e-7 against 2.2e-7 /
+// 4.0e-7 / 5.8e-7). Values past the largest bf16 (and infinities)
+// have a NaN limb.
+// Operand layouts (wave64): A[i][k], k = 8 (lane >> 5) + e in element e of lane i + 32 (k >> 3);
+// B[k][j] likewise by j; D[8 (r >> 2) + 4 (lane >> 5) + (r & 3)][lane & 31] in register r.
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+
+struct Split8 {                                              // eight consecutive k of one row, in limbs
+    v8bf h, m, l;
+};
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f){a, b}, v2bf));
+}
+__device__ __forceinline__ Split8 split8(v4f a, v4f b) {
+    v4u h, m, l;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        const float x0 = p < 2 ? a[2 * p] : b[2 * p - 4], x1 = p < 2 ? a[2 * p + 1] : b[2 * p - 3];
+        h[p] = bf16_pair(x0, x1);
+        const float r0 = x0 - __builtin_bit_cast(float, h[p] << 16);
+        const float r1 = x1 - __builtin_bit_cast(float, h[p] & 0xffff0000u);
+        m[p] = bf16_pair(r0, r1);
+        l[p] = bf16_pair(r0 - __builtin_bit_cast(float, m[p] << 16), r1 - __builtin_bit_cast(float, m[p] & 0xffff0000u));
+    }
+    return {__builtin_bit_cast(v8bf, h), __builtin_bit_cast(v8bf, m), __builtin_bit_cast(v8bf, l)};
+}
+__device__ __forceinline__ v16f mfma_32x32x16(v8bf a, v8bf b, v16f c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
 __device__ __forceinline__ v4f ld4(const float* p) { return *reinterpret_cast<const v4f*>(p); }
 
 // float4 read of an LDS image (16-byte aligned base) at a float offset that is a multiple of 4:

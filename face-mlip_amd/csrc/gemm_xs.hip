@@ -1,0 +1,6 @@
+// Row-block linear layers with a per-group input scale (rows_gemm.h, input mode 1).
+#include "rows_gemm.h"
+
+int face::launch_rows_xs(const RowsCtx& c, int NW, int NB, int xcd_order) {
+    return launch_rows_xm<1>(c, NW, NB, xcd_order);
+}

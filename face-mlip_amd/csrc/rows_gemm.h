@@ -1,0 +1,518 @@
+// Row-block linear layers of the node features on the matrix cores (gfx950), fp32 in and out:
+//
+//   y[m, :] = (beta y0[m, :] + (op(x)[m, :] * xs[m, :]) W^T + bias) * ys[m, :]    (per problem)
+//
+// for the tall activations of a pass, (k_l N, C) blocks against weights of at most a few
+// hundred columns: mix, tmix and proj (face/model.py:498-533, :537-544), the readout layers
+// (face/model.py:331-339) and their input gradients. xs / ys are per-atom scale rows picked by the
+// atom's element (the elem_scale factor of face/model.py:530-533) and are optional, as are beta and
+// bias. Up to eight problems share one launch.
+//
+// The products are six bf16 matrix products of the operands' three-way splits (common.h). A
+// workgroup of NW waves owns a tile of 32 NW rows and a slice of NSB = 32 NB output columns; each
+// wave keeps its 32 x NSB outputs in registers over the whole K loop. The x rows stream from memory
+// straight into the waves' A operands (lane i + 32 h holds columns 8 h .. 8 h + 7 of row i; a chunk of 32
+// columns is one 128-byte line per row), loaded one chunk ahead, scaled or transformed and split in
+// registers. The weight slice streams through LDS in chunks of 32 k, double-buffered, split once per
+// workgroup as it is staged and held in the order the B operands are read (one conflict-free
+// ds_read_b128 per limb and 32 columns); the loads of the next chunk are in flight during the current
+// one's products, one barrier per chunk. A slice streamed this way leaves room for two or more
+// workgroups per CU, whose prologues and stores hide under each other's products, and costs the same
+// for any K. D holds 32 columns of a row in 32 lanes: the stores are whole 128-byte lines.
+//
+// Every output is the same sequence of products whatever the tile, slice and grid, so results do
+// not depend on the launch shape or on the number of rows.
+#pragma once
+#include "common.h"
+
+namespace face {
+
+constexpr int kGemmRows = 32;                   // rows per wave
+constexpr int kGemmK = 32;                      // k per staged chunk
+constexpr int kGemmMaxProbs = 8;                // problems per launch
+constexpr int kGemmMaxGroups = 64;              // scale-table rows (elements)
+
+struct GemmProb {
+    const float* x;
+    int64_t ld_x, m;
+    const float* w;
+    int64_t ld_w;
+    float* y;
+    int64_t ld_y;
+    int n, k, s_off, slices;               // slices of 32 NB columns
+    float beta;
+    const float* x2;                       // input columns k >= k1 (column k - k1), or x
+    int64_t ld_x2;
+    int k1, x_op;                          // x_op on columns < k1: 0 none, 1 silu, 2 * silu'(xz)
+    const float* xz;
+    int64_t ld_xz;
+    const float* bias;
+    const float* y0;                       // initial sum beta * y0 (columns < n_y0), null: y
+    int64_t ld_y0;
+    int n_y0;
+    int64_t first_block;                   // first work item of this problem
+    int64_t w_off;                         // its split weights in the workspace (bytes)
+};
+
+// silu and its derivative with the hardware exp2 and reciprocal (about 1 ulp each)
+__device__ __forceinline__ float gemm_sigmoid(float x) {
+    return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.44269504088896341f * x));
+}
+__device__ __forceinline__ float gemm_op(float x, float z, int op) {
+    if (op == 1) return x * gemm_sigmoid(x);
+    if (op == 2) {                                                     // x * d silu(z) / dz
+        const float sg = gemm_sigmoid(z);
+        return x * (sg * (1.f + z * (1.f - sg)));
+    }
+    return x;
+}
+__device__ __forceinline__ v4f gemm_op4(v4f x, v4f z, int op) {
+    v4f o;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = gemm_op(x[r], z[r], op);
+    return o;
+}
+
+struct GemmArgs {
+    GemmProb p[kGemmMaxProbs];
+    int n_probs, w_kn;
+    const float *xs, *ys;
+    int any_bias;                          // some problem has a bias (side table present)
+    int ld_s, n_groups;
+    const int32_t* group;
+    int64_t period;
+    int kmax, side_lds;                    // largest K; the scale tables fit in LDS
+    int xcd_order;                         // items in XCD-contiguous ranges
+    const char* work;                      // split weights (PS kernels), else null
+};
+
+// A uniform base and a 32-bit byte offset per lane: one scalar address pair per access.
+__device__ __forceinline__ float* at_off(float* u, uint32_t bytes) {
+    return reinterpret_cast<float*>(reinterpret_cast<char*>(u) + bytes);
+}
+__device__ __forceinline__ const float* at_off(const float* u, uint32_t bytes) {
+    return reinterpret_cast<const float*>(reinterpret_cast<const char*>(u) + bytes);
+}
+__device__ __forceinline__ v4f ld4_off(const float* u, uint32_t bytes) { return ld4(at_off(u, bytes)); }
+
+// LDS after the two weight buffers: the row groups of every wave (32 ints each), then the scale rows of the slice's columns (ys) and of the problem's inputs (xs).
+static inline size_t gemm_lds(int NB, int NW, int64_t side_floats) {
+    return (size_t)2 * NB * 6144 + 4 * ((size_t)NW * kGemmRows + (size_t)side_floats);
+}
+
+// XM: input mode -- 0 plain, 1 the per-group x scale (xs), 2 split input, transform x_op or y0
+// PS: the weights come split from the workspace (split_weights_kernel)
+//
+// The loads ahead have no branches: past an edge (last chunk, last column, last row) they read the last
+// valid place again, whose products are not formed or not stored. (With guarded loads the compiler
+// waited for each before issuing the next.)
+template <int NB, int NW, int XM, bool PS>
+__global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(GemmArgs A) {
+    constexpr bool XS = XM == 1, XO = XM == 2;
+    constexpr int NSB = 32 * NB, NT = NW * kWave, BUF = NB * 6144;
+    constexpr int WI = (NSB * 4 + NT - 1) / NT;               // (column, 8 k) items per thread and chunk
+    constexpr int WU = PS ? (6 * NB + NW - 1) / NW : 2 * WI;  // 16-byte loads per thread and chunk
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    int* sgrp = reinterpret_cast<int*>(smem + 2 * BUF);
+    float* sys = reinterpret_cast<float*>(sgrp + NW * kGemmRows);
+    float* sxs = sys + (A.ys ? A.n_groups * NSB : 0);
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), j = lane & 31, hf = lane >> 5;
+    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+    // item -> (problem, row tile, column slice), slices fastest. In XCD order (workgroup b runs on
+    // XCD b % 8) each XCD takes a contiguous range, so the slices of a tile read its rows from one L2.
+    int it = blockIdx.x;
+    if (A.xcd_order) {
+        const int nbk = gridDim.x, xcd = it & 7, per = nbk >> 3, rem = nbk & 7;
+        it = xcd * per + min(xcd, rem) + (it >> 3);
+    }
+    int pi = 0;
+#pragma unroll 1
+    for (int k = 1; k < A.n_probs; ++k)
+        if (it >= A.p[k].first_block) pi = k;
+    const GemmProb& P = A.p[pi];
+    const int slices = P.slices, local = it - (int)P.first_block, tile = local / slices;
+    const int K = P.k, N = P.n, k1 = P.k1, x_op = XO ? P.x_op : 0;
+    const int n0 = (local - tile * slices) * NSB;
+    const int ns = min(NSB, N - n0);                          // a multiple of 16
+    const int ncb = (N + 31) >> 5;                            // 32-column blocks
+    const int64_t M = P.m, m0 = ((int64_t)tile * NW + wv) * kGemmRows;
+    const int64_t mb = min(m0, M - 1);                        // first row read (waves past m: the last row)
+    const int jr = (int)min((int64_t)j, M - 1 - mb);          // this lane's input row - mb
+    const int64_t ld_x = P.ld_x, ld_x2 = P.ld_x2, ld_xz = P.ld_xz;
+    const float *xb = P.x + mb * ld_x, *x2b = P.x2 + mb * ld_x2, *xzb = P.xz + mb * ld_xz;
+    const uint32_t xo = 4 * (uint32_t)(jr * (int)ld_x + 8 * hf), x2o = 4 * (uint32_t)(jr * (int)ld_x2 + 8 * hf);
+    const uint32_t xzo = 4 * (uint32_t)(jr * (int)ld_xz + 8 * hf);
+    const int grp = A.group ? A.group[(mb + jr) % A.period] : 0;
+    const float* wsrc = P.w;
+    const int64_t ld_w = P.ld_w;
+    const bool w_kn = A.w_kn != 0;
+    const char* wwork = PS ? A.work + P.w_off + (int64_t)(n0 >> 5) * 3072 : nullptr;
+    int woff[WU];                                             // of this wave's 1 KB pieces of a chunk
+#pragma unroll
+    for (int u = 0; u < WU; ++u) {
+        const int f = min(wv + u * NW, 6 * NB - 1), s = f >= 3 * NB;
+        woff[u] = s * ncb * 3072 + min(f - s * 3 * NB, 3 * (ncb - (n0 >> 5)) - 1) * 1024;
+    }
+
+    auto load_x = [&](int c, v4f (&xv)[4], v4f (&zv)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int k0 = min(kGemmK * c + 16 * s, K - 16);  // uniform
+            const bool second = XO && k0 >= k1;
+            const float* u = second ? x2b + (k0 - k1) : xb + k0;
+            const uint32_t o = second ? x2o : xo;
+            xv[2 * s] = ld4_off(u, o);
+            xv[2 * s + 1] = ld4_off(u, o + 16);
+            if (XO && x_op == 2 && !second) {
+                zv[2 * s] = ld4_off(xzb + k0, xzo);
+                zv[2 * s + 1] = ld4_off(xzb + k0, xzo + 16);
+            }
+        }
+    };
+    // weight item v of a chunk: 8 consecutive k (group kg) of one column; a wave's loads cover whole
+    // lines (4 groups of 16 columns, or 32 columns of 8 rows of a (k, n) weight)
+    auto item = [&](int u, int& col, int& kg) __attribute__((always_inline)) {
+        const int v = min(u * NT + tid, NSB * 4 - 1);
+        if (w_kn) col = 32 * (v >> 7) + (v & 31), kg = (v >> 5) & 3;
+        else col = 16 * (v >> 6) + (v & 15), kg = (v >> 4) & 3;
+    };
+    // LDS image of a chunk: [16-k step][column block][limb][64 lanes] of 16 bytes
+    auto load_w = [&](int c, v4f (&bw)[WU]) __attribute__((always_inline)) {
+        if (PS) {
+#pragma unroll
+            for (int u = 0; u < WU; ++u)
+                bw[u] = ld4_off(reinterpret_cast<const float*>(wwork + (int64_t)c * (ncb * 6144) + woff[u]), 16 * lane);
+        } else if (w_kn) {
+#pragma unroll
+            for (int u = 0; u < WI; ++u) {
+                int col, kg;
+                item(u, col, kg);
+                const float* p = wsrc + (int64_t)min(kGemmK * c + 8 * kg, K - 8) * ld_w + n0 + min(col, ns - 1);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) bw[2 * u][r] = p[r * ld_w];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) bw[2 * u + 1][r] = p[(r + 4) * ld_w];
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < WI; ++u) {
+                int col, kg;
+                item(u, col, kg);
+                const float* p = wsrc + (int64_t)(n0 + min(col, ns - 1)) * ld_w + min(kGemmK * c + 8 * kg, K - 8);
+                bw[2 * u] = ld4(p);
+                bw[2 * u + 1] = ld4(p + 4);
+            }
+        }
+    };
+    auto store_w = [&](int buf, const v4f (&bw)[WU]) __attribute__((always_inline)) {
+        if (PS) {
+#pragma unroll
+            for (int u = 0; u < WU; ++u)
+                st4(reinterpret_cast<float*>(smem + buf * BUF + min(wv + u * NW, 6 * NB - 1) * 1024) + 4 * lane, bw[u]);
+        } else {
+#pragma unroll
+            for (int u = 0; u < WI; ++u) {
+                int col, kg;
+                item(u, col, kg);
+                const Split8 w = split8(bw[2 * u], bw[2 * u + 1]);
+                v8bf* d = reinterpret_cast<v8bf*>(smem + buf * BUF + ((kg >> 1) * NB + (col >> 5)) * 3072) + (kg & 1) * 32 +
+                          (col & 31);
+                d[0] = w.h;
+                d[64] = w.m;
+                d[128] = w.l;
+            }
+        }
+    };
+
+    v4f xn[4], zn[4], bw[WU];
+    load_w(0, bw);
+    load_x(0, xn, zn);
+    if (hf == 0) sgrp[wv * kGemmRows + j] = grp;
+    if (A.side_lds && A.ys) {
+        for (int v = tid; v < A.n_groups * NSB; v += NT) {
+            const int g = v / NSB, c = v - g * NSB;
+            sys[v] = A.ys[(int64_t)g * A.ld_s + P.s_off + n0 + min(c, ns - 1)];
+        }
+    }
+    if (XS && A.side_lds) {
+        for (int v = tid; v < A.n_groups * K; v += NT) {
+            const int g = v / K, k = v - g * K;
+            sxs[g * A.kmax + k] = A.xs[(int64_t)g * A.ld_s + P.s_off + k];
+        }
+    }
+    store_w(0, bw);
+    // output element (row 8 (r >> 2) + 4 hf + (r & 3), column 32 nb + j) of the wave: a uniform base per
+    // (r, nb) and one byte offset per lane
+    const int64_t ld_y = P.ld_y;
+    float* yb = P.y + m0 * ld_y + n0;
+    const uint32_t yo = 4 * (uint32_t)(4 * hf * (int)ld_y + j);
+    const bool full = m0 + kGemmRows <= M;
+    auto row_ok = [&](int r) __attribute__((always_inline)) { return m0 + 8 * (r >> 2) + (r & 3) + 4 * hf < M; };
+    // accumulators start at beta y0, else zero
+    v16f acc[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[nb][r] = 0.f;
+    const float beta = P.beta;
+    if (beta != 0.f) {
+        const float* y0 = P.y0 ? P.y0 : P.y;
+        const int64_t ld0 = P.y0 ? P.ld_y0 : ld_y;
+        const float* y0b = y0 + m0 * ld0 + n0;
+        const uint32_t o0 = 4 * (uint32_t)(4 * hf * (int)ld0 + j);
+        const int n_y0 = min(P.n_y0 - n0, ns);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            if (full && 32 * nb + 32 <= n_y0) {               // uniform
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[nb][r] = *at_off(y0b + (8 * (r >> 2) + (r & 3)) * ld0 + 32 * nb, o0);
+            } else if (32 * nb < n_y0 && m0 < M) {
+                const int64_t c = min(32 * nb + j, n_y0 - 1);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {                // at the nearest valid place, zero outside
+                    const int64_t rr = min(m0 + 8 * (r >> 2) + (r & 3) + 4 * hf, M - 1);
+                    const float v = y0[rr * ld0 + n0 + c];
+                    acc[nb][r] = (32 * nb + j < n_y0 && row_ok(r)) ? v : 0.f;
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[nb][r] *= beta;
+        }
+    }
+    __syncthreads();
+    const int nchunk = (K + kGemmK - 1) / kGemmK;
+#pragma unroll 1
+    for (int c = 0; c < nchunk; ++c) {
+        const int buf = c & 1, cn = min(c + 1, nchunk - 1);
+        load_w(cn, bw);
+        Split8 xq[2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int k0 = min(kGemmK * c + 16 * s, K - 16);
+            v4f a = xn[2 * s], b = xn[2 * s + 1];
+            if (XS) {
+                if (A.side_lds) {
+                    a *= lds4_at(sxs, grp * A.kmax + k0 + 8 * hf);
+                    b *= lds4_at(sxs, grp * A.kmax + k0 + 8 * hf + 4);
+                } else {
+                    const float* t = A.xs + (int64_t)grp * A.ld_s + P.s_off + k0 + 8 * hf;
+                    a *= ld4(t);
+                    b *= ld4(t + 4);
+                }
+            }
+            if (XO && x_op && k0 < k1) {
+                a = gemm_op4(a, zn[2 * s], x_op);
+                b = gemm_op4(b, zn[2 * s + 1], x_op);
+            }
+            xq[s] = split8(a, b);
+        }
+        load_x(cn, xn, zn);
+        __builtin_amdgcn_sched_barrier(0);                    // the loads ahead are issued before the products
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            if (s && kGemmK * c + 16 >= K) break;
+            const v8bf* wf = reinterpret_cast<const v8bf*>(smem + buf * BUF + s * NB * 3072) + lane;
+            const Split8& x = xq[s];
+            // the limbs of the next column block are read ahead; the smallest products first
+            v8bf w[3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) w[q] = wf[q * 64];
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                v8bf wn[3];
+#pragma unroll
+                for (int q = 0; q < 3; ++q) wn[q] = nb + 1 < NB ? wf[(nb + 1) * 192 + q * 64] : w[q];
+                acc[nb] = mfma_32x32x16(x.l, w[0], acc[nb]);
+                acc[nb] = mfma_32x32x16(x.h, w[2], acc[nb]);
+                acc[nb] = mfma_32x32x16(x.m, w[1], acc[nb]);
+                acc[nb] = mfma_32x32x16(x.m, w[0], acc[nb]);
+                acc[nb] = mfma_32x32x16(x.h, w[1], acc[nb]);
+                acc[nb] = mfma_32x32x16(x.h, w[0], acc[nb]);
+#pragma unroll
+                for (int q = 0; q < 3; ++q) w[q] = wn[q];
+            }
+            // issue order: the reads of blocks 0 and 1, then per block its products and the reads of the
+            // block after the next one
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                if (nb == 0) __builtin_amdgcn_sched_group_barrier(0x100, NB > 1 ? 6 : 3, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
+                if (nb + 2 < NB) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+            }
+        }
+        store_w(buf ^ 1, bw);
+        __syncthreads();
+    }
+    // Operands that round to a bf16 infinity have a NaN limb, which every product they enter carries into
+    // the sums: a wave with a sum that is not finite forms its rows again in plain fp32 products.
+    float chk = 0.f;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) chk = fmaf(acc[nb][r], 0.f, chk);
+    if (__any(chk != chk)) {
+#pragma unroll 1
+        for (int i = 0; i < kGemmRows; ++i) {
+            const int64_t r = m0 + i;
+            if (r >= M) break;
+            const int64_t g = A.group ? A.group[r % A.period] : 0;
+#pragma unroll 1
+            for (int c = lane; c < ns; c += kWave) {
+                float s = 0.f;
+                if (beta != 0.f && n0 + c < P.n_y0)
+                    s = beta * (P.y0 ? P.y0[r * P.ld_y0 + n0 + c] : P.y[r * ld_y + n0 + c]);
+#pragma unroll 1
+                for (int k = 0; k < K; ++k) {
+                    float x = k < k1 ? P.x[r * ld_x + k] : P.x2[r * ld_x2 + k - k1];
+                    if (XS) x *= A.xs[g * A.ld_s + P.s_off + k];
+                    if (XO && k < k1) x = gemm_op(x, x_op == 2 ? P.xz[r * ld_xz + k] : 0.f, x_op);
+                    s = fmaf(x, w_kn ? wsrc[(int64_t)k * ld_w + n0 + c] : wsrc[(int64_t)(n0 + c) * ld_w + k], s);
+                }
+                if (P.bias) s += P.bias[n0 + c];
+                if (A.ys) s *= A.ys[g * A.ld_s + P.s_off + n0 + c];
+                P.y[r * ld_y + n0 + c] = s;
+            }
+        }
+        return;
+    }
+    // epilogue: bias and y scale, then stores of 128 bytes per row
+    if (P.bias) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            const float b = P.bias[n0 + min(32 * nb + j, ns - 1)];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[nb][r] += b;
+        }
+    }
+    if (A.ys) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int g = sgrp[wv * kGemmRows + 8 * (r >> 2) + 4 * hf + (r & 3)];
+            if (A.side_lds) {
+                const float* t = sys + g * NSB + j;
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) acc[nb][r] *= t[32 * nb];
+            } else {
+                const float* t = A.ys + (int64_t)g * A.ld_s + P.s_off + n0;
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) acc[nb][r] *= t[min(32 * nb + j, ns - 1)];
+            }
+        }
+    }
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+        if (full && 32 * nb + 32 <= ns) {                     // uniform
+#pragma unroll
+            for (int r = 0; r < 16; ++r) *at_off(yb + (8 * (r >> 2) + (r & 3)) * ld_y + 32 * nb, yo) = acc[nb][r];
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (32 * nb + j < ns && row_ok(r)) *at_off(yb + (8 * (r >> 2) + (r & 3)) * ld_y + 32 * nb, yo) = acc[nb][r];
+        }
+    }
+}
+
+// Splits the weights of a launch once: one wave per 16 k x 32 columns writes the three limbs in the
+// order of the LDS image, [16-k step][column block][limb][64 lanes] of 16 bytes, zeros past the last
+// column and step (an even number of steps). Launched before rows_gemm_kernel where many row tiles would each split them again.
+__global__ __launch_bounds__(kWave) inline void split_weights_kernel(GemmArgs A, char* work) {
+    int pi = 0;
+    const int64_t it = blockIdx.x;
+#pragma unroll 1
+    for (int k = 1; k < A.n_probs; ++k)
+        if (it >= A.p[k].first_block) pi = k;
+    const GemmProb& P = A.p[pi];
+    const int lane = threadIdx.x, ncb = (P.n + 31) >> 5;
+    const int64_t local = it - P.first_block;
+    const int step = (int)(local / ncb), cb = (int)(local - (int64_t)step * ncb);
+    const int col = 32 * cb + (lane & 31), k = 16 * step + 8 * (lane >> 5);
+    v4f a = {0.f, 0.f, 0.f, 0.f}, b = a;
+    if (col < P.n && k < P.k) {
+        if (A.w_kn) {
+            const float* p = P.w + (int64_t)k * P.ld_w + col;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) a[r] = p[r * P.ld_w], b[r] = p[(r + 4) * P.ld_w];
+        } else {
+            const float* p = P.w + (int64_t)col * P.ld_w + k;
+            a = ld4(p);
+            b = ld4(p + 4);
+        }
+    }
+    const Split8 w = split8(a, b);
+    v8bf* d = reinterpret_cast<v8bf*>(work + P.w_off + local * 3072) + lane;
+    d[0] = w.h;
+    d[64] = w.m;
+    d[128] = w.l;
+}
+
+// Everything a launch needs but its shape.
+struct RowsCtx {
+    GemmArgs A;                                  // problems filled, tiling not yet
+    const face_lin_problem* probs;
+    int n_probs, K, n_widest, max_lds, n_cu, n_groups;
+    bool x_scale, y_scale, any_ext;
+    char* work;                                  // workspace for split weights, or null
+    hipStream_t st;
+};
+
+// One launch of rows_gemm_kernel with NW waves per workgroup and NB column blocks of 32 per wave;
+// FACE_ERR_UNSUPPORTED, before anything is launched, if there is no such kernel.
+template <int XM>
+static int launch_rows_xm(const RowsCtx& c, int NW, int NB, int xcd_order) {
+    if (NB < 1 || NB > 16) return FACE_ERR_UNSUPPORTED;
+    GemmArgs A = c.A;
+    A.xcd_order = xcd_order;
+    A.work = c.work;
+    int64_t blocks = 0;
+    for (int i = 0; i < c.n_probs; ++i) {
+        const face_lin_problem& s = c.probs[i];
+        GemmProb& p = A.p[i];
+        p.slices = (s.n + 32 * NB - 1) / (32 * NB);
+        p.first_block = blocks;
+        blocks += (s.m + kGemmRows * NW - 1) / (kGemmRows * NW) * p.slices;
+    }
+    if (blocks == 0) return 0;
+    if (blocks > INT32_MAX) return FACE_ERR_UNSUPPORTED;
+    const int64_t side = (c.y_scale ? (int64_t)c.n_groups * 32 * NB : 0) + (c.x_scale ? (int64_t)c.n_groups * c.K : 0);
+    A.side_lds = gemm_lds(NB, NW, side) <= (size_t)c.max_lds;
+    const size_t lds = gemm_lds(NB, NW, A.side_lds ? side : 0);
+    auto go = [&](auto kern) -> int {
+        if (lds > 65536 &&
+            hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+            return FACE_ERR_UNSUPPORTED;
+        hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * kWave), lds, c.st, A);
+        FACE_LAUNCH_CHECK();
+        return 0;
+    };
+    if (c.work) {
+        switch (NB) {
+            case 2: return NW == 4 ? go(rows_gemm_kernel<2, 4, XM, true>) : FACE_ERR_UNSUPPORTED;
+            case 3: return NW == 4 ? go(rows_gemm_kernel<3, 4, XM, true>) : FACE_ERR_UNSUPPORTED;
+            case 4: return NW == 4 ? go(rows_gemm_kernel<4, 4, XM, true>) : FACE_ERR_UNSUPPORTED;
+            case 5: return NW == 4 ? go(rows_gemm_kernel<5, 4, XM, true>) : FACE_ERR_UNSUPPORTED;
+            case 6: return NW == 4 ? go(rows_gemm_kernel<6, 4, XM, true>) : FACE_ERR_UNSUPPORTED;
+            case 8: return NW == 8 ? go(rows_gemm_kernel<8, 8, XM, true>) : FACE_ERR_UNSUPPORTED;
+            default: return FACE_ERR_UNSUPPORTED;
+        }
+    }
+    switch (NW == 4 || NW == 8 ? 16 * NW + NB : 0) {
+        case 65: return go(rows_gemm_kernel<1, 4, XM, false>);
+        case 66: return go(rows_gemm_kernel<2, 4, XM, false>);
+        case 67: return go(rows_gemm_kernel<3, 4, XM, false>);
+        case 68: return go(rows_gemm_kernel<4, 4, XM, false>);
+        case 69: return go(rows_gemm_kernel<5, 4, XM, false>);
+        case 129: return go(rows_gemm_kernel<1, 8, XM, false>);
+        case 130: return go(rows_gemm_kernel<2, 8, XM, false>);
+        case 131: return go(rows_gemm_kernel<3, 8, XM, false>);
+        case 132: return go(rows_gemm_kernel<4, 8, XM, false>);
+        case 133: return go(rows_gemm_kernel<5, 8, XM, false>);
+        default: return FACE_ERR_UNSUPPORTED;
+    }
+}
+
+// The three input modes' launches, one translation unit each (gemm.hip, gemm_xs.hip, gemm_op.hip).
+int launch_rows_plain(const RowsCtx& c, int NW, int NB, int xcd_order);
+int launch_rows_xs(const RowsCtx& c, int NW, int NB, int xcd_order);
+int launch_rows_op(const RowsCtx& c, int NW, int NB, int xcd_order);
+
+}  // namespace face

@@ -1358,9 +1358,11 @@ def rows_linear(probs, w_kn=False, bias=None, xs=None, ys=None, group=None, peri
     tab = xs if xs is not None else ys
     if xs is not None and ys is not None and xs.shape[0] != ys.shape[0]:
         raise ValueError("rows_linear: xs and ys must have the same number of groups")
-    call("face_rows_linear", arr, len(probs), 1 if w_kn else 0, ptr(xs), ptr(ys),
+    need = _lib.lib().face_rows_linear_work(arr, len(probs))
+    work = torch.empty(need, dtype=torch.uint8, device=ref.device) if need else None
+    call("face_rows_linear_ws", arr, len(probs), 1 if w_kn else 0, ptr(xs), ptr(ys),
          0 if tab is None else tab.stride(0), 0 if tab is None else tab.shape[0], ptr(group), int(period),
-         _lib.stream_of(ref), label=label)
+         ptr(work), need, _lib.stream_of(ref), label=label)
 
 
 # mix and transport-mix backward in one launch up to this many atoms (launch-bound sizes; at

@@ -413,6 +413,15 @@ typedef struct {
 int face_rows_linear(const face_lin_problem* probs, int32_t n_probs, int32_t w_kn, const float* x_scale,
                      const float* y_scale, int32_t ld_scale, int32_t n_groups, const int32_t* group, int64_t period,
                      void* stream);
+/* The same with a workspace for the weights in the form the matrix cores take (split once per call
+ * by a launch of its own instead of by every row tile): work, 256-byte aligned, work_bytes of at
+ * least face_rows_linear_work(probs, n_probs), free for reuse on `stream` after the call; NULL is
+ * face_rows_linear. Results are bitwise the same. face_rows_linear_work gives 0 where splitting
+ * ahead does not pay (few rows): pass NULL then. */
+int64_t face_rows_linear_work(const face_lin_problem* probs, int32_t n_probs);
+int face_rows_linear_ws(const face_lin_problem* probs, int32_t n_probs, int32_t w_kn, const float* x_scale,
+                        const float* y_scale, int32_t ld_scale, int32_t n_groups, const int32_t* group, int64_t period,
+                        void* work, int64_t work_bytes, void* stream);
 
 /* ---------------------------------------------------------------- per-edge linear layers
  * Forward: y (E, ld_y) = x (E, ld_x) w^T + b + tab[idx[e]], w (F, K) row-major, b (F) and tab

@@ -1022,6 +1022,99 @@ def test_rows_linear_every_launch_shape_gives_bitwise_equal_rows(case, monkeypat
     assert ran >= 24
 
 
+def _rows_launch(x, w, y, w_kn, ahead, beta=0.0, xs=None, ys=None, grp=None, s_off=0):
+    """face_rows_linear_ws with the weights split in the kernel (ahead False) or ahead into a
+    workspace sized here from the header's rule, whatever face_rows_linear_work suggests."""
+    from face_amd import _lib
+    arr = (_lib.LinProblem * 1)(_lib.LinProblem(x.data_ptr(), x.stride(0), x.shape[0], w.data_ptr(), w.stride(0),
+                                                y.data_ptr(), y.stride(0), y.shape[1], x.shape[1], s_off, beta, None, 0,
+                                                x.shape[1], 0, None, 0, None, None, 0, 0, 0))
+    need = -(-x.shape[1] // 32) * 2 * -(-y.shape[1] // 32) * 3072 if ahead else 0
+    work = torch.empty(need, dtype=torch.uint8, device=DEV) if ahead else None
+    tab = xs if xs is not None else ys
+    _lib.call("face_rows_linear_ws", arr, 1, 1 if w_kn else 0, _lib.ptr(xs), _lib.ptr(ys),
+              0 if tab is None else tab.stride(0), 0 if tab is None else tab.shape[0], _lib.ptr(grp),
+              0 if grp is None else grp.shape[0], _lib.ptr(work), need, _lib.stream_of(y))
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("w_kn", [False, True])
+@pytest.mark.parametrize("m,n,k", [(1, 16, 16), (31, 48, 16), (33, 32, 48), (127, 176, 32), (129, 144, 80), (300, 304, 160),
+                                   (64, 528, 112)])
+def test_rows_linear_edges_and_weights_split_ahead(m, n, k, w_kn):
+    """Edges of the 32-row, 32-column and 32-k blocks (odd 16-column blocks of n and k, one row to one
+    past a tile), accumulating onto y, with the weights split in the kernel and ahead: the same bits,
+    and within float32 of torch fp64 (2^-22 |x| |w| per product, k of them, covers the three-way split
+    and the float32 sums)."""
+    say("rows_linear edges", m, n, k, w_kn)
+    torch.manual_seed(m + n + k)
+    x = torch.randn(m, k + 4, device=DEV)[:, :k]
+    w = torch.randn(k, n + 4, device=DEV)[:, :n] if w_kn else torch.randn(n, k + 4, device=DEV)[:, :k]
+    y0 = torch.randn(m, n + 8, device=DEV)
+    outs = []
+    for ahead in (False, True):
+        y = y0.clone()
+        _rows_launch(x, w, y[:, :n], w_kn, ahead, beta=0.5)
+        assert torch.equal(y[:, n:], y0[:, n:])                      # nothing past the last column
+        outs.append(y[:, :n])
+    assert torch.equal(outs[0], outs[1])
+    wd = w.double() if w_kn else w.double().t().contiguous()
+    ref = 0.5 * y0[:, :n].double() + x.double().contiguous() @ wd.contiguous()
+    bound = 2.0 ** -22 * (x.double().abs().contiguous() @ wd.abs().contiguous() + y0[:, :n].double().abs())
+    assert bool(((outs[0].double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("ahead", [False, True])
+@pytest.mark.parametrize("where", ["x", "w"])
+def test_rows_linear_values_past_bf16(where, ahead):
+    """Operands that round to a bf16 infinity (3.4e38), infinities and NaN: the results are those of
+    plain float32 products, and those of other 32-row tiles keep their bits."""
+    say("rows_linear past bf16", where, ahead)
+    torch.manual_seed(3)
+    m, n, k = 200, 96, 64
+    x, w = torch.randn(m, k, device=DEV), torch.randn(n, k, device=DEV)
+    w[:, 1] = w[:, 1].abs() + 0.5                                    # a definite sign against the infinity
+    plain = torch.empty(m, n, device=DEV)
+    _rows_launch(x, w, plain, False, ahead)
+    big = x.clone() if where == "x" else w.clone()
+    big[5, 0], big[70, 1], big[70, 2], big[80, 3] = 3.4e38, float("inf"), 1e30, float("nan")
+    small = w if where == "x" else x
+    small[:, 0] = small[:, 0].clamp(-0.5, 0.5)                       # 3.4e38 * 0.5 stays finite
+    if where == "w":
+        small[:, 1] = small[:, 1].abs() + 0.5
+    _rows_launch(x, w, plain, False, ahead)
+    out = torch.empty(m, n, device=DEV)
+    _rows_launch(big if where == "x" else x, big if where == "w" else w, out, False, ahead)
+    if where == "w":
+        plain, out = plain.t(), out.t()
+    ref = (big.double() @ small.double().t().contiguous())
+    touched = torch.zeros(out.shape[0], dtype=torch.bool, device=DEV)
+    touched[[5, 70, 80]] = True
+    if where == "x":
+        assert torch.equal(out[32:64], plain[32:64]) and torch.equal(out[96:], plain[96:])
+    rest = ref[~touched]
+    assert (out[~touched].double() - rest).abs().max() <= 1e-5 * rest.abs().max()
+    assert bool((out[70] == float("inf")).all()) and bool(torch.isnan(out[80]).all())
+    assert (out[5].double() - ref[5]).abs().max() <= 1e-6 * ref[5].abs().max()
+
+
+@pytest.mark.parametrize("side", ["xs", "ys"])
+def test_rows_linear_scale_tables_larger_than_lds(side):
+    """64 groups whose scale rows do not fit in LDS beside the weights: read from memory instead, the
+    results of a launch whose tables fit."""
+    say("rows_linear wide scale tables", side)
+    torch.manual_seed(4)
+    N, k, n = 500, 768, 512
+    x, w = torch.randn(N, k, device=DEV), torch.randn(n, k, device=DEV) / k ** 0.5
+    tab = torch.rand(64, 1024, device=DEV) + 0.5
+    grp = torch.randint(0, 64, (N,), device=DEV, dtype=torch.int32)
+    kw = {side: tab}
+    y = torch.empty(N, n, device=DEV)
+    _rows_launch(x, w, y, False, False, grp=grp, **kw)
+    ref = _lin_ref(x, w, False, None, 0.0, None, kw.get("xs"), kw.get("ys"), grp, N, 0)
+    assert rel(y, ref) < 1e-5
+
+
 @pytest.mark.parametrize("kc", [None, "1"])
 @pytest.mark.parametrize("w_kn", [False, True])
 def test_rows_linear_split_input_transforms_and_initial_sum(w_kn, kc, monkeypatch):
