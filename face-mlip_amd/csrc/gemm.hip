@@ -8,9 +8,7 @@
 
 namespace face {
 
-int launch_rows_plain(const RowsCtx& c, int NW, int NB, int xcd_order) {
-    return launch_rows_xm<0>(c, NW, NB, xcd_order);
-}
+int launch_rows_plain(const RowsCtx& c, RowsShape S) { return launch_rows_xm<0>(c, S); }
 
 static bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
@@ -21,11 +19,13 @@ using namespace face;
 // Validate problem s and fill p (everything but the tiling); 0 or a FACE_ERR_* status.
 static int fill_prob(const face_lin_problem& s, int w_kn, bool scaled, const float* x_scale, const float* y_scale,
                      int ld_scale, GemmProb& p) {
-    if (s.m < 0 || s.n < 16 || s.n % 16 || s.k < 16 || s.k % 16 || s.ld_y < s.n || s.ld_w < (w_kn ? s.n : s.k))
+    if (s.m < 0 || s.n < 16 || s.n % 16 || s.k < 16 || s.k % 16 || s.ld_y < s.n || s.ld_w < (w_kn ? s.n : (s.w2 ? s.k1 : s.k)))
         return FACE_ERR_ARG;
     const int k1 = s.x2 ? s.k1 : s.k;
     if (k1 < 0 || k1 > s.k || k1 % 16 || s.ld_x < k1 || (s.x2 && s.ld_x2 < s.k - k1)) return FACE_ERR_ARG;
     if (s.x_op < 0 || s.x_op > 2 || (s.x_op == 2 && (!s.xz || s.ld_xz < k1)) || (s.x_op && x_scale)) return FACE_ERR_ARG;
+    if (s.w2 && (!s.x2 || s.ld_w2 < (w_kn ? s.n : s.k - k1))) return FACE_ERR_ARG;
+    if (s.bias_row && !s.bias) return FACE_ERR_ARG;
     if (s.y0 && (s.n_y0 < 0 || s.n_y0 > s.n || s.n_y0 % 4 || s.ld_y0 < s.n_y0)) return FACE_ERR_ARG;
     if (scaled && (s.s_off < 0 || s.s_off % 4 || s.s_off + (x_scale ? s.k : 0) > ld_scale ||
                    s.s_off + (y_scale ? s.n : 0) > ld_scale))
@@ -37,6 +37,7 @@ static int fill_prob(const face_lin_problem& s, int w_kn, bool scaled, const flo
         (s.x_op == 2 && s.m * s.ld_xz >= lim) || (s.y0 && s.m * s.ld_y0 >= lim))
         return FACE_ERR_UNSUPPORTED;
     if (s.ld_x % 4 || s.ld_y % 4 || !al16(s.x) || !al16(s.y) || (!w_kn && (!al16(s.w) || s.ld_w % 4)) ||
+        (s.w2 && !w_kn && (!al16(s.w2) || s.ld_w2 % 4)) ||
         (s.x2 && (!al16(s.x2) || s.ld_x2 % 4)) || (s.x_op == 2 && (!al16(s.xz) || s.ld_xz % 4)) ||
         (s.bias && !al16(s.bias)) || (s.y0 && (!al16(s.y0) || s.ld_y0 % 4)))
         return FACE_ERR_UNSUPPORTED;
@@ -44,15 +45,16 @@ static int fill_prob(const face_lin_problem& s, int w_kn, bool scaled, const flo
     p.k = s.k, p.s_off = s.s_off, p.beta = s.beta;
     p.x2 = s.x2 ? s.x2 : s.x, p.ld_x2 = s.x2 ? s.ld_x2 : s.ld_x, p.k1 = k1;
     p.x_op = s.x_op, p.xz = s.x_op == 2 ? s.xz : s.x, p.ld_xz = s.x_op == 2 ? s.ld_xz : s.ld_x;
-    p.bias = s.bias;
+    p.w2 = s.w2 ? s.w2 : (w_kn ? s.w + (int64_t)k1 * s.ld_w : s.w + k1), p.ld_w2 = s.w2 ? s.ld_w2 : s.ld_w;
+    p.bias = s.bias, p.bias_row = s.bias_row;
     p.y0 = s.y0, p.ld_y0 = s.y0 ? s.ld_y0 : 0, p.n_y0 = s.y0 ? s.n_y0 : s.n;
     return 0;
 }
 
-static int launch_rows(const RowsCtx& c, int NW, int NB, int xcd_order) {
-    if (c.x_scale) return launch_rows_xs(c, NW, NB, xcd_order);
-    if (c.any_ext) return launch_rows_op(c, NW, NB, xcd_order);
-    return launch_rows_plain(c, NW, NB, xcd_order);
+static int launch_rows(const RowsCtx& c, RowsShape S) {
+    if (c.x_scale) return launch_rows_xs(c, S);
+    if (c.any_op) return launch_rows_op(c, S);
+    return c.any_ext ? launch_rows_split(c, S) : launch_rows_plain(c, S);
 }
 
 // Launch shape by size: the block count NB with the least estimated time. A workgroup's time is taken
@@ -67,7 +69,18 @@ static int launch_rows(const RowsCtx& c, int NW, int NB, int xcd_order) {
 // 160 -> 512: 267 against 276 us); else four (the same launch of 160 columns: 212 against 218 us).
 // The XCD order pays only where several slices share rows (proj 668 against 680 us; K = 480 -> 160 of
 // one slice 419 against 364 us: the plain order spreads neighbouring rows over the XCDs' channels).
-static void rows_shape(const RowsCtx& c, int& NW, int& NB, int& xcd) {
+// The direct kernel (K in four parts) takes launches of at most one workgroup per CU: 21 atoms, 512 -> 96
+// 8.9 against 16.4 us staged, 192 -> 192 5.2 against 7.5; 1,344 rows of 864 -> 192 (252 workgroups) 11.5
+// against 22, but 3,000 rows (564) 27 against 22. Two column blocks per wave where that brings a launch
+// of long K under the limit (4,000 rows of 512 -> 96: 13.3 against 16.6).
+static RowsShape rows_shape(const RowsCtx& c) {
+    int NW = 4, NB = 2;
+    for (int nb = 1; nb <= (c.K >= 384 ? 2 : 1) && !c.work; ++nb) {
+        int64_t w = 0;
+        for (int k = 0; k < c.n_probs; ++k)
+            w += (c.probs[k].m + kGemmRows - 1) / kGemmRows * ((c.probs[k].n + 32 * nb - 1) / (32 * nb));
+        if (w <= c.n_cu) return {4, nb, 0, 4};
+    }
     static constexpr int kSplitAhead[] = {8, 6, 5, 4, 3, 2}, kInKernel[] = {5, 4, 3, 2, 1};
     double best = 1e300;
     for (int i = 0; i < (c.work ? 6 : 5); ++i) {
@@ -90,7 +103,7 @@ static void rows_shape(const RowsCtx& c, int& NW, int& NB, int& xcd) {
             w8 += (c.probs[k].m + kGemmRows * 8 - 1) / (kGemmRows * 8) * ((c.probs[k].n + 32 * NB - 1) / (32 * NB));
         if (w8 >= 2 * c.n_cu) NW = 8;
     }
-    xcd = c.n_widest > 32 * NB;
+    return {NW, NB, c.n_widest > 32 * NB, 0};
 }
 
 // Workspace: the limbs of every problem, 3 KB per 16 k x 32 columns, for an even number of 16-k steps.
@@ -129,13 +142,14 @@ extern "C" int face_rows_linear_ws(const face_lin_problem* probs, int32_t n_prob
                                 int64_t period, void* work, int64_t work_bytes, void* stream) {
     if (!probs || n_probs < 1 || n_probs > kGemmMaxProbs) return FACE_ERR_ARG;
     int K = 16, n_widest = 16;
-    bool any_bias = false, any_ext = false;
+    bool any_bias = false, any_ext = false, any_op = false;
     for (int i = 0; i < n_probs; ++i) {
         if (probs[i].k < 16 || probs[i].k % 16) return FACE_ERR_ARG;
         if (probs[i].k > K) K = probs[i].k;
         if (probs[i].n > n_widest) n_widest = probs[i].n;
         if (probs[i].bias) any_bias = true;
-        if (probs[i].x_op || probs[i].x2 || probs[i].y0) any_ext = true;     // the XM = 2 kernels
+        if (probs[i].x_op) any_op = true;
+        if (probs[i].x_op || probs[i].x2 || probs[i].y0) any_ext = true;
     }
     const bool scaled = x_scale || y_scale;
     if (scaled && (!group || period < 1 || ld_scale < 1 || n_groups < 1 || n_groups > kGemmMaxGroups))
@@ -154,6 +168,7 @@ extern "C" int face_rows_linear_ws(const face_lin_problem* probs, int32_t n_prob
     if (x_scale && any_ext) return FACE_ERR_UNSUPPORTED;                 // x scale with split / op / y0
     c.probs = probs, c.n_probs = n_probs, c.K = K, c.n_widest = n_widest, c.max_lds = device_max_lds();
     c.n_cu = device_cu_count(), c.x_scale = x_scale != nullptr, c.y_scale = y_scale != nullptr, c.any_ext = any_ext;
+    c.any_op = any_op;
     c.n_groups = n_groups, c.st = (hipStream_t)stream;
     if (work) {
         if (((uintptr_t)work & 255) || work_layout(probs, n_probs, A.p) > work_bytes) return FACE_ERR_ARG;
@@ -166,19 +181,18 @@ extern "C" int face_rows_linear_ws(const face_lin_problem* probs, int32_t n_prob
         hipLaunchKernelGGL(split_weights_kernel, dim3((unsigned)blocks), dim3(kWave), 0, c.st, A, c.work);
         FACE_LAUNCH_CHECK();
     }
-    // FACE_GEMM_SHAPE="nw,n_sl,xcd" forces one launch shape, for tests that compare every shape's
+    // FACE_GEMM_SHAPE="nw,n_sl,xcd" forces one launch shape (nw < 0: the direct kernel, KW = -nw), for tests that compare every shape's
     // results (split ahead where there is such a kernel); FACE_ERR_UNSUPPORTED if there is none
     if (const char* fs = getenv("FACE_GEMM_SHAPE")) {
         int nw = 0, ns = 0, xcd = 0;
         if (sscanf(fs, "%d,%d,%d", &nw, &ns, &xcd) == 3 && ns > 0) {
             const int nb = ((n_widest + ns - 1) / ns + 31) / 32;
-            const int rc = launch_rows(c, nw, nb, xcd ? 1 : 0);
+            const RowsShape S = nw < 0 ? RowsShape{4, nb, 0, -nw} : RowsShape{nw, nb, xcd ? 1 : 0, 0};
+            const int rc = launch_rows(c, S);
             if (rc != FACE_ERR_UNSUPPORTED || !c.work) return rc;
             c.work = nullptr;                    // no such kernel for weights split ahead
-            return launch_rows(c, nw, nb, xcd ? 1 : 0);
+            return launch_rows(c, S);
         }
     }
-    int NW = 4, NB = 2, xcd = 0;
-    rows_shape(c, NW, NB, xcd);
-    return launch_rows(c, NW, NB, xcd);
+    return launch_rows(c, rows_shape(c));
 }

@@ -20,8 +20,9 @@
 // workgroups per CU, whose prologues and stores hide under each other's products, and costs the same
 // for any K. D holds 32 columns of a row in 32 lanes: the stores are whole 128-byte lines.
 //
-// Every output is the same sequence of products whatever the tile, slice and grid, so results do
-// not depend on the launch shape or on the number of rows.
+// Every output of the staged kernel is the same sequence of products whatever the tile, slice and
+// grid, so results do not depend on the launch shape or on the number of rows; launches small enough
+// for the direct kernel below (rows_shape) sum K in four parts.
 #pragma once
 #include "common.h"
 
@@ -46,7 +47,10 @@ struct GemmProb {
     int k1, x_op;                          // x_op on columns < k1: 0 none, 1 silu, 2 * silu'(xz)
     const float* xz;
     int64_t ld_xz;
+    const float* w2;                       // weights of the columns k >= k1 (w itself if not given)
+    int64_t ld_w2;
     const float* bias;
+    const float* bias_row;                 // per-row factor of the bias, or null
     const float* y0;                       // initial sum beta * y0 (columns < n_y0), null: y
     int64_t ld_y0;
     int n_y0;
@@ -100,7 +104,35 @@ static inline size_t gemm_lds(int NB, int NW, int64_t side_floats) {
     return (size_t)2 * NB * 6144 + 4 * ((size_t)NW * kGemmRows + (size_t)side_floats);
 }
 
-// XM: input mode -- 0 plain, 1 the per-group x scale (xs), 2 split input, transform x_op or y0
+// One row of a problem in plain fp32 products, for operands that do not split: columns n0 .. n0 + ns by
+// the lanes of a wave.
+template <int XM>
+__device__ __forceinline__ void plain_row(const GemmArgs& A, const GemmProb& P, int64_t r, int n0, int ns, int lane) {
+    if (r >= P.m) return;
+    const int64_t g = A.group ? A.group[r % A.period] : 0;
+#pragma unroll 1
+    for (int c = lane; c < ns; c += kWave) {
+        float s = 0.f;
+        if (P.beta != 0.f && n0 + c < P.n_y0)
+            s = P.beta * (P.y0 ? P.y0[r * P.ld_y0 + n0 + c] : P.y[r * P.ld_y + n0 + c]);
+#pragma unroll 1
+        for (int k = 0; k < P.k; ++k) {
+            const bool second = k >= P.k1;
+            float x = second ? P.x2[r * P.ld_x2 + k - P.k1] : P.x[r * P.ld_x + k];
+            if (XM == 1) x *= A.xs[g * A.ld_s + P.s_off + k];
+            if (XM == 3 && !second) x = gemm_op(x, P.x_op == 2 ? P.xz[r * P.ld_xz + k] : 0.f, P.x_op);
+            const float* w = second ? P.w2 : P.w;
+            const int64_t ld = second ? P.ld_w2 : P.ld_w, kk = second ? k - P.k1 : k;
+            s = fmaf(x, A.w_kn ? w[kk * ld + n0 + c] : w[(n0 + c) * ld + kk], s);
+        }
+        if (P.bias) s = fmaf(P.bias_row ? P.bias_row[r] : 1.f, P.bias[n0 + c], s);
+        if (A.ys) s *= A.ys[g * A.ld_s + P.s_off + n0 + c];
+        P.y[r * P.ld_y + n0 + c] = s;
+    }
+}
+
+// XM: input mode -- 0 plain, 1 the per-group x scale (xs), 2 split input (x2, w2) or y0, 3 these and the
+// transform x_op
 // PS: the weights come split from the workspace (split_weights_kernel)
 //
 // The loads ahead have no branches: past an edge (last chunk, last column, last row) they read the last
@@ -108,7 +140,7 @@ static inline size_t gemm_lds(int NB, int NW, int64_t side_floats) {
 // waited for each before issuing the next.)
 template <int NB, int NW, int XM, bool PS>
 __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(GemmArgs A) {
-    constexpr bool XS = XM == 1, XO = XM == 2;
+    constexpr bool XS = XM == 1, XO = XM >= 2, XF = XM == 3;
     constexpr int NSB = 32 * NB, NT = NW * kWave, BUF = NB * 6144;
     constexpr int WI = (NSB * 4 + NT - 1) / NT;               // (column, 8 k) items per thread and chunk
     constexpr int WU = PS ? (6 * NB + NW - 1) / NW : 2 * WI;  // 16-byte loads per thread and chunk
@@ -131,7 +163,7 @@ __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(
         if (it >= A.p[k].first_block) pi = k;
     const GemmProb& P = A.p[pi];
     const int slices = P.slices, local = it - (int)P.first_block, tile = local / slices;
-    const int K = P.k, N = P.n, k1 = P.k1, x_op = XO ? P.x_op : 0;
+    const int K = P.k, N = P.n, k1 = P.k1, x_op = XF ? P.x_op : 0;
     const int n0 = (local - tile * slices) * NSB;
     const int ns = min(NSB, N - n0);                          // a multiple of 16
     const int ncb = (N + 31) >> 5;                            // 32-column blocks
@@ -143,8 +175,8 @@ __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(
     const uint32_t xo = 4 * (uint32_t)(jr * (int)ld_x + 8 * hf), x2o = 4 * (uint32_t)(jr * (int)ld_x2 + 8 * hf);
     const uint32_t xzo = 4 * (uint32_t)(jr * (int)ld_xz + 8 * hf);
     const int grp = A.group ? A.group[(mb + jr) % A.period] : 0;
-    const float* wsrc = P.w;
-    const int64_t ld_w = P.ld_w;
+    const float *wsrc = P.w, *w2src = P.w2;
+    const int64_t ld_w = P.ld_w, ld_w2 = P.ld_w2;
     const bool w_kn = A.w_kn != 0;
     const char* wwork = PS ? A.work + P.w_off + (int64_t)(n0 >> 5) * 3072 : nullptr;
     int woff[WU];                                             // of this wave's 1 KB pieces of a chunk
@@ -163,7 +195,7 @@ __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(
             const uint32_t o = second ? x2o : xo;
             xv[2 * s] = ld4_off(u, o);
             xv[2 * s + 1] = ld4_off(u, o + 16);
-            if (XO && x_op == 2 && !second) {
+            if (XF && x_op == 2 && !second) {
                 zv[2 * s] = ld4_off(xzb + k0, xzo);
                 zv[2 * s + 1] = ld4_off(xzb + k0, xzo + 16);
             }
@@ -187,18 +219,22 @@ __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(
             for (int u = 0; u < WI; ++u) {
                 int col, kg;
                 item(u, col, kg);
-                const float* p = wsrc + (int64_t)min(kGemmK * c + 8 * kg, K - 8) * ld_w + n0 + min(col, ns - 1);
+                const int k = min(kGemmK * c + 8 * kg, K - 8);
+                const bool second = XO && k >= k1;
+                const int64_t ld = second ? ld_w2 : ld_w;
+                const float* p = (second ? w2src + (k - k1) * ld : wsrc + k * ld) + n0 + min(col, ns - 1);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) bw[2 * u][r] = p[r * ld_w];
+                for (int r = 0; r < 4; ++r) bw[2 * u][r] = p[r * ld];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) bw[2 * u + 1][r] = p[(r + 4) * ld_w];
+                for (int r = 0; r < 4; ++r) bw[2 * u + 1][r] = p[(r + 4) * ld];
             }
         } else {
 #pragma unroll
             for (int u = 0; u < WI; ++u) {
                 int col, kg;
                 item(u, col, kg);
-                const float* p = wsrc + (int64_t)(n0 + min(col, ns - 1)) * ld_w + min(kGemmK * c + 8 * kg, K - 8);
+                const int64_t k = min(kGemmK * c + 8 * kg, K - 8), f = n0 + min(col, ns - 1);
+                const float* p = XO && k >= k1 ? w2src + f * ld_w2 + (k - k1) : wsrc + f * ld_w + k;
                 bw[2 * u] = ld4(p);
                 bw[2 * u + 1] = ld4(p + 4);
             }
@@ -300,7 +336,7 @@ __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(
                     b *= ld4(t + 4);
                 }
             }
-            if (XO && x_op && k0 < k1) {
+            if (XF && x_op && k0 < k1) {
                 a = gemm_op4(a, zn[2 * s], x_op);
                 b = gemm_op4(b, zn[2 * s + 1], x_op);
             }
@@ -352,36 +388,20 @@ __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(
         for (int r = 0; r < 16; ++r) chk = fmaf(acc[nb][r], 0.f, chk);
     if (__any(chk != chk)) {
 #pragma unroll 1
-        for (int i = 0; i < kGemmRows; ++i) {
-            const int64_t r = m0 + i;
-            if (r >= M) break;
-            const int64_t g = A.group ? A.group[r % A.period] : 0;
-#pragma unroll 1
-            for (int c = lane; c < ns; c += kWave) {
-                float s = 0.f;
-                if (beta != 0.f && n0 + c < P.n_y0)
-                    s = beta * (P.y0 ? P.y0[r * P.ld_y0 + n0 + c] : P.y[r * ld_y + n0 + c]);
-#pragma unroll 1
-                for (int k = 0; k < K; ++k) {
-                    float x = k < k1 ? P.x[r * ld_x + k] : P.x2[r * ld_x2 + k - k1];
-                    if (XS) x *= A.xs[g * A.ld_s + P.s_off + k];
-                    if (XO && k < k1) x = gemm_op(x, x_op == 2 ? P.xz[r * ld_xz + k] : 0.f, x_op);
-                    s = fmaf(x, w_kn ? wsrc[(int64_t)k * ld_w + n0 + c] : wsrc[(int64_t)(n0 + c) * ld_w + k], s);
-                }
-                if (P.bias) s += P.bias[n0 + c];
-                if (A.ys) s *= A.ys[g * A.ld_s + P.s_off + n0 + c];
-                P.y[r * ld_y + n0 + c] = s;
-            }
-        }
+        for (int i = 0; i < kGemmRows; ++i) plain_row<XM>(A, P, m0 + i, n0, ns, lane);
         return;
     }
     // epilogue: bias and y scale, then stores of 128 bytes per row
     if (P.bias) {
+        const float* br = P.bias_row;
+        float f[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) f[r] = br ? br[min(m0 + 8 * (r >> 2) + (r & 3) + 4 * hf, M - 1)] : 1.f;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             const float b = P.bias[n0 + min(32 * nb + j, ns - 1)];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[nb][r] += b;
+            for (int r = 0; r < 16; ++r) acc[nb][r] = fmaf(f[r], b, acc[nb][r]);
         }
     }
     if (A.ys) {
@@ -412,6 +432,179 @@ __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(
     }
 }
 
+// Small launches: no staging. Each wave loads its columns' weights straight into its B operands (lane
+// j + 32 h: 8 consecutive k of column j), splits them itself and runs D steps of 16 k ahead, without LDS
+// or barriers in the loop; KW of the four waves of a workgroup share a 32-row tile, each a contiguous
+// part of K, and add their sums through LDS in wave order. What bounds these launches is the chain of a
+// wave -- split, products that wait for each other, 0.4 us per 16 k with one wave per SIMD -- times the
+// length of K, not the products or the memory: a quarter of K per wave takes 21 rows of 864 -> 192 from 22 us
+// (staged) to 9.1, and 1,344 rows from 22 to 11.5.
+template <int NB, int KW, int XM>
+__global__ __launch_bounds__(4 * kWave, 2) void rows_gemm_direct_kernel(GemmArgs A) {
+    constexpr bool XS = XM == 1, XO = XM >= 2, XF = XM == 3;
+    constexpr int NSB = 32 * NB, RT = 4 / KW, D = NB >= 3 ? 2 : 3, NR = 16 / KW;
+    __shared__ float ssum[KW > 1 ? KW * NB * 16 * kWave : 1];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), j = lane & 31, hf = lane >> 5;
+    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave), kp = wv % KW, it = blockIdx.x;
+    int pi = 0;
+#pragma unroll 1
+    for (int k = 1; k < A.n_probs; ++k)
+        if (it >= A.p[k].first_block) pi = k;
+    const GemmProb& P = A.p[pi];
+    const int slices = P.slices, local = it - (int)P.first_block, tile = local / slices;
+    const int K = P.k, N = P.n, k1 = P.k1, x_op = XF ? P.x_op : 0, nk = K >> 4;
+    const int n0 = (local - tile * slices) * NSB, ns = min(NSB, N - n0);
+    const int64_t M = P.m, m0 = ((int64_t)tile * RT + wv / KW) * kGemmRows;
+    const int64_t row = min(m0 + j, M - 1);
+    const float *xr = P.x + row * P.ld_x + 8 * hf, *x2r = P.x2 + row * P.ld_x2 + 8 * hf;
+    const float* xzr = P.xz + row * P.ld_xz + 8 * hf;
+    const int grp = A.group ? A.group[row % A.period] : 0;
+    const float* xsr = XS ? A.xs + (int64_t)grp * A.ld_s + P.s_off + 8 * hf : nullptr;
+    const bool w_kn = A.w_kn != 0;
+    const int64_t ld_w = P.ld_w, ld_w2 = P.ld_w2;
+    int64_t wo[NB], wo2[NB];                                  // this lane's column (and k half) in w and w2
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+        const int64_t f = n0 + min(32 * nb + j, ns - 1);
+        wo[nb] = w_kn ? 8 * hf * ld_w + f : f * ld_w + 8 * hf;
+        wo2[nb] = w_kn ? 8 * hf * ld_w2 + f : f * ld_w2 + 8 * hf;
+    }
+    struct Step {
+        v4f x[2], z[2], s[2], w[NB][2];
+    };
+    auto load = [&](int st, Step& b) __attribute__((always_inline)) {
+        const int k0 = 16 * min(st, nk - 1);                  // uniform
+        const bool second = XO && k0 >= k1;
+        const float* p = second ? x2r + (k0 - k1) : xr + k0;
+        b.x[0] = ld4(p);
+        b.x[1] = ld4(p + 4);
+        if (XF && x_op == 2 && !second) {
+            b.z[0] = ld4(xzr + k0);
+            b.z[1] = ld4(xzr + k0 + 4);
+        }
+        if (XS) {
+            b.s[0] = ld4(xsr + k0);
+            b.s[1] = ld4(xsr + k0 + 4);
+        }
+        const float* w = second ? P.w2 : P.w;
+        const int64_t ld = second ? ld_w2 : ld_w, kk = second ? k0 - k1 : k0;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            const float* q = w + (second ? wo2[nb] : wo[nb]) + (w_kn ? kk * ld : kk);
+            if (w_kn) {
+#pragma unroll
+                for (int r = 0; r < 8; ++r) b.w[nb][r >> 2][r & 3] = q[r * ld];
+            } else {
+                b.w[nb][0] = ld4(q);
+                b.w[nb][1] = ld4(q + 4);
+            }
+        }
+    };
+    const int s0 = nk * kp / KW, s1 = nk * (kp + 1) / KW;
+    Step b[D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(s0 + d, b[d]);
+    v16f acc[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[nb][r] = 0.f;
+    const float beta = P.beta;
+    const float* y0 = P.y0 ? P.y0 : P.y;
+    const int64_t ld_y = P.ld_y, ld0 = P.y0 ? P.ld_y0 : ld_y;
+    auto out_row = [&](int r) __attribute__((always_inline)) { return m0 + 8 * (r >> 2) + (r & 3) + 4 * hf; };
+    if (beta != 0.f && kp == 0) {
+        const int n_y0 = min(P.n_y0 - n0, ns);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            if (32 * nb >= n_y0) break;
+            const int64_t c = n0 + min(32 * nb + j, n_y0 - 1);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {                    // at the nearest valid place, zero outside
+                const float v = y0[min(out_row(r), M - 1) * ld0 + c];
+                acc[nb][r] = (32 * nb + j < n_y0 && out_row(r) < M) ? beta * v : 0.f;
+            }
+        }
+    }
+    for (int st = s0; st < s1; st += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            if (st + d >= s1) break;                          // uniform
+            Step& c = b[d];
+            if (XS) c.x[0] *= c.s[0], c.x[1] *= c.s[1];
+            if (XF && x_op && 16 * (st + d) < k1) {
+                c.x[0] = gemm_op4(c.x[0], c.z[0], x_op);
+                c.x[1] = gemm_op4(c.x[1], c.z[1], x_op);
+            }
+            const Split8 x = split8(c.x[0], c.x[1]);
+            Split8 w[NB];
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) w[nb] = split8(c.w[nb][0], c.w[nb][1]);
+            load(st + d + D, c);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) acc[nb] = mfma_32x32x16(x.l, w[nb].h, acc[nb]);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) acc[nb] = mfma_32x32x16(x.h, w[nb].l, acc[nb]);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) acc[nb] = mfma_32x32x16(x.m, w[nb].m, acc[nb]);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) acc[nb] = mfma_32x32x16(x.m, w[nb].h, acc[nb]);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) acc[nb] = mfma_32x32x16(x.h, w[nb].m, acc[nb]);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) acc[nb] = mfma_32x32x16(x.h, w[nb].h, acc[nb]);
+        }
+    }
+    // the NR accumulator registers this wave finishes, of rows out_row(NR kp + i)
+    const int rb = NR * (KW > 1 ? kp : 0);
+    float v[NB][NR];
+    if (KW > 1) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) ssum[((kp * NB + nb) * 16 + r) * kWave + lane] = acc[nb][r];
+        __syncthreads();
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                v[nb][i] = ssum[(nb * 16 + rb + i) * kWave + lane];
+#pragma unroll
+                for (int k = 1; k < KW; ++k) v[nb][i] += ssum[((k * NB + nb) * 16 + rb + i) * kWave + lane];
+            }
+    } else {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int i = 0; i < NR; ++i) v[nb][i] = acc[nb][i];
+    }
+    float chk = 0.f;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int i = 0; i < NR; ++i) chk = fmaf(v[nb][i], 0.f, chk);
+    if (__any(chk != chk)) {
+#pragma unroll 1
+        for (int i = 0; i < 2 * NR; ++i)
+            plain_row<XM>(A, P, m0 + 8 * ((rb + (i >> 1)) >> 2) + ((rb + (i >> 1)) & 3) + 4 * (i & 1), n0, ns, lane);
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+        const int64_t r = out_row(rb + i), rc = min(r, M - 1);
+        const float f = P.bias_row ? P.bias_row[rc] : 1.f;
+        const float* t = A.ys ? A.ys + (int64_t)A.group[rc % A.period] * A.ld_s + P.s_off + n0 : nullptr;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            const int c = min(32 * nb + j, ns - 1);
+            float o = v[nb][i];
+            if (P.bias) o = fmaf(f, P.bias[n0 + c], o);
+            if (A.ys) o *= t[c];
+            if (32 * nb + j < ns && r < M) P.y[r * ld_y + n0 + c] = o;
+        }
+    }
+}
+
 // Splits the weights of a launch once: one wave per 16 k x 32 columns writes the three limbs in the
 // order of the LDS image, [16-k step][column block][limb][64 lanes] of 16 bytes, zeros past the last
 // column and step (an even number of steps). Launched before rows_gemm_kernel where many row tiles would each split them again.
@@ -428,12 +621,15 @@ __global__ __launch_bounds__(kWave) inline void split_weights_kernel(GemmArgs A,
     const int col = 32 * cb + (lane & 31), k = 16 * step + 8 * (lane >> 5);
     v4f a = {0.f, 0.f, 0.f, 0.f}, b = a;
     if (col < P.n && k < P.k) {
+        const bool second = k >= P.k1;
+        const float* w = second ? P.w2 : P.w;
+        const int64_t ld = second ? P.ld_w2 : P.ld_w, kk = second ? k - P.k1 : k;
         if (A.w_kn) {
-            const float* p = P.w + (int64_t)k * P.ld_w + col;
+            const float* p = w + kk * ld + col;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) a[r] = p[r * P.ld_w], b[r] = p[(r + 4) * P.ld_w];
+            for (int r = 0; r < 4; ++r) a[r] = p[r * ld], b[r] = p[(r + 4) * ld];
         } else {
-            const float* p = P.w + (int64_t)col * P.ld_w + k;
+            const float* p = w + col * ld + kk;
             a = ld4(p);
             b = ld4(p + 4);
         }
@@ -445,47 +641,64 @@ __global__ __launch_bounds__(kWave) inline void split_weights_kernel(GemmArgs A,
     d[128] = w.l;
 }
 
+// Launch shape: NB column blocks of 32 per wave; NW waves of the staged kernel (KW = 0) or KW waves per
+// row tile of the direct one.
+struct RowsShape {
+    int NW, NB, xcd, KW;
+};
+
 // Everything a launch needs but its shape.
 struct RowsCtx {
     GemmArgs A;                                  // problems filled, tiling not yet
     const face_lin_problem* probs;
     int n_probs, K, n_widest, max_lds, n_cu, n_groups;
-    bool x_scale, y_scale, any_ext;
+    bool x_scale, y_scale, any_ext, any_op;
     char* work;                                  // workspace for split weights, or null
     hipStream_t st;
 };
 
-// One launch of rows_gemm_kernel with NW waves per workgroup and NB column blocks of 32 per wave;
-// FACE_ERR_UNSUPPORTED, before anything is launched, if there is no such kernel.
+// One launch of a shape; FACE_ERR_UNSUPPORTED, before anything is launched, if there is no such kernel.
 template <int XM>
-static int launch_rows_xm(const RowsCtx& c, int NW, int NB, int xcd_order) {
-    if (NB < 1 || NB > 16) return FACE_ERR_UNSUPPORTED;
+static int launch_rows_xm(const RowsCtx& c, RowsShape S) {
+    if (S.NB < 1 || S.NB > 16 || (S.KW && c.work)) return FACE_ERR_UNSUPPORTED;
     GemmArgs A = c.A;
-    A.xcd_order = xcd_order;
+    A.xcd_order = S.xcd;
     A.work = c.work;
+    const int waves = S.KW ? 4 : S.NW, rows = kGemmRows * (S.KW ? 4 / S.KW : S.NW);
     int64_t blocks = 0;
     for (int i = 0; i < c.n_probs; ++i) {
         const face_lin_problem& s = c.probs[i];
         GemmProb& p = A.p[i];
-        p.slices = (s.n + 32 * NB - 1) / (32 * NB);
+        p.slices = (s.n + 32 * S.NB - 1) / (32 * S.NB);
         p.first_block = blocks;
-        blocks += (s.m + kGemmRows * NW - 1) / (kGemmRows * NW) * p.slices;
+        blocks += (s.m + rows - 1) / rows * p.slices;
     }
     if (blocks == 0) return 0;
     if (blocks > INT32_MAX) return FACE_ERR_UNSUPPORTED;
-    const int64_t side = (c.y_scale ? (int64_t)c.n_groups * 32 * NB : 0) + (c.x_scale ? (int64_t)c.n_groups * c.K : 0);
-    A.side_lds = gemm_lds(NB, NW, side) <= (size_t)c.max_lds;
-    const size_t lds = gemm_lds(NB, NW, A.side_lds ? side : 0);
+    size_t lds = 0;
+    if (!S.KW) {
+        const int64_t side = (c.y_scale ? (int64_t)c.n_groups * 32 * S.NB : 0) + (c.x_scale ? (int64_t)c.n_groups * c.K : 0);
+        A.side_lds = gemm_lds(S.NB, S.NW, side) <= (size_t)c.max_lds;
+        lds = gemm_lds(S.NB, S.NW, A.side_lds ? side : 0);
+    }
     auto go = [&](auto kern) -> int {
         if (lds > 65536 &&
             hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
             return FACE_ERR_UNSUPPORTED;
-        hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW * kWave), lds, c.st, A);
+        hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(waves * kWave), lds, c.st, A);
         FACE_LAUNCH_CHECK();
         return 0;
     };
+    if (S.KW) {
+        switch (S.KW * 16 + S.NB) {
+            case 65: return go(rows_gemm_direct_kernel<1, 4, XM>);
+            case 66: return go(rows_gemm_direct_kernel<2, 4, XM>);
+            default: return FACE_ERR_UNSUPPORTED;
+        }
+    }
+    const int NW = S.NW;
     if (c.work) {
-        switch (NB) {
+        switch (S.NB) {
             case 2: return NW == 4 ? go(rows_gemm_kernel<2, 4, XM, true>) : FACE_ERR_UNSUPPORTED;
             case 3: return NW == 4 ? go(rows_gemm_kernel<3, 4, XM, true>) : FACE_ERR_UNSUPPORTED;
             case 4: return NW == 4 ? go(rows_gemm_kernel<4, 4, XM, true>) : FACE_ERR_UNSUPPORTED;
@@ -495,7 +708,7 @@ static int launch_rows_xm(const RowsCtx& c, int NW, int NB, int xcd_order) {
             default: return FACE_ERR_UNSUPPORTED;
         }
     }
-    switch (NW == 4 || NW == 8 ? 16 * NW + NB : 0) {
+    switch (NW == 4 || NW == 8 ? 16 * NW + S.NB : 0) {
         case 65: return go(rows_gemm_kernel<1, 4, XM, false>);
         case 66: return go(rows_gemm_kernel<2, 4, XM, false>);
         case 67: return go(rows_gemm_kernel<3, 4, XM, false>);
@@ -510,9 +723,10 @@ static int launch_rows_xm(const RowsCtx& c, int NW, int NB, int xcd_order) {
     }
 }
 
-// The three input modes' launches, one translation unit each (gemm.hip, gemm_xs.hip, gemm_op.hip).
-int launch_rows_plain(const RowsCtx& c, int NW, int NB, int xcd_order);
-int launch_rows_xs(const RowsCtx& c, int NW, int NB, int xcd_order);
-int launch_rows_op(const RowsCtx& c, int NW, int NB, int xcd_order);
+// The input modes' launches, one translation unit each (gemm.hip, gemm_xs.hip, gemm_split.hip, gemm_op.hip).
+int launch_rows_plain(const RowsCtx& c, RowsShape S);
+int launch_rows_xs(const RowsCtx& c, RowsShape S);
+int launch_rows_split(const RowsCtx& c, RowsShape S);
+int launch_rows_op(const RowsCtx& c, RowsShape S);
 
 }  // namespace face

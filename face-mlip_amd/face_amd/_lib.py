@@ -97,7 +97,8 @@ class LinProblem(ctypes.Structure):
                 ("k", ctypes.c_int32), ("s_off", ctypes.c_int32), ("beta", ctypes.c_float),
                 ("x2", ctypes.c_void_p), ("ld_x2", ctypes.c_int64), ("k1", ctypes.c_int32), ("x_op", ctypes.c_int32),
                 ("xz", ctypes.c_void_p), ("ld_xz", ctypes.c_int64), ("bias", ctypes.c_void_p),
-                ("y0", ctypes.c_void_p), ("ld_y0", ctypes.c_int64), ("n_y0", ctypes.c_int32), ("pad_", ctypes.c_int32)]
+                ("y0", ctypes.c_void_p), ("ld_y0", ctypes.c_int64), ("n_y0", ctypes.c_int32), ("pad_", ctypes.c_int32),
+                ("w2", ctypes.c_void_p), ("ld_w2", ctypes.c_int64), ("bias_row", ctypes.c_void_p)]
 
 
 def lib():

@@ -1321,12 +1321,15 @@ def node_ln(y0, y1, y2, y3, a, b, eq, C, lw, lb, eps):
 
 
 # ----------------------------------------------------------------------------- row-block linear layers
-def lin(x, w, y, s_off=0, beta=0.0, x2=None, x_op=0, xz=None, bias=None, y0=None, n_y0=None):
+def lin(x, w, y, s_off=0, beta=0.0, x2=None, x_op=0, xz=None, bias=None, y0=None, n_y0=None, w2=None,
+        bias_row=None):
     """One problem of rows_linear: y = (beta y0 + op(x | x2) w^T + bias) [* scales]; x (m, k1),
     x2 (m, k - k1) the rest of the input columns (no concatenated copy), x_op on the x columns:
-    0 none, 1 silu, 2 x * silu'(xz); y0 the initial sum (default y) over its first n_y0 columns.
+    0 none, 1 silu, 2 x * silu'(xz); y0 the initial sum (default y) over its first n_y0 columns; w2 the
+    weights of the x2 columns (default: the rest of w); bias_row (m,) a per-row factor of the bias.
     2-d fp32 views with unit column stride."""
-    return dict(x=x, w=w, y=y, s_off=s_off, beta=beta, x2=x2, x_op=x_op, xz=xz, bias=bias, y0=y0, n_y0=n_y0)
+    return dict(x=x, w=w, y=y, s_off=s_off, beta=beta, x2=x2, x_op=x_op, xz=xz, bias=bias, y0=y0, n_y0=n_y0,
+                w2=w2, bias_row=bias_row)
 
 
 def rows_linear(probs, w_kn=False, bias=None, xs=None, ys=None, group=None, period=1, label="rows_linear"):
@@ -1348,12 +1351,16 @@ def rows_linear(probs, w_kn=False, bias=None, xs=None, ys=None, group=None, peri
         k = k1 + (x2.shape[1] if x2 is not None else 0)
         for t in (x2, xz, y0):
             assert t is None or (t.dim() == 2 and t.stride(1) == 1 and t.shape[0] == x.shape[0])
+        w2, br = pr["w2"], pr["bias_row"]
+        assert w2 is None or (w2.dim() == 2 and w2.stride(1) == 1)
+        assert br is None or (br.is_contiguous() and br.numel() == x.shape[0])
         n_y0 = pr["n_y0"] if pr["n_y0"] is not None else (y0.shape[1] if y0 is not None else y.shape[1])
         arr[i] = _lib.LinProblem(x.data_ptr(), x.stride(0), x.shape[0], w.data_ptr(), w.stride(0), y.data_ptr(),
                                  y.stride(0), y.shape[1], k, int(pr["s_off"]), float(pr["beta"]),
                                  ptr(x2), 0 if x2 is None else x2.stride(0), k1, int(pr["x_op"]),
                                  ptr(xz), 0 if xz is None else xz.stride(0), ptr(b),
-                                 ptr(y0), 0 if y0 is None else y0.stride(0), int(n_y0), 0)
+                                 ptr(y0), 0 if y0 is None else y0.stride(0), int(n_y0), 0, ptr(w2),
+                                 0 if w2 is None else w2.stride(0), ptr(br))
         ref = y
     tab = xs if xs is not None else ys
     if xs is not None and ys is not None and xs.shape[0] != ys.shape[0]:

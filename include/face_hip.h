@@ -380,7 +380,10 @@ int face_radial_spline_order_noalloc(const float* r, const int32_t* pair, int64_
  *   bias            (n) added to every row;
  *   y0, ld_y0, n_y0 initial value of the sum: beta * y0[r, c] for columns c < n_y0 (a multiple
  *                   of 4), 0 beyond; y0 NULL: beta * y[r, :] (y0 may be another tensor, e.g. a
- *                   residual). */
+ *                   residual);
+ *   w2, ld_w2       weights of the columns k >= k1 (with x2): (n, k - k1), or (k - k1, n) if w_kn;
+ *                   NULL: the rest of w;
+ *   bias_row        (m) per-row factor of the bias (with bias), NULL: 1. */
 typedef struct {
     const float* x;
     int64_t ld_x, m;
@@ -399,6 +402,9 @@ typedef struct {
     const float* y0;
     int64_t ld_y0;
     int32_t n_y0, pad_;
+    const float* w2;
+    int64_t ld_w2;
+    const float* bias_row;
 } face_lin_problem;
 /* For each problem (1..8 of them, host array):
  *   y[r, :] = (beta y0[r, :] + (op(x)[r, :] * xs[r, :]) w^T + bias) * ys[r, :]
@@ -416,8 +422,9 @@ int face_rows_linear(const face_lin_problem* probs, int32_t n_probs, int32_t w_k
 /* The same with a workspace for the weights in the form the matrix cores take (split once per call
  * by a launch of its own instead of by every row tile): work, 256-byte aligned, work_bytes of at
  * least face_rows_linear_work(probs, n_probs), free for reuse on `stream` after the call; NULL is
- * face_rows_linear. Results are bitwise the same. face_rows_linear_work gives 0 where splitting
- * ahead does not pay (few rows): pass NULL then. */
+ * face_rows_linear. Results are bitwise the same, but for launches of a few row tiles, where
+ * face_rows_linear sums K in four parts. face_rows_linear_work gives 0 where splitting ahead does
+ * not pay (few rows): pass NULL then. */
 int64_t face_rows_linear_work(const face_lin_problem* probs, int32_t n_probs);
 int face_rows_linear_ws(const face_lin_problem* probs, int32_t n_probs, int32_t w_kn, const float* x_scale,
                         const float* y_scale, int32_t ld_scale, int32_t n_groups, const int32_t* group, int64_t period,

@@ -1028,7 +1028,7 @@ def _rows_launch(x, w, y, w_kn, ahead, beta=0.0, xs=None, ys=None, grp=None, s_o
     from face_amd import _lib
     arr = (_lib.LinProblem * 1)(_lib.LinProblem(x.data_ptr(), x.stride(0), x.shape[0], w.data_ptr(), w.stride(0),
                                                 y.data_ptr(), y.stride(0), y.shape[1], x.shape[1], s_off, beta, None, 0,
-                                                x.shape[1], 0, None, 0, None, None, 0, 0, 0))
+                                                x.shape[1], 0, None, 0, None, None, 0, 0, 0, None, 0, None))
     need = -(-x.shape[1] // 32) * 2 * -(-y.shape[1] // 32) * 3072 if ahead else 0
     work = torch.empty(need, dtype=torch.uint8, device=DEV) if ahead else None
     tab = xs if xs is not None else ys
@@ -1041,27 +1041,33 @@ def _rows_launch(x, w, y, w_kn, ahead, beta=0.0, xs=None, ys=None, grp=None, s_o
 @pytest.mark.parametrize("w_kn", [False, True])
 @pytest.mark.parametrize("m,n,k", [(1, 16, 16), (31, 48, 16), (33, 32, 48), (127, 176, 32), (129, 144, 80), (300, 304, 160),
                                    (64, 528, 112)])
-def test_rows_linear_edges_and_weights_split_ahead(m, n, k, w_kn):
+def test_rows_linear_edges_and_weights_split_ahead(m, n, k, w_kn, monkeypatch):
     """Edges of the 32-row, 32-column and 32-k blocks (odd 16-column blocks of n and k, one row to one
-    past a tile), accumulating onto y, with the weights split in the kernel and ahead: the same bits,
-    and within float32 of torch fp64 (2^-22 |x| |w| per product, k of them, covers the three-way split
-    and the float32 sums)."""
+    past a tile), accumulating onto y: the direct kernel (K in four parts, the rules' choice at these
+    sizes) and the staged kernel with the weights split in it and ahead, the latter two with the same
+    bits, all within float32 of torch fp64 (2^-22 |x| |w| per product covers the three-way split and the
+    float32 sums)."""
     say("rows_linear edges", m, n, k, w_kn)
     torch.manual_seed(m + n + k)
     x = torch.randn(m, k + 4, device=DEV)[:, :k]
     w = torch.randn(k, n + 4, device=DEV)[:, :n] if w_kn else torch.randn(n, k + 4, device=DEV)[:, :k]
     y0 = torch.randn(m, n + 8, device=DEV)
-    outs = []
-    for ahead in (False, True):
-        y = y0.clone()
-        _rows_launch(x, w, y[:, :n], w_kn, ahead, beta=0.5)
-        assert torch.equal(y[:, n:], y0[:, n:])                      # nothing past the last column
-        outs.append(y[:, :n])
-    assert torch.equal(outs[0], outs[1])
     wd = w.double() if w_kn else w.double().t().contiguous()
     ref = 0.5 * y0[:, :n].double() + x.double().contiguous() @ wd.contiguous()
     bound = 2.0 ** -22 * (x.double().abs().contiguous() @ wd.abs().contiguous() + y0[:, :n].double().abs())
-    assert bool(((outs[0].double() - ref).abs() <= bound).all())
+    outs = []
+    for shape, ahead in ((None, False), (f"-4,{-(-n // 64)},0", False), (f"4,{-(-n // 96)},1", False),
+                         (f"8,{-(-n // 160)},0", False), (None, True)):
+        if shape is None:
+            monkeypatch.delenv("FACE_GEMM_SHAPE", raising=False)
+        else:
+            monkeypatch.setenv("FACE_GEMM_SHAPE", shape)
+        y = y0.clone()
+        _rows_launch(x, w, y[:, :n], w_kn, ahead, beta=0.5)
+        assert torch.equal(y[:, n:], y0[:, n:])                      # nothing past the last column
+        assert bool(((y[:, :n].double() - ref).abs() <= bound).all()), (shape, ahead)
+        outs.append(y[:, :n])
+    assert torch.equal(outs[2], outs[3]) and torch.equal(outs[2], outs[4])
 
 
 @pytest.mark.parametrize("ahead", [False, True])
@@ -1076,7 +1082,7 @@ def test_rows_linear_values_past_bf16(where, ahead):
     w[:, 1] = w[:, 1].abs() + 0.5                                    # a definite sign against the infinity
     plain = torch.empty(m, n, device=DEV)
     _rows_launch(x, w, plain, False, ahead)
-    big = x.clone() if where == "x" else w.clone()
+    big = x.clone() if where == "x" else w.clone()              # three column blocks: the direct kernel
     big[5, 0], big[70, 1], big[70, 2], big[80, 3] = 3.4e38, float("inf"), 1e30, float("nan")
     small = w if where == "x" else x
     small[:, 0] = small[:, 0].clamp(-0.5, 0.5)                       # 3.4e38 * 0.5 stays finite
