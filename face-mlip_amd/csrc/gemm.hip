@@ -22,7 +22,7 @@ static int fill_prob(const face_lin_problem& s, int w_kn, bool scaled, const flo
     if (s.m < 0 || s.n < 16 || s.n % 16 || s.k < 16 || s.k % 16 || s.ld_y < s.n || s.ld_w < (w_kn ? s.n : (s.w2 ? s.k1 : s.k)))
         return FACE_ERR_ARG;
     const int k1 = s.x2 ? s.k1 : s.k;
-    if (k1 < 0 || k1 > s.k || k1 % 16 || s.ld_x < k1 || (s.x2 && s.ld_x2 < s.k - k1)) return FACE_ERR_ARG;
+    if (k1 < 0 || k1 > s.k || k1 % 16 || (s.ld_x < k1 && s.ld_x != 0) || (s.x2 && s.ld_x2 < s.k - k1)) return FACE_ERR_ARG;
     if (s.x_op < 0 || s.x_op > 2 || (s.x_op == 2 && (!s.xz || s.ld_xz < k1)) || (s.x_op && x_scale)) return FACE_ERR_ARG;
     if (s.w2 && (!s.x2 || s.ld_w2 < (w_kn ? s.n : s.k - k1))) return FACE_ERR_ARG;
     if (s.bias_row && !s.bias) return FACE_ERR_ARG;
@@ -39,14 +39,14 @@ static int fill_prob(const face_lin_problem& s, int w_kn, bool scaled, const flo
     if (s.ld_x % 4 || s.ld_y % 4 || !al16(s.x) || !al16(s.y) || (!w_kn && (!al16(s.w) || s.ld_w % 4)) ||
         (s.w2 && !w_kn && (!al16(s.w2) || s.ld_w2 % 4)) ||
         (s.x2 && (!al16(s.x2) || s.ld_x2 % 4)) || (s.x_op == 2 && (!al16(s.xz) || s.ld_xz % 4)) ||
-        (s.bias && !al16(s.bias)) || (s.y0 && (!al16(s.y0) || s.ld_y0 % 4)))
+        (s.y0 && (!al16(s.y0) || s.ld_y0 % 4)))
         return FACE_ERR_UNSUPPORTED;
     p.x = s.x, p.ld_x = s.ld_x, p.m = s.m, p.w = s.w, p.ld_w = s.ld_w, p.y = s.y, p.ld_y = s.ld_y, p.n = s.n;
     p.k = s.k, p.s_off = s.s_off, p.beta = s.beta;
     p.x2 = s.x2 ? s.x2 : s.x, p.ld_x2 = s.x2 ? s.ld_x2 : s.ld_x, p.k1 = k1;
     p.x_op = s.x_op, p.xz = s.x_op == 2 ? s.xz : s.x, p.ld_xz = s.x_op == 2 ? s.ld_xz : s.ld_x;
     p.w2 = s.w2 ? s.w2 : (w_kn ? s.w + (int64_t)k1 * s.ld_w : s.w + k1), p.ld_w2 = s.w2 ? s.ld_w2 : s.ld_w;
-    p.bias = s.bias, p.bias_row = s.bias_row;
+    p.bias = s.bias, p.bias_row = s.bias_row, p.sum_row = s.sum_row;
     p.y0 = s.y0, p.ld_y0 = s.y0 ? s.ld_y0 : 0, p.n_y0 = s.y0 ? s.n_y0 : s.n;
     return 0;
 }
@@ -148,8 +148,8 @@ extern "C" int face_rows_linear_ws(const face_lin_problem* probs, int32_t n_prob
         if (probs[i].k > K) K = probs[i].k;
         if (probs[i].n > n_widest) n_widest = probs[i].n;
         if (probs[i].bias) any_bias = true;
-        if (probs[i].x_op) any_op = true;
-        if (probs[i].x_op || probs[i].x2 || probs[i].y0) any_ext = true;
+        if (probs[i].x_op || probs[i].sum_row) any_op = true;
+        if (probs[i].x_op || probs[i].sum_row || probs[i].x2 || probs[i].y0) any_ext = true;
     }
     const bool scaled = x_scale || y_scale;
     if (scaled && (!group || period < 1 || ld_scale < 1 || n_groups < 1 || n_groups > kGemmMaxGroups))
@@ -195,4 +195,34 @@ extern "C" int face_rows_linear_ws(const face_lin_problem* probs, int32_t n_prob
         }
     }
     return launch_rows(c, rows_shape(c));
+}
+
+// y[r] = b + sum_k silu(x[r, k]) w[k]: the energy row of the readout's last layer (face/model.py:336). One
+// column is far below the matrix cores' 32, and the layer's other columns need it neither as padding nor
+// as a second pass: one wave per row reads the activations once, whole lines of 16 bytes per lane.
+__global__ __launch_bounds__(256) void silu_dot_kernel(const float* __restrict__ x, int64_t ld_x, int64_t m, int k,
+                                                       const float* __restrict__ w, const float* __restrict__ b,
+                                                       float* __restrict__ y) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t r = (int64_t)blockIdx.x * 4 + threadIdx.x / kWave;
+    if (r >= m) return;
+    float s = 0.f;
+    for (int c = 4 * lane; c < k; c += 4 * kWave) {
+        const v4f a = ld4(x + r * ld_x + c), f = ld4(w + c);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s = fmaf(a[i] * gemm_sigmoid(a[i]), f[i], s);
+    }
+    s = group_sum(s, kWave);
+    if (lane == 0) y[r] = s + (b ? *b : 0.f);
+}
+
+extern "C" int face_silu_dot(const float* x, int64_t ld_x, int64_t m, int32_t k, const float* w, const float* b, float* y,
+                             void* stream) {
+    if (m < 0 || k < 4 || k % 4 || ld_x < k || (m > 0 && (!x || !w || !y))) return FACE_ERR_ARG;
+    if (ld_x % 4 || !al16(x) || !al16(w) || m > (int64_t)INT32_MAX) return FACE_ERR_UNSUPPORTED;
+    if (m == 0) return 0;
+    hipLaunchKernelGGL(silu_dot_kernel, dim3((unsigned)((m + 3) / 4)), dim3(256), 0, (hipStream_t)stream, x, ld_x, m, k, w,
+                       b, y);
+    FACE_LAUNCH_CHECK();
+    return 0;
 }

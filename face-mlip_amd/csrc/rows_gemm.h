@@ -51,6 +51,7 @@ struct GemmProb {
     int64_t ld_w2;
     const float* bias;
     const float* bias_row;                 // per-row factor of the bias, or null
+    const float* sum_row;                  // per-row factor of the sum before the bias, or null
     const float* y0;                       // initial sum beta * y0 (columns < n_y0), null: y
     int64_t ld_y0;
     int n_y0;
@@ -125,6 +126,7 @@ __device__ __forceinline__ void plain_row(const GemmArgs& A, const GemmProb& P, 
             const int64_t ld = second ? P.ld_w2 : P.ld_w, kk = second ? k - P.k1 : k;
             s = fmaf(x, A.w_kn ? w[kk * ld + n0 + c] : w[(n0 + c) * ld + kk], s);
         }
+        if (P.sum_row) s *= P.sum_row[r];
         if (P.bias) s = fmaf(P.bias_row ? P.bias_row[r] : 1.f, P.bias[n0 + c], s);
         if (A.ys) s *= A.ys[g * A.ld_s + P.s_off + n0 + c];
         P.y[r * P.ld_y + n0 + c] = s;
@@ -392,6 +394,14 @@ __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(
         return;
     }
     // epilogue: bias and y scale, then stores of 128 bytes per row
+    if (XF && P.sum_row) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float f = P.sum_row[min(m0 + 8 * (r >> 2) + (r & 3) + 4 * hf, M - 1)];
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) acc[nb][r] *= f;
+        }
+    }
     if (P.bias) {
         const float* br = P.bias_row;
         float f[16];
@@ -592,12 +602,13 @@ __global__ __launch_bounds__(4 * kWave, 2) void rows_gemm_direct_kernel(GemmArgs
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
         const int64_t r = out_row(rb + i), rc = min(r, M - 1);
-        const float f = P.bias_row ? P.bias_row[rc] : 1.f;
+        const float f = P.bias_row ? P.bias_row[rc] : 1.f, sr = XF && P.sum_row ? P.sum_row[rc] : 1.f;
         const float* t = A.ys ? A.ys + (int64_t)A.group[rc % A.period] * A.ld_s + P.s_off + n0 : nullptr;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             const int c = min(32 * nb + j, ns - 1);
             float o = v[nb][i];
+            if (XF && P.sum_row) o *= sr;
             if (P.bias) o = fmaf(f, P.bias[n0 + c], o);
             if (A.ys) o *= t[c];
             if (32 * nb + j < ns && r < M) P.y[r * ld_y + n0 + c] = o;

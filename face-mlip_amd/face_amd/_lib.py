@@ -79,6 +79,7 @@ _SIGS = {
     "face_edge_linear_fwd": (ctypes.c_int, [P, I32, I64, I32, P, P, I32, P, I32, P, P, I32, P]),
     "face_edge_linear_bwd": (ctypes.c_int, [P, I32, I32, P, I32, P, P, I64, P, I32, P, I32, P]),
     "face_rows_linear": (ctypes.c_int, [P, I32, I32, P, P, I32, I32, P, I64, P]),
+    "face_silu_dot": (ctypes.c_int, [P, I64, I64, I32, P, P, P, P]),
     "face_rows_linear_work": (I64, [P, I32]),
     "face_rows_linear_ws": (ctypes.c_int, [P, I32, I32, P, P, I32, I32, P, I64, P, I64, P]),
     "face_eq_gate_fwd": (ctypes.c_int, [P, P, P, I64, I32, P, P, P]),
@@ -98,7 +99,8 @@ class LinProblem(ctypes.Structure):
                 ("x2", ctypes.c_void_p), ("ld_x2", ctypes.c_int64), ("k1", ctypes.c_int32), ("x_op", ctypes.c_int32),
                 ("xz", ctypes.c_void_p), ("ld_xz", ctypes.c_int64), ("bias", ctypes.c_void_p),
                 ("y0", ctypes.c_void_p), ("ld_y0", ctypes.c_int64), ("n_y0", ctypes.c_int32), ("pad_", ctypes.c_int32),
-                ("w2", ctypes.c_void_p), ("ld_w2", ctypes.c_int64), ("bias_row", ctypes.c_void_p)]
+                ("w2", ctypes.c_void_p), ("ld_w2", ctypes.c_int64), ("bias_row", ctypes.c_void_p),
+                ("sum_row", ctypes.c_void_p)]
 
 
 def lib():

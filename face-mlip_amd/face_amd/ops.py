@@ -394,19 +394,62 @@ def dir_transport(Vb, Mb, phi, Y, graph, Kd, transport):
     return DirTransport.apply(Vb, Mb, phi, Y, graph, Kd, transport)
 
 
+def _rows16(*ts):
+    """Whether every tensor (None skipped) is a float32 device matrix or vector whose rows the row-block
+    kernels take as they are: unit column stride, 16-byte aligned rows."""
+    return all(t is None or (t.is_cuda and t.dtype == torch.float32 and t.stride(-1) == 1 and t.data_ptr() % 16 == 0
+                             and (t.dim() == 1 or t.stride(0) % 4 == 0)) for t in ts)
+
+
 class ReadoutMLP(torch.autograd.Function):
-    """The readout after the LayerNorm on the library GEMMs (face/model.py:331-339, the gate of
-    :286-287): z0 = [inv | h] W0^T + b0 (two accumulating GEMMs, no concatenated copy),
-    o = W2 silu(W1 silu(z0) + b1) + b2, e = o[:, :1], h_new = h + o[:, 1:], gvm = inv Wg^T + bg.
-    As one autograd node its backward accumulates where autograd would add: d inv takes the gate
-    term in the second GEMM's epilogue, d h = gh + dz0 W0[:, 9C:10C] in one GEMM. last (the final
-    pass, whose h_new nobody reads): only the energy row of the last layer is computed and its
-    input gradient is the outer product ge W2[0]. W0a / W0b are the inv / h column blocks of W0.
-    Weights receive no gradient; h's only when h takes one (the first pass's rows are constants)."""
+    """The readout after the LayerNorm (face/model.py:331-339, the gate of :286-287):
+    z0 = [inv | h] W0^T + b0 (no concatenated copy), o = W2 silu(W1 silu(z0) + b1) + b2,
+    e = o[:, :1], h_new = h + o[:, 1:], gvm = inv Wg^T + bg. As one autograd node its backward
+    accumulates where autograd would add: d inv takes the gate term as further input columns of the same
+    product, d h = gh + dz0 W0[:, 9C:10C]. last (the final pass, whose h_new nobody reads): only the
+    energy row of the last layer is computed. W0a / W0b are the inv / h column blocks of W0.
+    Weights receive no gradient; h's only when h takes one (the first pass's rows are constants).
+
+    Widths that are multiples of 16 run on the row-block kernels, SiLU and its derivative applied to
+    the rows as they load: z0 and the gate row in one launch, then z1, the residual rows, the energy
+    row; backward in three launches (10,752 atoms, C = 160, forward and backward: 660 us on the
+    library's float32 products with the activations between them, 340 us here). Other widths, and
+    weights without 16-byte aligned rows, take the library products."""
 
     @staticmethod
     def forward(ctx, inv, h, W0a, W0b, b0, W1, b1, W2, b2, Wg, bg, last, hb):
-        if hb is not None:                                # b0 + h W0b^T precomputed (h a constant)
+        ctx.last = last
+        ctx.w = (W0a, W0b, W1, W2, Wg)
+        C, H1, H2 = W0b.shape[1], W0a.shape[0], W1.shape[0]
+        N, dev = inv.shape[0], inv.device
+        ctx.rows = (N > 0 and all(v % 16 == 0 for v in (C, H1, H2, W0a.shape[1])) and W2.shape[0] == C + 1
+                    and (Wg is None or (Wg.shape[0] % 16 == 0 and bg is not None))
+                    and all(b is not None for b in (b0, b1, b2))
+                    and _rows16(W0a, W0b, b0, W1, b1, W2, Wg, bg) and inv.dtype == torch.float32
+                    and h.dtype == torch.float32 and inv.is_cuda)
+        if ctx.rows:
+            inv_, h_ = _aligned_rows(inv), _aligned_rows(h)
+            z0 = torch.empty(N, H1, device=dev)
+            if hb is not None:                            # b0 + h W0b^T precomputed (h a constant)
+                probs = [lin(inv_, W0a, z0, beta=1.0, y0=_aligned_rows(hb))]
+            else:
+                probs = [lin(inv_, W0a, z0, x2=h_, w2=W0b, bias=b0)]
+            gvm = None
+            if Wg is not None:
+                gvm = torch.empty(N, Wg.shape[0], device=dev)
+                probs.append(lin(inv_, Wg, gvm, bias=bg))
+            rows_linear(probs, label="readout_in")
+            z1 = torch.empty(N, H2, device=dev)
+            rows_linear([lin(z0, W1, z1, x_op=1, bias=b1)], label="readout_hid")
+            h_new = None
+            if not last:
+                h_new = torch.empty(N, C, device=dev)
+                rows_linear([lin(z1, W2[1:], h_new, x_op=1, bias=b2[1:], beta=1.0, y0=h_)], label="readout_out")
+            e = torch.empty(N, 1, device=dev)
+            call("face_silu_dot", ptr(z1), H2, N, H2, ptr(W2), ptr(b2), ptr(e), _lib.stream_of(e), label="readout_energy")
+            ctx.save_for_backward(z0, z1)
+            return e, h_new, gvm
+        if hb is not None:
             z0 = torch.addmm(hb, inv, W0a.t())
         else:
             z0 = torch.addmm(b0, inv, W0a.t())
@@ -422,8 +465,6 @@ class ReadoutMLP(torch.autograd.Function):
             h_new = torch.add(h, o[:, 1:])
         gvm = torch.addmm(bg, inv, Wg.t()) if Wg is not None else None
         ctx.save_for_backward(z0, z1)
-        ctx.w = (W0a, W0b, W1, W2, Wg)
-        ctx.last = last
         return e, h_new, gvm
 
     @staticmethod
@@ -432,21 +473,45 @@ class ReadoutMLP(torch.autograd.Function):
         W0a, W0b, W1, W2, Wg = ctx.w
         N = z0.shape[0]
         C = W0b.shape[1]
+        need_h = ctx.needs_input_grad[1]                  # not for the first pass's constant rows
         if ge is None:
             ge = z0.new_zeros(N, 1)
+        if not ctx.last and gh is None:
+            gh = z0.new_zeros(N, C)
+        gate = ggvm is not None and Wg is not None
+        if ctx.rows:
+            dev = z0.device
+            ge_ = ge.float().contiguous().view(-1)
+            da0 = torch.empty_like(z0)
+            if ctx.last:                                  # da1 = ge W2[0]: one input row, its factor on the sums
+                rows_linear([lin(W2[:1].expand(N, -1), W1, da0, x_op=2, xz=z1, sum_row=ge_)], w_kn=True,
+                            label="readout_hid_bwd")
+            else:
+                gh_ = _aligned_rows(gh)
+                da1 = torch.empty_like(z1)
+                rows_linear([lin(gh_, W2[1:], da1, bias=W2[0], bias_row=ge_)], w_kn=True, label="readout_out_bwd")
+                rows_linear([lin(da1, W1, da0, x_op=2, xz=z1)], w_kn=True, label="readout_hid_bwd")
+            dinv = torch.empty(N, W0a.shape[1], device=dev)
+            probs = [lin(da0, W0a, dinv, x_op=2, xz=z0, x2=_aligned_rows(ggvm) if gate else None,
+                         w2=Wg if gate else None)]
+            dh = None
+            if need_h:
+                dh = torch.empty(N, C, device=dev)
+                probs.append(lin(da0, W0b, dh, x_op=2, xz=z0, beta=0.0 if ctx.last else 1.0,
+                                 y0=None if ctx.last else gh_))
+            rows_linear(probs, w_kn=True, label="readout_in_bwd")
+            return dinv, dh, None, None, None, None, None, None, None, None, None, None, None
         if ctx.last:
             da1 = ge * W2[:1]                                                     # (N, 2C)
         else:
-            if gh is None:
-                gh = z0.new_zeros(N, C)
             da1 = torch.cat([ge, gh], 1) @ W2
         da0 = torch.ops.aten.silu_backward(da1, z1) @ W1
         dz0 = torch.ops.aten.silu_backward(da0, z0)
         dinv = dz0 @ W0a
-        if ggvm is not None and Wg is not None:
+        if gate:
             dinv.addmm_(ggvm, Wg)
         dh = None
-        if ctx.needs_input_grad[1]:                       # not for the first pass's constant rows
+        if need_h:
             dh = torch.addmm(gh, dz0, W0b) if (not ctx.last) else dz0 @ W0b
         return dinv, dh, None, None, None, None, None, None, None, None, None, None, None
 
@@ -1322,14 +1387,15 @@ def node_ln(y0, y1, y2, y3, a, b, eq, C, lw, lb, eps):
 
 # ----------------------------------------------------------------------------- row-block linear layers
 def lin(x, w, y, s_off=0, beta=0.0, x2=None, x_op=0, xz=None, bias=None, y0=None, n_y0=None, w2=None,
-        bias_row=None):
+        bias_row=None, sum_row=None):
     """One problem of rows_linear: y = (beta y0 + op(x | x2) w^T + bias) [* scales]; x (m, k1),
     x2 (m, k - k1) the rest of the input columns (no concatenated copy), x_op on the x columns:
     0 none, 1 silu, 2 x * silu'(xz); y0 the initial sum (default y) over its first n_y0 columns; w2 the
-    weights of the x2 columns (default: the rest of w); bias_row (m,) a per-row factor of the bias.
+    weights of the x2 columns (default: the rest of w); bias_row / sum_row (m,) per-row factors of the bias
+    and of the sum before it; x may have one row for all (stride 0).
     2-d fp32 views with unit column stride."""
     return dict(x=x, w=w, y=y, s_off=s_off, beta=beta, x2=x2, x_op=x_op, xz=xz, bias=bias, y0=y0, n_y0=n_y0,
-                w2=w2, bias_row=bias_row)
+                w2=w2, bias_row=bias_row, sum_row=sum_row)
 
 
 def rows_linear(probs, w_kn=False, bias=None, xs=None, ys=None, group=None, period=1, label="rows_linear"):
@@ -1351,16 +1417,17 @@ def rows_linear(probs, w_kn=False, bias=None, xs=None, ys=None, group=None, peri
         k = k1 + (x2.shape[1] if x2 is not None else 0)
         for t in (x2, xz, y0):
             assert t is None or (t.dim() == 2 and t.stride(1) == 1 and t.shape[0] == x.shape[0])
-        w2, br = pr["w2"], pr["bias_row"]
+        w2, br, sr = pr["w2"], pr["bias_row"], pr["sum_row"]
         assert w2 is None or (w2.dim() == 2 and w2.stride(1) == 1)
-        assert br is None or (br.is_contiguous() and br.numel() == x.shape[0])
+        for t in (br, sr):
+            assert t is None or (t.is_contiguous() and t.dtype == torch.float32 and t.numel() == x.shape[0])
         n_y0 = pr["n_y0"] if pr["n_y0"] is not None else (y0.shape[1] if y0 is not None else y.shape[1])
         arr[i] = _lib.LinProblem(x.data_ptr(), x.stride(0), x.shape[0], w.data_ptr(), w.stride(0), y.data_ptr(),
                                  y.stride(0), y.shape[1], k, int(pr["s_off"]), float(pr["beta"]),
                                  ptr(x2), 0 if x2 is None else x2.stride(0), k1, int(pr["x_op"]),
                                  ptr(xz), 0 if xz is None else xz.stride(0), ptr(b),
                                  ptr(y0), 0 if y0 is None else y0.stride(0), int(n_y0), 0, ptr(w2),
-                                 0 if w2 is None else w2.stride(0), ptr(br))
+                                 0 if w2 is None else w2.stride(0), ptr(br), ptr(sr))
         ref = y
     tab = xs if xs is not None else ys
     if xs is not None and ys is not None and xs.shape[0] != ys.shape[0]:
@@ -1390,12 +1457,19 @@ class ScaledMix(torch.autograd.Function):
         C = wm[0].shape[0]
         dev = Af[0].device
         outs = [torch.empty(a.shape[0], N, C, device=dev) for a in Af]
+        # the transport sums are further input columns of ranks 1 and 2, with their own weights (24,000
+        # atoms, C = 160, 512 transport columns: 190 + 345 us for the library's products written first and
+        # accumulated onto, 390 us in the one launch)
         Ds = {1: D1, 2: D2}
-        for l, D in Ds.items():
-            if D is not None:
-                torch.mm(D.reshape(-1, D.shape[-1]), wt[l - 1].t(), out=outs[l].view(-1, C))
-        probs = [(a.reshape(-1, a.shape[-1]), wm[l], outs[l].view(-1, C), l * C,
-                  1.0 if Ds.get(l) is not None else 0.0) for l, a in enumerate(Af)]
+        probs = []
+        for l, a in enumerate(Af):
+            x, y, D = a.reshape(-1, a.shape[-1]), outs[l].view(-1, C), Ds.get(l)
+            D = None if D is None else D.reshape(-1, D.shape[-1])
+            if D is not None and not (D.shape[1] % 16 == 0 and _rows16(D, wt[l - 1])):
+                torch.mm(D, wt[l - 1].t(), out=y)
+                probs.append(lin(x, wm[l], y, l * C, 1.0))
+            else:
+                probs.append(lin(x, wm[l], y, l * C, x2=D, w2=None if D is None else wt[l - 1]))
         rows_linear(probs, ys=s_tab, group=group, period=N, label="mix_fwd")
         ctx.save_for_backward(s_tab, group)
         ctx.wm, ctx.wt, ctx.has_D = wm, wt, (D1 is not None, D2 is not None)

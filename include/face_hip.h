@@ -383,7 +383,9 @@ int face_radial_spline_order_noalloc(const float* r, const int32_t* pair, int64_
  *                   residual);
  *   w2, ld_w2       weights of the columns k >= k1 (with x2): (n, k - k1), or (k - k1, n) if w_kn;
  *                   NULL: the rest of w;
- *   bias_row        (m) per-row factor of the bias (with bias), NULL: 1. */
+ *   bias_row        (m) per-row factor of the bias (with bias), NULL: 1;
+ *   sum_row         (m) per-row factor of the sum before the bias, NULL: 1;
+ *   ld_x = 0        one input row x (k1) for every output row. */
 typedef struct {
     const float* x;
     int64_t ld_x, m;
@@ -405,6 +407,7 @@ typedef struct {
     const float* w2;
     int64_t ld_w2;
     const float* bias_row;
+    const float* sum_row;
 } face_lin_problem;
 /* For each problem (1..8 of them, host array):
  *   y[r, :] = (beta y0[r, :] + (op(x)[r, :] * xs[r, :]) w^T + bias) * ys[r, :]
@@ -429,6 +432,11 @@ int64_t face_rows_linear_work(const face_lin_problem* probs, int32_t n_probs);
 int face_rows_linear_ws(const face_lin_problem* probs, int32_t n_probs, int32_t w_kn, const float* x_scale,
                         const float* y_scale, int32_t ld_scale, int32_t n_groups, const int32_t* group, int64_t period,
                         void* work, int64_t work_bytes, void* stream);
+
+/* y[r] = b[0] + sum_k silu(x[r, k]) w[k], r < m: the energy row of the readout's last layer
+ * (face/model.py:336). x, w 16-byte aligned, k and ld_x multiples of 4; b may be NULL. */
+int face_silu_dot(const float* x, int64_t ld_x, int64_t m, int32_t k, const float* w, const float* b, float* y,
+                  void* stream);
 
 /* ---------------------------------------------------------------- per-edge linear layers
  * Forward: y (E, ld_y) = x (E, ld_x) w^T + b + tab[idx[e]], w (F, K) row-major, b (F) and tab

@@ -1028,7 +1028,7 @@ def _rows_launch(x, w, y, w_kn, ahead, beta=0.0, xs=None, ys=None, grp=None, s_o
     from face_amd import _lib
     arr = (_lib.LinProblem * 1)(_lib.LinProblem(x.data_ptr(), x.stride(0), x.shape[0], w.data_ptr(), w.stride(0),
                                                 y.data_ptr(), y.stride(0), y.shape[1], x.shape[1], s_off, beta, None, 0,
-                                                x.shape[1], 0, None, 0, None, None, 0, 0, 0, None, 0, None))
+                                                x.shape[1], 0, None, 0, None, None, 0, 0, 0, None, 0, None, None))
     need = -(-x.shape[1] // 32) * 2 * -(-y.shape[1] // 32) * 3072 if ahead else 0
     work = torch.empty(need, dtype=torch.uint8, device=DEV) if ahead else None
     tab = xs if xs is not None else ys
@@ -1102,6 +1102,41 @@ def test_rows_linear_values_past_bf16(where, ahead):
     assert (out[~touched].double() - rest).abs().max() <= 1e-5 * rest.abs().max()
     assert bool((out[70] == float("inf")).all()) and bool(torch.isnan(out[80]).all())
     assert (out[5].double() - ref[5]).abs().max() <= 1e-6 * ref[5].abs().max()
+
+
+@pytest.mark.parametrize("last,gate,const_h", [(False, True, False), (False, False, True), (True, False, False),
+                                               (True, True, False)])
+@pytest.mark.parametrize("N,C", [(1, 16), (33, 48), (700, 160), (40, 24)])
+def test_readout_mlp_matches_torch(N, C, last, gate, const_h):
+    """ops.readout_mlp on the row-block kernels (C a multiple of 16) and on the library products (24)
+    against torch in fp64: outputs and the gradients of the invariant row and h, with h given or folded
+    into a constant (hb), the gate row, and the last pass's energy row alone. 5e-6 of the largest value:
+    four float32 layers of at most 10 C = 1,600 terms."""
+    from face_amd import ops
+    say("readout_mlp", N, C, last, gate, const_h)
+    torch.manual_seed(N + C)
+    r = lambda *s: torch.randn(*s, device=DEV) / s[-1] ** 0.5
+    inv, h = torch.randn(N, 9 * C, device=DEV, requires_grad=True), torch.randn(N, C, device=DEV, requires_grad=True)
+    W0, b0, W1, b1, W2, b2 = r(2 * C, 10 * C + 4), r(2 * C), r(2 * C, 2 * C), r(2 * C), r(C + 1, 2 * C), r(C + 1)
+    Wg, bg = (r(2 * C, 9 * C), r(2 * C)) if gate else (None, None)
+    W0a, W0b = W0[:, :9 * C], W0[:, 9 * C:10 * C]
+    hb = (h.detach().double() @ W0b.double().t().contiguous() + b0.double()).float() if const_h else None
+    outs = ops.readout_mlp(inv, h, W0a, W0b, b0, W1, b1, W2, b2, Wg, bg, last, hb)
+    ups = [None if o is None else torch.randn_like(o) for o in outs]
+    F = torch.nn.functional
+    d = lambda t: t.detach().cpu().double()
+    inv_, h_ = d(inv).requires_grad_(True), d(h).requires_grad_(True)
+    z0 = F.linear(inv_, d(W0a)) + (d(hb) if const_h else F.linear(h_, d(W0b), d(b0)))
+    o = F.linear(F.silu(F.linear(F.silu(z0), d(W1), d(b1))), d(W2), d(b2))
+    refs = [o[:, :1], None if last else h_ + o[:, 1:], F.linear(inv_, d(Wg), d(bg)) if gate else None]
+    loss = lambda os, us: sum((x * u).sum() for x, u in zip(os, us) if x is not None)
+    got = torch.autograd.grad(loss(outs, ups), [inv, h], allow_unused=True)
+    want = torch.autograd.grad(loss(refs, [None if u is None else d(u) for u in ups]), [inv_, h_], allow_unused=True)
+    for a, b in zip(outs, refs):
+        assert (a is None) == (b is None) and (a is None or rel(a, b) < 5e-6)
+    assert rel(got[0], want[0]) < 5e-6
+    if not const_h:
+        assert rel(got[1], want[1]) < 5e-6
 
 
 @pytest.mark.parametrize("side", ["xs", "ys"])
