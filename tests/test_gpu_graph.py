@@ -64,6 +64,19 @@ def test_liquid_3000_exact(method):
     check_graph([st], 5.0, method=method)
 
 
+@pytest.mark.parametrize("method", ["cell", "small"])
+@pytest.mark.parametrize("n,rc", [(130, 4.0), (150, 6.4), (63, 7.5)])
+def test_dense_rows_of_many_images_exact(n, rc, method):
+    """Rows past 256 pairs (the cell list's keys in LDS; 130 atoms stay below, the others reach ~ 330 and
+    more), several images per neighbour and bins that wrap more than once, in a skewed cell."""
+    say("dense rows", n, rc, method)
+    rng = np.random.default_rng(n)
+    cell = np.array([[8.0, 0, 0], [1.5, 7.5, 0], [-0.7, 0.9, 8.3]])
+    st = {"pos": rng.random((n, 3)) @ cell + rng.integers(-1, 2, (n, 3)) @ cell, "Z": np.full(n, 6), "cell": cell,
+          "pbc": np.ones(3, bool)}
+    check_graph([st], rc, method=method)
+
+
 @pytest.mark.parametrize("k", [3, 4])
 def test_liquid_full_size_exact(k):
     """The 24,000-atom (1.25 M pairs) and 100,000-atom (6.9 M pairs) liquids at full size against
