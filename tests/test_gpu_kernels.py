@@ -359,6 +359,32 @@ def test_node_algebra_dropin_matches_reference_spec(eq):
     assert max(errs) < TOL, errs
 
 
+@pytest.mark.parametrize("eq", [True, False])
+@pytest.mark.parametrize("N,C", [(1, 1), (1, 255), (2, 128), (1, 257), (37, 48)])
+def test_node_algebra_dense_rows_equal_strided(N, C, eq):
+    """The kernels of dense (N, C, k) operands, 256 rows per workgroup (1, 255, 256, 257 and 1,776 rows),
+    against the strided ones on the same values stored component-major: outputs and all gradients. Both
+    form the same sums of at most 27 terms; contraction may differ (1e-6 of the largest value)."""
+    from face_amd.node_kernel import node_algebra
+    say("node dense", N, C, eq)
+    torch.manual_seed(N * C)
+    base = [torch.randn(N, C, k, device=DEV) for k in (3, 3, 3, 6, 6, 6, 10, 10)]
+    ab = [torch.randn(4, C, device=DEV) for _ in range(2)]
+    ups = [torch.randn(N, C, 8, device=DEV), torch.randn(N, C, 3, device=DEV), torch.randn(N, C, 3, 3, device=DEV)]
+    res = []
+    for dense in (True, False):
+        if dense:
+            ins = [x.clone().requires_grad_(True) for x in base]
+        else:                                        # strides (C, 1, N C)
+            ins = [x.permute(2, 0, 1).contiguous().permute(1, 2, 0).requires_grad_(True) for x in base]
+        a, b = [x.clone().requires_grad_(True) for x in ab]
+        outs = node_algebra(*ins, a, b, eq)[:3 if eq else 1]
+        grads = torch.autograd.grad(outs, ins + ([a, b] if eq else []), ups[:len(outs)])
+        res.append(list(outs) + list(grads))
+    for x, y in zip(*res):
+        assert x.shape == y.shape and rel(x, y) < 1e-6
+
+
 def test_node_features_product_layout():
     """Strided P/Q/S read from projection outputs, families written into the readout row,
     symmetrised gated products (face/model.py:244-249,274-276)."""
