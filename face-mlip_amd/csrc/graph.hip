@@ -191,6 +191,58 @@ __global__ __launch_bounds__(1024) void exclusive_scan_kernel(const int32_t* __r
     if (tid == 1023) out[n] = part[1023];
 }
 
+// Row pointers and the two sizes the host needs, stats = {pairs, longest row}, in one workgroup: chunks
+// of 8192 counts (8 to a thread; lane prefix sums, then the 16 wave totals), the running total carried
+// between the chunks. One launch instead of a cumulative sum, a fill, a copy and a maximum.
+constexpr int kScanPer = 8;
+__global__ __launch_bounds__(1024) void nbr_scan_kernel(const int32_t* __restrict__ counts, int64_t n,
+                                                        int32_t* __restrict__ row_ptr, int32_t* __restrict__ stats) {
+    __shared__ int32_t tot[1024 / kWave], mx[1024 / kWave];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+    int32_t run = 0, m = 0;
+    for (int64_t q0 = 0; q0 < n; q0 += 1024 * kScanPer) {
+        const int64_t q = q0 + tid * kScanPer;
+        int32_t v[kScanPer], sum = 0;
+#pragma unroll
+        for (int k = 0; k < kScanPer; ++k) {
+            const int32_t c = counts[min(q + k, n - 1)];     // in range without a branch per load
+            v[k] = q + k < n ? c : 0;
+        }
+#pragma unroll
+        for (int k = 0; k < kScanPer; ++k) {
+            m = max(m, v[k]);
+            sum += v[k];
+        }
+        int32_t before = sum;
+        for (int o = 1; o < kWave; o <<= 1) {
+            const int32_t u = __shfl_up(before, o, kWave);
+            if (lane >= o) before += u;
+        }
+        if (lane == kWave - 1) tot[wv] = before;
+        __syncthreads();
+        int32_t at = run + before - sum;
+        for (int w = 0; w < 1024 / kWave; ++w) {
+            if (w < wv) at += tot[w];
+            run += tot[w];
+        }
+#pragma unroll
+        for (int k = 0; k < kScanPer; ++k) {
+            if (q + k < n) row_ptr[q + k] = at;
+            at += v[k];
+        }
+        __syncthreads();
+    }
+    for (int o = kWave / 2; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, kWave));
+    if (lane == 0) mx[wv] = m;
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 0; w < 1024 / kWave; ++w) m = max(m, mx[w]);
+        row_ptr[n] = run;
+        stats[0] = run;
+        stats[1] = m;
+    }
+}
+
 __global__ __launch_bounds__(256) void nbr_scatter_kernel(int64_t N, const int32_t* __restrict__ bin_of,
                                                           const int32_t* __restrict__ bin_start,
                                                           int32_t* __restrict__ bin_fill,
@@ -297,6 +349,7 @@ __global__ __launch_bounds__(kNbrWaves * kWave) void nbr_rev_kernel(const int32_
                                                                     const int32_t* __restrict__ col,
                                                                     const int32_t* __restrict__ S, int64_t N,
                                                                     int32_t* __restrict__ rev,
+                                                                    int32_t* __restrict__ recv,
                                                                     int32_t* __restrict__ missing) {
     const int64_t i = blockIdx.x * (int64_t)kNbrWaves + threadIdx.x / kWave;
     if (i >= N) return;
@@ -320,6 +373,7 @@ __global__ __launch_bounds__(kNbrWaves * kWave) void nbr_rev_kernel(const int32_
             found = e;
         }
         rev[e] = (int32_t)found;
+        if (recv) recv[e] = (int32_t)i;
     }
 }
 
@@ -451,13 +505,25 @@ extern "C" int face_nbr_fill(const double* pos, int64_t N, const int32_t* atom_s
     return 0;
 }
 
+extern "C" int face_nbr_scan(const int32_t* counts, int64_t N, int32_t* row_ptr, int32_t* stats, void* stream) {
+    if (N < 0 || !row_ptr || !stats || (N > 0 && !counts)) return FACE_ERR_ARG;
+    hipLaunchKernelGGL(nbr_scan_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, counts, N, row_ptr, stats);
+    FACE_LAUNCH_CHECK();
+    return 0;
+}
+
 extern "C" int face_nbr_rev(const int32_t* row_ptr, const int32_t* col, const int32_t* S, int64_t N, int32_t* rev,
                             int32_t* missing, void* stream) {
+    return face_nbr_rev_recv(row_ptr, col, S, N, rev, nullptr, missing, stream);
+}
+
+extern "C" int face_nbr_rev_recv(const int32_t* row_ptr, const int32_t* col, const int32_t* S, int64_t N, int32_t* rev,
+                                 int32_t* recv, int32_t* missing, void* stream) {
     if (N < 0) return FACE_ERR_ARG;
     if (N == 0) return 0;
     if (!row_ptr || !col || !S || !rev || !missing) return FACE_ERR_ARG;
     hipLaunchKernelGGL(nbr_rev_kernel, dim3(wblk(N)), dim3(kNbrWaves * kWave), 0, (hipStream_t)stream, row_ptr, col, S, N, rev,
-                       missing);
+                       recv, missing);
     FACE_LAUNCH_CHECK();
     return 0;
 }

@@ -43,6 +43,8 @@ _SIGS = {
     "face_nbr_count": (ctypes.c_int, [P, I64, P, P, P, P, P, F64, P, P, P, P, P, P, P]),
     "face_nbr_fill": (ctypes.c_int, [P, I64, P, P, P, P, P, F64, P, P, P, P, P, P, P, P, P, P, P, P]),
     "face_nbr_rev": (ctypes.c_int, [P, P, P, I64, P, P, P]),
+    "face_nbr_rev_recv": (ctypes.c_int, [P, P, P, I64, P, P, P, P]),
+    "face_nbr_scan": (ctypes.c_int, [P, I64, P, P, P]),
     "face_nbr_rev_shift": (ctypes.c_int, [P, P, P, I64, P, P, P]),
     "face_nbr_padded": (ctypes.c_int, [P, P, P, P, P, I64, I32, P, P, P, P]),
     "face_edge_geom_fwd": (ctypes.c_int, [P, P, P, P, P, I64, P, I32, F32, F32, P, P, P, P, P]),
@@ -88,7 +90,7 @@ _SIGS = {
     "face_layer_norm_bwd": (ctypes.c_int, [P, P, I64, I32, P, P, P, P, P]),
 }
 
-ABI_VERSION = 25
+ABI_VERSION = 26
 
 
 class LinProblem(ctypes.Structure):

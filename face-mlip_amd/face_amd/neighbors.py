@@ -39,9 +39,9 @@ def _inv_cell(cell, pbc):
     return np.linalg.inv(cell) if pbc.any() else np.zeros((3, 3))
 
 
-def _grid(cell, rc):
+def _grid(cell, rc, inv=None):
     """Bins per axis (each >= rc wide along its reciprocal axis) and bins searched per side."""
-    inv = np.linalg.inv(cell)
+    inv = np.linalg.inv(cell) if inv is None else inv
     fd = 1.0 / np.linalg.norm(inv, axis=0)            # face distances (reciprocal axes = columns)
     nb = np.maximum(1, np.floor(fd / rc).astype(np.int64))
     while nb.prod() > (1 << 22):
@@ -51,14 +51,26 @@ def _grid(cell, rc):
     return [int(x) for x in nb] + [int(x) for x in s]
 
 
-def _build_one_cell_list(pos64, cell, rc, dev, st):
-    """CSR rows for one fully periodic structure with the cell-list generator."""
+def _scan(counts, dev, st):
+    """row_ptr (N+1), pairs and longest row of `counts`: one launch and one read by the host."""
+    N = counts.shape[0]
+    row_ptr = torch.empty(N + 1, dtype=torch.int32, device=dev)
+    stats = torch.empty(2, dtype=torch.int32, device=dev)
+    call("face_nbr_scan", ptr(counts), N, ptr(row_ptr), ptr(stats), st)
+    E, max_row = stats.tolist()
+    return row_ptr, E, max_row
+
+
+def _build_one_cell_list(pos64, cell, rc, dev, st, flags):
+    """CSR rows for one fully periodic structure with the cell-list generator; flags[0] counts
+    overflowing pairs."""
     N = pos64.shape[0]
-    nbh = _grid(cell, rc)
+    inv = np.linalg.inv(cell)
+    nbh = _grid(cell, rc, inv)
     nb_arr = (_lib.I32 * 6)(*nbh)
     nbins = nbh[0] * nbh[1] * nbh[2]
-    cell_d = torch.as_tensor(cell.reshape(9), dtype=torch.float64, device=dev)
-    inv_d = torch.as_tensor(np.linalg.inv(cell).reshape(9), dtype=torch.float64, device=dev)
+    both = torch.as_tensor(np.concatenate([cell.reshape(9), inv.reshape(9)]), dtype=torch.float64, device=dev)
+    cell_d, inv_d = both[:9], both[9:]
     i32 = dict(dtype=torch.int32, device=dev)
     bin_of = torch.empty(N, **i32)
     wrap = torch.empty(N, 3, **i32)
@@ -71,22 +83,19 @@ def _build_one_cell_list(pos64, cell, rc, dev, st):
     counts = torch.empty(N, **i32)
     call("face_nbr_count", ptr(pos64), N, None, None, ptr(cell_d), None, None, float(rc), nb_arr, ptr(bin_of),
          ptr(wrap), ptr(bin_start), ptr(bin_atoms), ptr(counts), st)
-    row_ptr = torch.zeros(N + 1, **i32)
-    row_ptr[1:] = torch.cumsum(counts, 0)
-    E = int(row_ptr[-1])
+    row_ptr, E, max_row = _scan(counts, dev, st)
     key = torch.empty(E, dtype=torch.int64, device=dev)
     col = torch.empty(E, **i32)
     S = torch.empty(E, 3, **i32)
     shift = torch.empty(E, 3, dtype=torch.float32, device=dev)
-    overflow = torch.zeros(1, **i32)
     call("face_nbr_fill", ptr(pos64), N, None, None, ptr(cell_d), None, None, float(rc), nb_arr, ptr(bin_of),
          ptr(wrap), ptr(bin_start), ptr(bin_atoms), ptr(row_ptr), ptr(key), ptr(col), ptr(S), ptr(shift),
-         ptr(overflow), st)
-    return counts, row_ptr, col, S, shift, overflow
+         ptr(flags), st)
+    return counts, row_ptr, col, S, shift, max_row
 
 
-def _build_small(pos64, sizes, cells, pbcs, rc, dev, st):
-    """CSR rows for a batch of structures with the all-pairs generator."""
+def _build_small(pos64, sizes, cells, pbcs, rc, dev, st, flags):
+    """CSR rows for a batch of structures with the all-pairs generator; flags as above."""
     N = pos64.shape[0]
     nstr = len(sizes)
     i32 = dict(dtype=torch.int32, device=dev)
@@ -100,16 +109,13 @@ def _build_small(pos64, sizes, cells, pbcs, rc, dev, st):
     counts = torch.empty(N, **i32)
     call("face_nbr_count", ptr(pos64), N, ptr(atom_struct), ptr(struct_ptr), ptr(cell_d), ptr(inv_d), ptr(pbc_d),
          float(rc), None, None, None, None, None, ptr(counts), st)
-    row_ptr = torch.zeros(N + 1, **i32)
-    row_ptr[1:] = torch.cumsum(counts, 0)
-    E = int(row_ptr[-1])
+    row_ptr, E, max_row = _scan(counts, dev, st)
     col = torch.empty(E, **i32)
     S = torch.empty(E, 3, **i32)
     shift = torch.empty(E, 3, dtype=torch.float32, device=dev)
-    overflow = torch.zeros(1, **i32)
     call("face_nbr_fill", ptr(pos64), N, ptr(atom_struct), ptr(struct_ptr), ptr(cell_d), ptr(inv_d), ptr(pbc_d),
-         float(rc), None, None, None, None, None, ptr(row_ptr), None, ptr(col), ptr(S), ptr(shift), ptr(overflow), st)
-    return counts, row_ptr, col, S, shift, overflow
+         float(rc), None, None, None, None, None, ptr(row_ptr), None, ptr(col), ptr(S), ptr(shift), ptr(flags), st)
+    return counts, row_ptr, col, S, shift, max_row
 
 
 def _check_image_span(pos, cell, pbc, rc):
@@ -119,8 +125,8 @@ def _check_image_span(pos, cell, pbc, rc):
         raise ValueError("positions must be finite")
     if pbc.any():
         inv = np.linalg.inv(cell)
-        f = pos @ inv
-        span = (f.max(0) - f.min(0)) + 2 * rc * np.linalg.norm(inv, axis=0)
+        f = inv.T @ pos.T                               # (3, n): each axis reduced over contiguous values
+        span = (f.max(1) - f.min(1)) + 2 * rc * np.linalg.norm(inv, axis=0)
         if (span[pbc] > 256).any():
             raise ValueError("periodic structure spans more than 256 cells: wrap the positions first")
 
@@ -146,7 +152,7 @@ def build_graph(structures, rc, device="cuda", dtype=torch.float32, method="auto
     pos_np = np.concatenate([p[0] for p in parts]) if parts else np.zeros((0, 3))
     Z_np = np.concatenate([p[1] for p in parts]) if parts else np.zeros(0, np.int64)
     N = len(pos_np)
-    pos64 = torch.as_tensor(pos_np, dtype=torch.float64, device=dev)
+    pos64 = torch.as_tensor(pos_np, dtype=torch.float64, device=dev).contiguous()   # any strides come in
     st = _lib.stream_of(pos64)
     if method == "cell":
         if not all(p[3].all() for p in parts):
@@ -157,9 +163,14 @@ def build_graph(structures, rc, device="cuda", dtype=torch.float32, method="auto
     else:
         big = [k for k, p in enumerate(parts) if sizes[k] > CELL_LIST_MIN_ATOMS and p[3].all()]
     i32 = dict(dtype=torch.int32, device=dev)
+    flags = torch.zeros(2, **i32)                        # overflowing pairs, pairs without their reverse
+    # the host's own arrays go up while the GPU works: everything below is queued before the one read
+    # of `flags` that ends the build (the pair count is the only other one)
     if not big:
-        counts, row_ptr, col, S, shift, overflow = _build_small(pos64, sizes, [p[2] for p in parts],
-                                                                [p[3] for p in parts], rc, dev, st)
+        counts, row_ptr, col, S, shift, max_row = _build_small(pos64, sizes, [p[2] for p in parts],
+                                                               [p[3] for p in parts], rc, dev, st, flags)
+    elif nstr == 1:
+        counts, row_ptr, col, S, shift, max_row = _build_one_cell_list(pos64, parts[0][2], rc, dev, st, flags)
     else:
         # every structure separately (cell list where it applies), then stitched with offsets
         off = np.concatenate([[0], np.cumsum(sizes)])
@@ -167,30 +178,30 @@ def build_graph(structures, rc, device="cuda", dtype=torch.float32, method="auto
         for k, (p, n) in enumerate(zip(parts, sizes)):
             sl = pos64[off[k]:off[k] + n]
             if k in big:
-                pieces.append(_build_one_cell_list(sl.contiguous(), p[2], rc, dev, st))
+                pieces.append(_build_one_cell_list(sl, p[2], rc, dev, st, flags))
             else:
-                pieces.append(_build_small(sl.contiguous(), [n], [p[2]], [p[3]], rc, dev, st))
+                pieces.append(_build_small(sl, [n], [p[2]], [p[3]], rc, dev, st, flags))
         counts = torch.cat([q[0] for q in pieces])
         col = torch.cat([q[2] + int(off[k]) for k, q in enumerate(pieces)])
         S = torch.cat([q[3] for q in pieces])
         shift = torch.cat([q[4] for q in pieces])
-        overflow = sum(q[5] for q in pieces)
-        row_ptr = torch.zeros(N + 1, **i32)
-        row_ptr[1:] = torch.cumsum(counts, 0)
+        row_ptr, _, max_row = _scan(counts, dev, st)
     E = col.shape[0]
-    rev = torch.empty(E, **i32)
-    missing = torch.zeros(1, **i32)
-    call("face_nbr_rev", ptr(row_ptr), ptr(col), ptr(S), N, ptr(rev), ptr(missing), st)
-    if int(overflow.item()) != 0:
-        raise RuntimeError("pair-list build: a row overflowed its counted size")
-    if int(missing.item()) != 0:
-        raise RuntimeError("pair-list build: pair list is not symmetric")
-    max_row = int(counts.max()) if N else 0
-    recv = torch.repeat_interleave(torch.arange(N, device=dev, dtype=torch.int32), counts.long(), output_size=E)
-    batch = torch.as_tensor(np.repeat(np.arange(nstr), sizes), dtype=torch.long, device=dev)
+    rev, recv = torch.empty(E, **i32), torch.empty(E, **i32)
+    call("face_nbr_rev_recv", ptr(row_ptr), ptr(col), ptr(S), N, ptr(rev), ptr(recv), ptr(flags[1:]), st)
+    Z = torch.as_tensor(Z_np, dtype=torch.long, device=dev)
+    if nstr == 1:
+        batch = torch.zeros(N, dtype=torch.long, device=dev)
+    else:
+        batch = torch.as_tensor(np.repeat(np.arange(nstr), sizes), dtype=torch.long, device=dev)
     struct_ptr = torch.as_tensor(np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32), **i32)
-    return Graph(pos64.to(dtype), torch.as_tensor(Z_np, dtype=torch.long, device=dev), batch, nstr, struct_ptr,
-                 row_ptr, col, recv, shift.to(dtype), rev, max_row, S)
+    pos, shift = pos64.to(dtype), shift.to(dtype)
+    overflow, missing = flags.tolist()
+    if overflow != 0:
+        raise RuntimeError("pair-list build: a row overflowed its counted size")
+    if missing != 0:
+        raise RuntimeError("pair-list build: pair list is not symmetric")
+    return Graph(pos, Z, batch, nstr, struct_ptr, row_ptr, col, recv, shift, rev, max_row, S)
 
 
 def padded_view(graph):

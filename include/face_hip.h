@@ -265,6 +265,11 @@ int face_nbr_fill(const double* pos, int64_t N, const int32_t* atom_struct, cons
  * without one (a non-symmetric list). */
 int face_nbr_rev(const int32_t* row_ptr, const int32_t* col, const int32_t* S, int64_t N, int32_t* rev,
                  int32_t* missing, void* stream);
+/* The same, also writing the receiver (row) of every edge: recv (E) int32, NULL: face_nbr_rev. */
+int face_nbr_rev_recv(const int32_t* row_ptr, const int32_t* col, const int32_t* S, int64_t N, int32_t* rev,
+                      int32_t* recv, int32_t* missing, void* stream);
+/* row_ptr (N+1) = exclusive prefix sums of counts (N), stats (2) = {total, largest count}. */
+int face_nbr_scan(const int32_t* counts, int64_t N, int32_t* row_ptr, int32_t* stats, void* stream);
 /* Reverse map for an edge list given by fp32 shift vectors (e.g. a padded graph converted
  * to CSR): the reverse of (i, j, shift) is (j, i, -shift) with bitwise-equal components. */
 int face_nbr_rev_shift(const int32_t* row_ptr, const int32_t* col, const float* shift, int64_t N, int32_t* rev,

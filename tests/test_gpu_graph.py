@@ -144,3 +144,23 @@ def test_padded_view_matches_reference_layout():
         assert np.array_equal(got["shift"].cpu().numpy(), want["shift"].numpy())
         assert np.array_equal(got["batch"].cpu().numpy(), want["batch"].numpy())
         assert np.array_equal(got["pos"].cpu().numpy(), want["pos"].numpy())
+
+
+@pytest.mark.parametrize("n", [0, 1, 63, 64, 511, 513, 8191, 8192, 8193, 20003])
+def test_scan_of_row_counts(n):
+    from face_amd.neighbors import _scan
+    from face_amd import _lib
+    counts = torch.randint(0, 150, (n,), dtype=torch.int32, device="cuda", generator=torch.Generator("cuda").manual_seed(n))
+    row_ptr, total, longest = _scan(counts, counts.device, _lib.stream_of(counts))
+    want = np.concatenate([[0], np.cumsum(counts.cpu().numpy())])
+    assert np.array_equal(row_ptr.cpu().numpy(), want)
+    assert total == want[-1] and longest == (int(counts.max()) if n else 0)
+
+
+@pytest.mark.parametrize("method", ["cell", "small"])
+def test_positions_of_any_strides(method):
+    rng = np.random.default_rng(8)
+    pos = rng.uniform(0, 9.0, (3, 150)).T                # column-major, as a transposed file read gives
+    st = dict(pos=pos, Z=np.ones(150, int), cell=np.eye(3) * 9.0, pbc=True)
+    check_graph([dict(st, pbc=np.ones(3, bool))], 4.0, method)
+    check_graph([dict(st, pbc=np.ones(3, bool), pos=np.repeat(pos, 2, 0)[::2])], 4.0, method)
