@@ -10,131 +10,98 @@
 // X = d, T = msg(h), idx = col). The backward's table reduction walks each atom's reverse
 // edges (rev) the way the gather backward does, so no atomics are needed and the sums are
 // bitwise reproducible; the same pass applies W to each visited edge.
-#include "common.h"
+#include "edges.h"
+
+#include <algorithm>
 
 namespace face {
 
 // ------------------------------------------------------------------ forward
-// The (F, K) weight block sits whole in LDS (160 KB at F = 640, K = 64) as the A operand of
-// v_mfma_f32_16x16x4f32; each wave loads the X rows of 16 BB edges once as B operands (K index
-// q of instruction r of chunk kb = input feature 16 kb + 4q + r) and walks all output blocks, so
-// the output streams out at the write rate: D = W . X^T holds output feature 4q + r of edge j
-// in register r of lane j + 16q, one float4 store of Y[e][f .. f + 3] per lane and block.
-// LDS image: lin_off / lin_layout (common.h).
-constexpr int kLinWaves = 16;
+// D = W . X^T in 32 x 32 blocks as split bf16 products (edges.h): the weight blocks of the workgroup's
+// features sit in LDS as limbs, each wave splits the X rows of 32 edges once and walks the blocks, lane
+// e holding features 8 g + 4 (lane >> 5) + 0..3 of edge e, one float4 store each. Bound by the write of
+// Y; six blocks of 64 inputs (72 KB) leave room for two workgroups per CU.
+constexpr int kLinWaves = 4, kLinBlocks = 6;
 
-template <int KB, int BB, int FB, bool HAS_B, bool HAS_T>
-__global__ __launch_bounds__(kLinWaves * kWave) void edge_linear_fwd_kernel(
+template <int KB, bool HAS_T>
+__global__ __launch_bounds__(kLinWaves * kWave) __attribute__((amdgpu_waves_per_eu(2))) void edge_linear_fwd_kernel(
     const float* __restrict__ X, int ld_X, int64_t E, const float* __restrict__ w, const float* __restrict__ b,
-    int F, int f_chunk, int S, int rot, const float* __restrict__ T, int ld_T, const int32_t* __restrict__ idx,
-    float* __restrict__ Y, int ld_Y) {
-    constexpr int K = 16 * KB, NCH = K / 4;
-    extern __shared__ float sW[];
-    const int tid = threadIdx.x, lane = tid & (kWave - 1);
-    const int f_beg = blockIdx.y * f_chunk;
-    const int nf = min(f_chunk, F - f_beg);                           // a multiple of 16
-    const bool rt = rot != 0;
-    for (int v0 = 0; v0 < nf * NCH; v0 += 4 * (int)blockDim.x) {
-        v4f buf[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int v = v0 + u * (int)blockDim.x + tid;
-            if (v < nf * NCH) buf[u] = ld4(w + (int64_t)(f_beg + v / NCH) * K + 4 * (v % NCH));
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int v = v0 + u * (int)blockDim.x + tid;
-            if (v < nf * NCH) st4(sW + lin_off(v / NCH, v % NCH, S, NCH, rt), buf[u]);
-        }
-    }
-    __syncthreads();
-    const int j = lane & 15, q = lane >> 4;
-    const int wv_id = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int64_t ntile = (E + 16 * BB - 1) / (16 * BB);
-    const int64_t stride = (int64_t)gridDim.x * kLinWaves;
-    const v4f z4 = {0.f, 0.f, 0.f, 0.f};
-    int64_t t = (int64_t)blockIdx.x * kLinWaves + wv_id;
+    int F, int nblk, const float* __restrict__ T, int ld_T, const int32_t* __restrict__ idx, float* __restrict__ Y,
+    int ld_Y) {
+    constexpr int K = 16 * KB;
+    extern __shared__ v8bf sW[];                             // nblk limb images, then 32 nblk bias values
+    float* const sb = reinterpret_cast<float*>(sW + nblk * kLimbImage<KB>);
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), half = lane >> 5;
+    const int f_beg = blockIdx.y * nblk * 32;
+    const int nf = min(nblk * 32, F - f_beg);                // a multiple of 16
+    bool big = stage_limbs<KB>(sW, (nf + 31) / 32, [&](int blk, int f) {
+        const int ff = 32 * blk + f;
+        return ff < nf ? w + (int64_t)(f_beg + ff) * K : nullptr;
+    });
+    for (int f = tid; f < nf; f += blockDim.x) sb[f] = b ? b[f_beg + f] : 0.f;
+    big = __syncthreads_or(big);
+    const int64_t ntile = (E + 31) / 32, stride = (int64_t)gridDim.x * kLinWaves;
+    int64_t t = (int64_t)blockIdx.x * kLinWaves + __builtin_amdgcn_readfirstlane(tid / kWave);
     if (t >= ntile) return;
-    // X rows (B operands) and table rows of a tile's 16 BB edges; rows past E repeat edge E - 1
-    // (never stored). The next tile's rows are loaded while the current one computes, and moved
-    // in before its output blocks start, so that no load is outstanding inside the block loop:
-    // a wait there would also wait for the Y stores issued after it.
-    v4f xn[BB][KB];
-    int64_t trn[BB];
+    // rows past E repeat edge E - 1 (never stored); the next tile's rows are loaded while the current
+    // one computes
+    v4f xn[2 * KB];
+    int64_t rn = 0;
     auto load_tile = [&](int64_t tt) __attribute__((always_inline)) {
+        const int64_t e = min(tt * 32 + (lane & 31), E - 1);
 #pragma unroll
-        for (int bb = 0; bb < BB; ++bb) {
-            const int64_t e = tt * 16 * BB + 16 * bb + j;
-            const int64_t ec = e < E ? e : E - 1;
-#pragma unroll
-            for (int kb = 0; kb < KB; ++kb) xn[bb][kb] = ld4(X + ec * ld_X + 16 * kb + 4 * q);
-            trn[bb] = HAS_T ? (idx ? (int64_t)idx[ec] : ec) : 0;
+        for (int s = 0; s < KB; ++s) {
+            xn[2 * s] = ld4(X + e * ld_X + 16 * s + 8 * half);
+            xn[2 * s + 1] = ld4(X + e * ld_X + 16 * s + 8 * half + 4);
         }
+        if (HAS_T) rn = idx ? (int64_t)idx[e] : e;
     };
     load_tile(t);
     for (; t < ntile; t += stride) {
-        const int64_t e0 = t * 16 * BB;
-        v4f xv[BB][KB];
-        int64_t trow[BB];
+        const int64_t e = t * 32 + (lane & 31);
+        Split8 x[KB];
+        float mx = 0.f;
 #pragma unroll
-        for (int bb = 0; bb < BB; ++bb) {
-            trow[bb] = trn[bb];
-#pragma unroll
-            for (int kb = 0; kb < KB; ++kb) xv[bb][kb] = xn[bb][kb];
+        for (int s = 0; s < KB; ++s) {
+            x[s] = split8(xn[2 * s], xn[2 * s + 1]);
+            mx = max_abs8(xn[2 * s], xn[2 * s + 1], mx);
         }
+        const bool plain = big || __any(mx > kLimbMax);
+        const float* const Tr = HAS_T ? T + rn * ld_T + f_beg + 4 * half : nullptr;
         if (t + stride < ntile) load_tile(t + stride);
+        float* const Ye = Y + e * ld_Y + f_beg + 4 * half;
 #pragma unroll 1
-        for (int fb0 = 0; fb0 < nf; fb0 += 16 * FB) {
-            // epilogue operands, issued ahead of the products: the bias through scalar loads
-            // (16 features of a block are wave-uniform; lane (j, q) takes 4q .. 4q + 3), the
-            // table rows as vector loads
-            v4f bias[FB], tv[FB][BB];
+        for (int f0 = 0; f0 < nf; f0 += 32) {
+            const int ng = nf - f0 < 32 ? 2 : 4;             // groups of 8 features
+            v4f tv[4];
+            if (HAS_T) {
 #pragma unroll
-            for (int fb = 0; fb < FB; ++fb) {
-                const int fc = min(fb0 + 16 * fb, nf - 16);
-                bias[fb] = z4;
-                if (HAS_B) {
-                    const float* bp = b + f_beg + fc;
-                    float bs[16];
+                for (int g = 0; g < 4; ++g) tv[g] = ld4(Tr + f0 + (g < ng ? 8 * g : 0));
+            }
+            v16f acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            const v8bf* img = sW + (f0 / 32) * kLimbImage<KB>;
 #pragma unroll
-                    for (int u = 0; u < 16; ++u)      // wave-uniform values: scalar loads
-                        bs[u] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(bp[u])));
+            for (int s = 0; s < KB; ++s) acc = limb_step<false>(x[s], img + 3 * s * kWave, lane, acc);
+            if (plain) {
+                const float* xe = X + min(e, E - 1) * ld_X;
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) bias[fb][r] = q == 0 ? bs[r] : (q == 1 ? bs[4 + r] : (q == 2 ? bs[8 + r] : bs[12 + r]));
+                for (int r = 0; r < 16; ++r) {
+                    const float* wf = w + (int64_t)(f_beg + min(f0 + d_row(r) + 4 * half, nf - 1)) * K;
+                    float s = 0.f;
+#pragma unroll 1
+                    for (int k = 0; k < K; ++k) s = fmaf(xe[k], wf[k], s);
+                    acc[r] = s;
                 }
-#pragma unroll
-                for (int bb = 0; bb < BB; ++bb)
-                    tv[fb][bb] = HAS_T ? ld4(T + trow[bb] * ld_T + f_beg + fc + 4 * q) : z4;
-            }
-            v4f acc[FB][BB];
-#pragma unroll
-            for (int fb = 0; fb < FB; ++fb)
-#pragma unroll
-                for (int bb = 0; bb < BB; ++bb) acc[fb][bb] = z4;
-#pragma unroll
-            for (int kb = 0; kb < KB; ++kb) {
-                v4f wa[FB];
-#pragma unroll
-                for (int fb = 0; fb < FB; ++fb)
-                    wa[fb] = fb0 + 16 * fb < nf
-                                 ? lds4_at(sW, lin_off(fb0 + 16 * fb + j, 4 * kb + q, S, NCH, rt))
-                                 : z4;
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-#pragma unroll
-                    for (int fb = 0; fb < FB; ++fb)
-#pragma unroll
-                        for (int bb = 0; bb < BB; ++bb) acc[fb][bb] = mfma_16x16x4(wa[fb][r], xv[bb][kb][r], acc[fb][bb]);
             }
 #pragma unroll
-            for (int fb = 0; fb < FB; ++fb) {
-                if (fb0 + 16 * fb < nf) {
-                    const int f = f_beg + fb0 + 16 * fb + 4 * q;
+            for (int g = 0; g < 4; ++g) {
+                if (g < ng) {
+                    const v4f bs = lds4_at(sb, f0 + 8 * g + 4 * half);
+                    v4f y;
 #pragma unroll
-                    for (int bb = 0; bb < BB; ++bb) {
-                        const int64_t e = e0 + 16 * bb + j;
-                        if (e < E) st4(Y + e * ld_Y + f, acc[fb][bb] + bias[fb] + tv[fb][bb]);
-                    }
+                    for (int i = 0; i < 4; ++i) y[i] = acc[4 * g + i] + bs[i];
+                    if (HAS_T) y += tv[g];
+                    if (e < E) st4(Ye + f0 + 8 * g, y);
                 }
             }
         }
@@ -233,8 +200,6 @@ __global__ __launch_bounds__(kLinBwdWaves * kWave) void edge_linear_bwd_kernel(
     }
 }
 
-static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
-
 }  // namespace face
 
 using namespace face;
@@ -249,32 +214,22 @@ extern "C" int face_edge_linear_fwd(const float* x, int32_t ld_x, int64_t E, int
     if (ld_x % 4 || ld_y % 4 || (tab && ld_tab % 4) || !aligned16(x) || !aligned16(w) || !aligned16(y) ||
         (b && !aligned16(b)) || (tab && !aligned16(tab)))
         return FACE_ERR_UNSUPPORTED;
-    const int max_lds = device_max_lds();
-    int S = 0, rot = 0, f_chunk = 0;
-    if (!lin_layout(F, K, max_lds, S, rot, f_chunk)) return FACE_ERR_UNSUPPORTED;
-    const size_t lds = (size_t)f_chunk * S * sizeof(float);
-    // 32 edges per tile (BB = 2) for the plain head; the gathered-table form keeps 16 (BB = 1): its
-    // table rows (FB x BB float4 per lane) on top of the 32-edge operands spill at 16 waves
-    const int BB = tab ? 1 : 2;
-    constexpr int FB = 2;
-    const int64_t ntile = (E + 16 * BB - 1) / (16 * BB);
-    int64_t wgs = device_cu_count();                  // persistent: one 16-wave workgroup per CU
-    const int64_t need = (ntile + kLinWaves - 1) / kLinWaves;
+    const int all = (F + 31) / 32, parts = (all + kLinBlocks - 1) / kLinBlocks, nblk = (all + parts - 1) / parts;
+    const size_t lds = (size_t)nblk * (K / 16 * 3 * kWave * 16 + 32 * sizeof(float));
+    if ((int64_t)lds > device_max_lds()) return FACE_ERR_UNSUPPORTED;
+    int64_t wgs = std::max<int64_t>(1, 2 * (int64_t)device_cu_count() / parts);   // persistent, two workgroups per CU
+    const int64_t need = ((E + 31) / 32 + kLinWaves - 1) / kLinWaves;
     if (need < wgs) wgs = need;
-    const dim3 grid((unsigned)wgs, (unsigned)((F + f_chunk - 1) / f_chunk)), block(kLinWaves * kWave);
+    const dim3 grid((unsigned)wgs, (unsigned)((all + nblk - 1) / nblk)), block(kLinWaves * kWave);
     const hipStream_t st = (hipStream_t)stream;
 #define FACE_LINF(KB_)                                                                                        \
     do {                                                                                                      \
-        auto kern = b ? (tab ? edge_linear_fwd_kernel<KB_, 1, FB, true, true>                                 \
-                             : edge_linear_fwd_kernel<KB_, 2, FB, true, false>)                               \
-                      : (tab ? edge_linear_fwd_kernel<KB_, 1, FB, false, true>                                \
-                             : edge_linear_fwd_kernel<KB_, 2, FB, false, false>);                             \
+        auto kern = tab ? edge_linear_fwd_kernel<KB_, true> : edge_linear_fwd_kernel<KB_, false>;             \
         if (lds > 65536 &&                                                                                    \
             hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=    \
                 hipSuccess)                                                                                   \
             return FACE_ERR_UNSUPPORTED;                                                                      \
-        hipLaunchKernelGGL(kern, grid, block, lds, st, x, ld_x, E, w, b, F, f_chunk, S, rot, tab, ld_tab, idx, \
-                           y, ld_y);                                                                          \
+        hipLaunchKernelGGL(kern, grid, block, lds, st, x, ld_x, E, w, b, F, nblk, tab, ld_tab, idx, y, ld_y); \
     } while (0)
     switch (K / 16) {
         case 1: FACE_LINF(1); break;

@@ -890,13 +890,11 @@ class CPRadialDensity(torch.autograd.Function):
         row = graph.col if gathered else None
         h2_, w_, b_ = _aligned_rows(h2.detach()), _aligned16(w_cp.detach()), _aligned16(b_cp.detach())
         H = h2_.shape[1]
-        code = _lib.FACE_ERR_UNSUPPORTED
-        if not gathered:
-            R = torch.empty(graph.E, 4 * C, device=h2.device)
-            code = _lib.call_status("face_cp_radial_fwd", ptr(h2_), h2_.stride(0), H, ptr(w_), ptr(b_), ptr(env_),
-                                    ptr(msg_), ld_msg, None, ptr(Y_), ld_Y, ptr(graph.row_ptr), graph.N, graph.E, C,
-                                    *_lib.ranks_of_blocks(outs), ptr(R), 4 * C, _lib.stream_of(R),
-                                    label="cp_radial_fwd")
+        R = torch.empty(graph.E, 4 * C, device=h2.device)
+        code = _lib.call_status("face_cp_radial_fwd", ptr(h2_), h2_.stride(0), H, ptr(w_), ptr(b_), ptr(env_),
+                                ptr(msg_), ld_msg, ptr(row), ptr(Y_), ld_Y, ptr(graph.row_ptr), graph.N, graph.E, C,
+                                *_lib.ranks_of_blocks(outs), ptr(R), 4 * C, _lib.stream_of(R),
+                                label=_cp_label("cp_radial_fwd", gathered))
         if code == _lib.FACE_ERR_UNSUPPORTED:
             R = radial_head(h2_, w_, b_)                                                          # (E, 4C)
             call("face_cp_density_fwd", ptr(R), R.stride(0), ptr(env_), ptr(msg_), ld_msg, ptr(row), ptr(Y_), ld_Y,
