@@ -90,8 +90,13 @@ __global__ __launch_bounds__(kCrfWaves * kWave) __attribute__((amdgpu_waves_per_
     // per half), loaded while the tile before it computes; edges past the share repeat its last one
     v4f hn[2 * HB];
     float yn[10], xn;
+    const float* const x_lo = env ? env : Y;          // always a valid row: no branch around the load
+    const float* const x_hi = msg_row ? reinterpret_cast<const float*>(msg_row) : Y;
     auto load_tile = [&](int64_t t0) __attribute__((always_inline)) {
-        const int64_t e = min(t0 + (lane & 31), e_end - 1);
+        int ln = lane;                                // through an empty asm: addresses are formed here, not
+        asm volatile("" : "+v"(ln));                  // held for the whole launch
+        const int half = ln >> 5;
+        const int64_t e = min(t0 + (ln & 31), e_end - 1);
 #pragma unroll
         for (int s = 0; s < HB; ++s) {
             hn[2 * s] = ld4(h2 + e * ld_h2 + 16 * s + 8 * half);
@@ -99,7 +104,7 @@ __global__ __launch_bounds__(kCrfWaves * kWave) __attribute__((amdgpu_waves_per_
         }
         const float* ye = Y + e * ld_Y + 10 * half;
         __builtin_memcpy(yn, ye, sizeof(yn));         // rows of any alignment
-        xn = half ? (msg_row ? __builtin_bit_cast(float, msg_row[e]) : 0.f) : (env ? env[e] : 1.f);
+        xn = (half ? x_hi : x_lo)[e];
     };
     load_tile(e_beg);
     for (int64_t t0 = e_beg; t0 < e_end; t0 += 32) {
@@ -116,7 +121,7 @@ __global__ __launch_bounds__(kCrfWaves * kWave) __attribute__((amdgpu_waves_per_
             float* d = yt + (lane & 31) * kCrfRow + 12 * half;
 #pragma unroll
             for (int k = 0; k < 10; ++k) d[k] = yn[k];
-            yt[(lane & 31) * kCrfRow + 10 + half] = xn;
+            yt[(lane & 31) * kCrfRow + 10 + half] = half || env ? xn : 1.f;
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -132,8 +137,6 @@ __global__ __launch_bounds__(kCrfWaves * kWave) __attribute__((amdgpu_waves_per_
 #pragma unroll
             for (int r = 0; r < 16; ++r) me[r] = mt[(int64_t)min(d_row(r) + 4 * half, n - 1) * ld_msg + cc];
         }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) me[r] *= yl[d_row(r) * kCrfRow + 10];
         if (t0 + 32 < e_end) load_tile(t0 + 32);
         int64_t nxt = at;
         // ranks L0 .. L0 + NL - 1 (monomials X0 .. X1 - 1): R, its rows out, the pooling
@@ -146,11 +149,12 @@ __global__ __launch_bounds__(kCrfWaves * kWave) __attribute__((amdgpu_waves_per_
             for (int l = 0; l < NL; ++l)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[l][r] = 0.f;
+            limb_products<HB, NL, true>(
+                x, [&](int l) __attribute__((always_inline)) { return lds + (L0 + l) * kLimbImage<HB>; }, lane, acc);
+            if (L0 == 0) {                            // here, where the products have covered the loads
 #pragma unroll
-            for (int s = 0; s < HB; ++s)
-#pragma unroll
-                for (int l = 0; l < NL; ++l)
-                    acc[l] = limb_step<true>(x[s], lds + ((L0 + l) * HB + s) * 3 * kWave, lane, acc[l]);
+                for (int r = 0; r < 16; ++r) me[r] *= yl[d_row(r) * kCrfRow + 10];
+            }
             if (plain) {                              // a row at a time: this branch holds few registers
                 int64_t row0 = t0 * ld_h2;            // (and its addresses stay in it)
                 int last = n - 1;

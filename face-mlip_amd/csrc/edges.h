@@ -115,20 +115,34 @@ __device__ __forceinline__ bool stage_limbs(v8bf* img, int nblk, Row row) {
     return big > kLimbMax;
 }
 
-// acc += x w over one 16-input step, EDGES the rows (A operand) or the columns (B operand) of D.
-template <bool EDGES_ARE_ROWS>
-__device__ __forceinline__ v16f limb_step(const Split8& x, const v8bf* w, int lane, v16f acc) {
-    const v8bf wh = w[lane], wm = w[kWave + lane], wl = w[2 * kWave + lane];
-    auto mm = [&](v8bf xe, v8bf we) __attribute__((always_inline)) {
-        acc = EDGES_ARE_ROWS ? mfma_32x32x16(xe, we, acc) : mfma_32x32x16(we, xe, acc);
-    };
-    mm(x.l, wh);
-    mm(x.h, wl);
-    mm(x.m, wm);
-    mm(x.m, wh);
-    mm(x.h, wm);
-    mm(x.h, wh);
-    return acc;
+// acc[l] += x w_l over all 16-input steps for NL feature blocks (images img(l)), EDGES the rows (A operand)
+// or the columns (B operand) of D. One operand's registers hold the next operand as soon as its last
+// product is issued, so every read has 3 to 5 products (96 to 160 cycles) to arrive and the weights take
+// 12 registers; the barriers keep that order (left to itself the compiler waits for each read).
+template <int HB, int NL, bool EDGES_ARE_ROWS, typename Img>
+__device__ __forceinline__ void limb_products(const Split8 (&x)[HB], Img img, int lane, v16f (&acc)[NL]) {
+    v8bf w0 = img(0)[lane], w1 = img(0)[kWave + lane], w2 = img(0)[2 * kWave + lane];
+#pragma unroll
+    for (int i = 0; i < HB * NL; ++i) {
+        const int s = i / NL, l = i % NL;
+        const bool more = i + 1 < HB * NL;
+        const v8bf* nx = img((i + 1) % NL) + (more ? (i + 1) / NL : 0) * 3 * kWave + lane;
+        auto mm = [&](v8bf xe, v8bf we) __attribute__((always_inline)) {
+            acc[l] = EDGES_ARE_ROWS ? mfma_32x32x16(xe, we, acc[l]) : mfma_32x32x16(we, xe, acc[l]);
+        };
+        mm(x[s].h, w2);
+        if (more) w2 = nx[2 * kWave];
+        __builtin_amdgcn_sched_barrier(0);
+        mm(x[s].m, w1);
+        mm(x[s].h, w1);
+        if (more) w1 = nx[kWave];
+        __builtin_amdgcn_sched_barrier(0);
+        mm(x[s].l, w0);
+        mm(x[s].m, w0);
+        mm(x[s].h, w0);
+        if (more) w0 = nx[0];
+        __builtin_amdgcn_sched_barrier(0);
+    }
 }
 
 // Row (of 32) that register r of a lane holds in the layout of D.

@@ -78,10 +78,12 @@ __global__ __launch_bounds__(kLinWaves * kWave) __attribute__((amdgpu_waves_per_
 #pragma unroll
                 for (int g = 0; g < 4; ++g) tv[g] = ld4(Tr + f0 + (g < ng ? 8 * g : 0));
             }
-            v16f acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            const v8bf* img = sW + (f0 / 32) * kLimbImage<KB>;
+            v16f ac[1];
 #pragma unroll
-            for (int s = 0; s < KB; ++s) acc = limb_step<false>(x[s], img + 3 * s * kWave, lane, acc);
+            for (int r = 0; r < 16; ++r) ac[0][r] = 0.f;
+            limb_products<KB, 1, false>(
+                x, [&](int) __attribute__((always_inline)) { return sW + (f0 / 32) * kLimbImage<KB>; }, lane, ac);
+            v16f& acc = ac[0];
             if (plain) {
                 const float* xe = X + min(e, E - 1) * ld_X;
 #pragma unroll
