@@ -19,7 +19,8 @@ ARCH = os.environ.get("FACE_OFFLOAD_ARCH", "gfx950")
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang",
          "-packed-fp32-ops", "-Wall"]
 # graph.hip evaluates the pair-acceptance test in fp64 with a fixed operation order: no contraction.
-SOURCES = {"capi.hip": "fast", "density.hip": "fast", "cprad.hip": "fast", "node.hip": "fast", "edge.hip": "fast", "graph.hip": "off",
+SOURCES = {"capi.hip": "fast", "density.hip": "fast", "cprad.hip": "fast", "densfac.hip": "fast", "node.hip": "fast",
+           "edge.hip": "fast", "graph.hip": "off",
            "transport.hip": "fast", "radial.hip": "fast", "linear.hip": "fast",
            "gemm.hip": "fast", "gemm_xs.hip": "fast", "gemm_split.hip": "fast", "gemm_op.hip": "fast", "densmix.hip": "fast"}
 
@@ -39,7 +40,8 @@ def stale(src):
     if not os.path.exists(obj):
         return True
     t = os.path.getmtime(obj)
-    return any(os.path.getmtime(os.path.join(HERE, f)) > t for f in (src, "common.h", "edges.h", "rows_gemm.h", "../../include/face_hip.h"))
+    return any(os.path.getmtime(os.path.join(HERE, f)) > t
+               for f in (src, "common.h", "edges.h", "densfac.h", "rows_gemm.h", "../../include/face_hip.h"))
 
 
 def build(jobs=None, verbose=False, changed_only=False):

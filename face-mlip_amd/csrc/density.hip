@@ -10,7 +10,7 @@
 // column c) lives at p[l(x)] + i*sa + (x - x0(l))*sx + c. The reference layout (N, NX, W) is
 // p[l] = base + x0(l)*W, sa = NX*W, sx = W; the model keeps each rank as its own (k_l, N, W)
 // tensor (p[l] = D_l, sa = W, sx = N*W) so the channel-mixing GEMMs read contiguous blocks.
-#include "edges.h"
+#include "densfac.h"
 
 #include <algorithm>
 #include <cstdlib>
@@ -280,418 +280,6 @@ __global__ __launch_bounds__(kBlock) void density_bwd_kernel(
                 for (int kk = 0; kk < KS; ++kk) {
                     const int k = g * KS + kk;
                     if (k < K) dmsg[e * ld_dmsg + k] = dmg[kk];
-                }
-            }
-        }
-    }
-}
-
-// ------------------------------------------------------------------ factor backward on MFMA
-// B = 16 basis functions, NX = 20 monomials, K = 16 KB message channels: with the columns of
-// G[i] flattened as (x, b), the 16-column block x is monomial x. Tiles of 16 edges; per monomial
-// x two v_mfma_f32_16x16x4f32 chains:
-//   S[e, b]  = sum_k msg[e, k] G[x, b, k]       (A = msg rows, K index q of instruction r of chunk
-//                                                c = channel 16 c + 4q + r; B = G rows)
-//   dmsg[e, k] += sum_b Y[e, x] phi[e, b] G[x, b, k]   (A = Y[e, x] phi[e, :], K index q of
-//                                                instruction r = basis 4q + r; B = G columns)
-// both with edge 4q + r in register r of lane j + 16q (column j = basis b, resp. channel k).
-// From S: dphi[e, b] += S Y[e, x], and dY[e, x] = sum_b S phi[e, b], a sum over the 16 lanes
-// of a row group. WPA = 1: one wave per atom (kDbWaves atoms per workgroup). WPA > 1: one atom
-// per workgroup, its WPA waves split the monomials and sum their dphi / dmsg partials in LDS
-// (small systems, where one wave per atom leaves the SIMDs idle).
-constexpr int kDbWaves = 8;
-constexpr int kDbYS = 21;                                // Y tile row stride (floats)
-
-template <int KB, int WPA>
-__global__ __launch_bounds__((WPA > 1 ? WPA : kDbWaves) * kWave) void density_bwd_mfma_kernel(
-    const float* __restrict__ phi, int ld_phi, const float* __restrict__ msg, int ld_msg,
-    const int32_t* __restrict__ msg_row, const float* __restrict__ Y, int ld_Y, const int32_t* __restrict__ row_ptr,
-    int64_t N, int M, RankIn G, float* __restrict__ dphi, int ld_dphi, float* __restrict__ dmsg, int ld_dmsg,
-    float* __restrict__ dY, int ld_dY) {
-    constexpr int K = 16 * KB, NXW = 20 / WPA, NSLOT = (NXW + 15) / 16;
-    constexpr int YW = WPA > 1 ? 1 : kDbWaves;           // Y tiles: one per atom of the workgroup
-    constexpr int PW = WPA > 1 ? WPA : 1;
-    __shared__ float sY[YW][16 * kDbYS];
-    __shared__ float sP[PW][16 * (16 + K)];               // dphi | dmsg partials (WPA > 1)
-    const int lane = threadIdx.x & (kWave - 1), j = lane & 15, q = lane >> 4;
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int64_t n = WPA > 1 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * kDbWaves + wv;
-    if (n >= N) return;                                  // WPA = 1 only: no workgroup barrier there
-    const int x0 = WPA > 1 ? wv * NXW : 0;
-    float* ys = sY[WPA > 1 ? 0 : wv];
-    const v4f z4 = {0.f, 0.f, 0.f, 0.f};
-    int64_t a, bnd;
-    row_range(row_ptr, n, M, a, bnd);
-    for (int64_t e0 = a; e0 < bnd; e0 += 16) {
-        const int ne = (int)min((int64_t)16, bnd - e0);
-        // the tile's Y (16 x 20) into LDS, zero past the row end
-        if (WPA > 1) {
-            __syncthreads();                             // previous tile's Y and partials consumed
-            for (int v = threadIdx.x; v < 320; v += WPA * kWave) {
-                const int t = v / 20, x = v - t * 20;
-                ys[t * kDbYS + x] = t < ne ? Y[(e0 + t) * ld_Y + x] : 0.f;
-            }
-            __syncthreads();
-        } else {
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int u = 0; u < 5; ++u) {
-                const int v = u * kWave + lane, t = v / 20, x = v - t * 20;
-                ys[t * kDbYS + x] = t < ne ? Y[(e0 + t) * ld_Y + x] : 0.f;
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-        // edge e0 + j: message row and phi[4q .. 4q + 3] (A operands), zero past the row end
-        const bool oki = j < ne;
-        const int64_t ei = e0 + min(j, ne - 1);
-        const int64_t rowi = msg_row ? (int64_t)msg_row[ei] : ei;
-        v4f mA[KB];
-#pragma unroll
-        for (int c = 0; c < KB; ++c) mA[c] = oki ? ld4(msg + rowi * ld_msg + 16 * c + 4 * q) : z4;
-        const v4f ph4 = oki ? ld4(phi + ei * ld_phi + 4 * q) : z4;
-        // edges e0 + 4q + r at basis j (for dY)
-        float phT[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) phT[r] = phi[(e0 + min(4 * q + r, ne - 1)) * ld_phi + j];
-        v4f dph = z4, dm[KB];
-#pragma unroll
-        for (int c = 0; c < KB; ++c) dm[c] = z4;
-        float dyk[4][NSLOT];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int sl = 0; sl < NSLOT; ++sl) dyk[r][sl] = 0.f;
-#pragma unroll 2
-        for (int xx = 0; xx < NXW; ++xx) {
-            const int x = x0 + xx;
-            const float* gx = G.at(n, x);                // (16 b) x K
-            v4f sv = z4;
-#pragma unroll
-            for (int c = 0; c < KB; ++c) {
-                const v4f gv = ld4(gx + j * K + 16 * c + 4 * q);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) sv = mfma_16x16x4(mA[c][r], gv[r], sv);
-            }
-            const float yi = ys[j * kDbYS + x];
-#pragma unroll
-            for (int c = 0; c < KB; ++c)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) dm[c] = mfma_16x16x4(yi * ph4[r], gx[(4 * q + r) * K + 16 * c + j], dm[c]);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                dph[r] = fmaf(sv[r], ys[(4 * q + r) * kDbYS + x], dph[r]);
-                float v = sv[r] * phT[r];
-                v = row16_sum(v);
-                if (j == (xx & 15)) dyk[r][xx >> 4] = v;
-            }
-        }
-        // dY of this wave's monomials
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int t = 4 * q + r;
-            if (dY && t < ne) {
-#pragma unroll
-                for (int sl = 0; sl < NSLOT; ++sl)
-                    if (16 * sl + j < NXW) dY[(e0 + t) * ld_dY + x0 + 16 * sl + j] = dyk[r][sl];
-            }
-        }
-        if (WPA > 1) {
-            // partials of the WPA waves summed by wave 0
-            float* mine = sP[wv];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                mine[(4 * q + r) * 16 + j] = dph[r];
-#pragma unroll
-                for (int c = 0; c < KB; ++c) mine[256 + (4 * q + r) * K + 16 * c + j] = dm[c][r];
-            }
-            __syncthreads();
-            if (wv == 0) {
-#pragma unroll
-                for (int w = 1; w < WPA; ++w) {
-                    const float* o = sP[w];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        dph[r] += o[(4 * q + r) * 16 + j];
-#pragma unroll
-                        for (int c = 0; c < KB; ++c) dm[c][r] += o[256 + (4 * q + r) * K + 16 * c + j];
-                    }
-                }
-            }
-        }
-        if (WPA == 1 || wv == 0) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int t = 4 * q + r;
-                if (t < ne) {
-                    const int64_t e = e0 + t;
-                    if (dphi) dphi[e * ld_dphi + j] = dph[r];
-                    if (dmsg) {
-#pragma unroll
-                        for (int c = 0; c < KB; ++c) dmsg[e * ld_dmsg + 16 * c + j] = dm[c][r];
-                    }
-                }
-            }
-        }
-    }
-}
-
-// ------------------------------------------------------------------ factor backward, small systems
-// One atom per workgroup of 4 waves, wave w on monomials 5w .. 5w + 4 (the per-monomial MFMA
-// chains of density_bwd_mfma_kernel), for K <= 32. The wave's G operands (5 monomials x 16 b x K,
-// both operand layouts: 80 registers at K = 32) are read once per atom, while the first tile's
-// rows load, and stay in registers over the atom's tiles; per 16-edge tile the Y tile, the message
-// rows and phi are issued together before the workgroup barrier. A tile then costs one memory
-// latency instead of one per pair of monomials (the G reads of density_bwd_mfma_kernel). The
-// four waves' dphi / dmsg partials are summed through LDS by all four. At K = 32 the kernel holds
-// ~230 registers (two waves per SIMD); capped at four waves per SIMD it spills 312 bytes and runs
-// 1.8x slower. Measured against density_bwd_mfma_kernel<2, 4>: 35.5 -> 27.3 us (864-atom FCC),
-// 37.6 -> 32.3 us (1,344 atoms), 153 -> 113 us (2,000 atoms of 70 neighbours), same bits.
-constexpr int kDsWaves = 4;
-
-template <int KB>
-__global__ __launch_bounds__(kDsWaves * kWave) void density_bwd_split_kernel(
-    const float* __restrict__ phi, int ld_phi, const float* __restrict__ msg, int ld_msg,
-    const int32_t* __restrict__ msg_row, const float* __restrict__ Y, int ld_Y, const int32_t* __restrict__ row_ptr,
-    int M, RankIn G, float* __restrict__ dphi, int ld_dphi, float* __restrict__ dmsg, int ld_dmsg,
-    float* __restrict__ dY, int ld_dY) {
-    constexpr int K = 16 * KB, NXW = 20 / kDsWaves;
-    __shared__ float sY[16 * kDbYS];
-    __shared__ float sP[kDsWaves][16 * (16 + K)];        // dphi | dmsg partials
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), j = lane & 15, q = lane >> 4;
-    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int64_t n = blockIdx.x;
-    const int x0 = wv * NXW;
-    const v4f z4 = {0.f, 0.f, 0.f, 0.f};
-    // G_x operands: gv = G[x][b = j][16c + 4q .. + 3] (S chain), gs = G[x][b = 4q + r][16c + j] (dmsg chain)
-    v4f gv[NXW][KB];
-    float gs[NXW][KB][4];
-#pragma unroll
-    for (int xx = 0; xx < NXW; ++xx) {
-        const float* gx = G.at(n, x0 + xx);
-#pragma unroll
-        for (int c = 0; c < KB; ++c) {
-            gv[xx][c] = ld4(gx + j * K + 16 * c + 4 * q);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) gs[xx][c][r] = gx[(4 * q + r) * K + 16 * c + j];
-        }
-    }
-    int64_t a, bnd;
-    row_range(row_ptr, n, M, a, bnd);
-    for (int64_t e0 = a; e0 < bnd; e0 += 16) {
-        const int ne = (int)min((int64_t)16, bnd - e0);
-        // this tile's loads, all issued before the barrier: the Y tile (16 x 20, zero past the row
-        // end; 320 values over 256 threads), the message row and phi of edge e0 + j, phi of edges
-        // e0 + 4q + r at basis j
-        float yl[2];
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int v = u * kDsWaves * kWave + tid, t = v / 20, x = v - t * 20;
-            yl[u] = (v < 320 && t < ne) ? Y[(e0 + t) * ld_Y + x] : 0.f;
-        }
-        const bool oki = j < ne;
-        const int64_t ei = e0 + min(j, ne - 1);
-        const int64_t rowi = msg_row ? (int64_t)msg_row[ei] : ei;
-        v4f mA[KB];
-#pragma unroll
-        for (int c = 0; c < KB; ++c) mA[c] = oki ? ld4(msg + rowi * ld_msg + 16 * c + 4 * q) : z4;
-        const v4f ph4 = oki ? ld4(phi + ei * ld_phi + 4 * q) : z4;
-        float phT[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) phT[r] = phi[(e0 + min(4 * q + r, ne - 1)) * ld_phi + j];
-        __syncthreads();                                 // previous tile's Y and partials consumed
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int v = u * kDsWaves * kWave + tid, t = v / 20, x = v - t * 20;
-            if (v < 320) sY[t * kDbYS + x] = yl[u];
-        }
-        __syncthreads();
-        v4f dph = z4, dm[KB];
-#pragma unroll
-        for (int c = 0; c < KB; ++c) dm[c] = z4;
-        float dyk[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) dyk[r] = 0.f;
-#pragma unroll
-        for (int xx = 0; xx < NXW; ++xx) {
-            const int x = x0 + xx;
-            v4f sv = z4;
-#pragma unroll
-            for (int c = 0; c < KB; ++c)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) sv = mfma_16x16x4(mA[c][r], gv[xx][c][r], sv);
-            const float yi = sY[j * kDbYS + x];
-#pragma unroll
-            for (int c = 0; c < KB; ++c)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) dm[c] = mfma_16x16x4(yi * ph4[r], gs[xx][c][r], dm[c]);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                dph[r] = fmaf(sv[r], sY[(4 * q + r) * kDbYS + x], dph[r]);
-                float v = sv[r] * phT[r];
-                v = row16_sum(v);
-                if (j == xx) dyk[r] = v;
-            }
-        }
-        // dY of this wave's monomials: lane j < 5 holds monomial x0 + j of edge e0 + 4q + r
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int t = 4 * q + r;
-            if (dY && t < ne && j < NXW) dY[(e0 + t) * ld_dY + x0 + j] = dyk[r];
-        }
-        // partials of the four waves, summed by all four: thread tid takes values tid, tid + 256, ...
-        // of the block (dphi | dmsg), adding the waves' partials in wave order (one wave doing all
-        // the sums and stores left the other three waiting at the next tile's barrier: 864 atoms
-        // 27.6 -> 27.0 us, 64 molecules 32.1 -> 31.0 us)
-        float* mine = sP[wv];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            mine[(4 * q + r) * 16 + j] = dph[r];
-#pragma unroll
-            for (int c = 0; c < KB; ++c) mine[256 + (4 * q + r) * K + 16 * c + j] = dm[c][r];
-        }
-        __syncthreads();
-        constexpr int NV = 16 * (16 + K), NU = (NV + kDsWaves * kWave - 1) / (kDsWaves * kWave);
-#pragma unroll
-        for (int u = 0; u < NU; ++u) {
-            const int v = u * kDsWaves * kWave + tid;
-            if (v < NV) {
-                float sum = sP[0][v];
-#pragma unroll
-                for (int w = 1; w < kDsWaves; ++w) sum += sP[w][v];
-                if (v < 256) {
-                    const int t = v >> 4, b = v & 15;
-                    if (dphi && t < ne) dphi[(e0 + t) * ld_dphi + b] = sum;
-                } else {
-                    const int t = (v - 256) / K, k = (v - 256) - t * K;
-                    if (dmsg && t < ne) dmsg[(e0 + t) * ld_dmsg + k] = sum;
-                }
-            }
-        }
-    }
-}
-
-// ------------------------------------------------------------------ factor backward, G in LDS
-// Large systems (long rows, K up to 64): one workgroup of 4 waves per atom stages the atom's G
-// (20 x 16 x K) in LDS in two halves of 10 monomials (row stride K + 4: the 16 rows one
-// instruction reads sit on distinct banks), so that G is read from memory once per group of 4
-// edge tiles of the atom instead of once per tile and monomial. Wave w takes tile w of each
-// group and keeps its operands (msg, phi) and accumulators (dphi, dmsg) in registers over both
-// halves; per monomial the two MFMA chains of density_bwd_mfma_kernel run against the LDS copy,
-// and dY[e, x] is complete per monomial.
-constexpr int kDbLWaves = 4;
-
-template <int KB>
-__global__ __launch_bounds__(kDbLWaves * kWave) void density_bwd_lds_kernel(
-    const float* __restrict__ phi, int ld_phi, const float* __restrict__ msg, int ld_msg,
-    const int32_t* __restrict__ msg_row, const float* __restrict__ Y, int ld_Y, const int32_t* __restrict__ row_ptr,
-    RankIn G, float* __restrict__ dphi, int ld_dphi, float* __restrict__ dmsg, int ld_dmsg, float* __restrict__ dY,
-    int ld_dY) {
-    constexpr int K = 16 * KB, GS = K + 4, XH = 10;
-    __shared__ float sG[XH * 16 * GS];
-    __shared__ float sY[kDbLWaves][16 * kDbYS];
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), j = lane & 15, q = lane >> 4;
-    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int64_t n = blockIdx.x;
-    const v4f z4 = {0.f, 0.f, 0.f, 0.f};
-    const int64_t a = row_ptr[n], bnd = row_ptr[n + 1];
-    const int ntile = (int)((bnd - a + 15) / 16);
-    float* ys = sY[wv];
-#pragma unroll 1
-    for (int g0 = 0; g0 < ntile; g0 += kDbLWaves) {
-        // this wave's tile of the group: operands and accumulators
-        const int t = g0 + wv;
-        const int64_t e0 = a + 16 * (int64_t)t;
-        const int ne = t < ntile ? (int)min((int64_t)16, bnd - e0) : 0;
-        v4f mA[KB], ph4 = z4, dph = z4, dm[KB];
-        float phT[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int c = 0; c < KB; ++c) dm[c] = mA[c] = z4;
-        if (ne > 0) {
-#pragma unroll
-            for (int u = 0; u < 5; ++u) {
-                const int v = u * kWave + lane, tt = v / 20, x = v - tt * 20;
-                ys[tt * kDbYS + x] = tt < ne ? Y[(e0 + tt) * ld_Y + x] : 0.f;
-            }
-            const bool oki = j < ne;
-            const int64_t ei = e0 + min(j, ne - 1);
-            const int64_t rowi = msg_row ? (int64_t)msg_row[ei] : ei;
-#pragma unroll
-            for (int c = 0; c < KB; ++c) mA[c] = oki ? ld4(msg + rowi * ld_msg + 16 * c + 4 * q) : z4;
-            ph4 = oki ? ld4(phi + ei * ld_phi + 4 * q) : z4;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) phT[r] = phi[(e0 + min(4 * q + r, ne - 1)) * ld_phi + j];
-        }
-#pragma unroll 1
-        for (int h = 0; h < 2; ++h) {
-            // stage G[x0 .. x0 + 9] of the atom: 16 rows of K per monomial, row stride GS
-            __syncthreads();                                   // previous half (or group) consumed
-            const int x0 = XH * h;
-            constexpr int NV = XH * 16 * K / 4;
-            for (int v0 = 0; v0 < NV; v0 += 4 * kDbLWaves * kWave) {
-                v4f b4[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int v = v0 + u * kDbLWaves * kWave + tid;
-                    if (v < NV) {
-                        const int xl = v / (4 * K), rem = v - xl * 4 * K;        // rem: float4 index in (16, K)
-                        b4[u] = ld4(G.at(n, x0 + xl) + 4 * rem);
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int v = v0 + u * kDbLWaves * kWave + tid;
-                    if (v < NV) {
-                        const int xl = v / (4 * K), rem = v - xl * 4 * K, b = rem / (K / 4), k4 = rem - b * (K / 4);
-                        st4(sG + (xl * 16 + b) * GS + 4 * k4, b4[u]);
-                    }
-                }
-            }
-            __syncthreads();
-            if (ne > 0) {
-                float dyk[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-                for (int xl = 0; xl < XH; ++xl) {
-                    const int x = x0 + xl;
-                    const float* gx = sG + xl * 16 * GS;
-                    v4f sv = z4;
-#pragma unroll
-                    for (int c = 0; c < KB; ++c) {
-                        const v4f gv = *reinterpret_cast<const v4f*>(gx + j * GS + 16 * c + 4 * q);
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) sv = mfma_16x16x4(mA[c][r], gv[r], sv);
-                    }
-                    const float yi = ys[j * kDbYS + x];
-#pragma unroll
-                    for (int c = 0; c < KB; ++c)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            dm[c] = mfma_16x16x4(yi * ph4[r], gx[(4 * q + r) * GS + 16 * c + j], dm[c]);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        dph[r] = fmaf(sv[r], ys[(4 * q + r) * kDbYS + x], dph[r]);
-                        float v = sv[r] * phT[r];
-                        v = row16_sum(v);
-                        if (j == xl) dyk[r] = v;
-                    }
-                }
-                if (dY && j < XH) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int te = 4 * q + r;
-                        if (te < ne) dY[(e0 + te) * ld_dY + x0 + j] = dyk[r];
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int te = 4 * q + r;
-            if (te < ne) {
-                const int64_t e = e0 + te;
-                if (dphi) dphi[e * ld_dphi + j] = dph[r];
-                if (dmsg) {
-#pragma unroll
-                    for (int c = 0; c < KB; ++c) dmsg[e * ld_dmsg + 16 * c + j] = dm[c][r];
                 }
             }
         }
@@ -1679,15 +1267,6 @@ extern "C" int face_density_fwd(const float* phi, int32_t ld_phi, const float* m
     return launch_fwd_nx<4>(cpt, grid, lds, st, phi, ld_phi, msg, ld_msg, msg_row, Y, ld_Y, row_ptr, M, B, K, D);
 }
 
-// Route of the factor backward for CSR rows: G staged in LDS per atom for systems of at least 64
-// atoms per CU (density_bwd_lds_kernel), the per-wave kernel below that. FACE_DENSITY_BWD_LDS=0 / 1
-// in the environment forces either (read on every call).
-static bool use_lds_bwd(int64_t N) {
-    const char* e = getenv("FACE_DENSITY_BWD_LDS");
-    if (e && (e[0] == '0' || e[0] == '1')) return e[0] == '1';
-    return N >= (int64_t)device_cu_count() * 64;
-}
-
 extern "C" int face_density_bwd(const float* phi, int32_t ld_phi, const float* msg, int32_t ld_msg,
                                 const int32_t* msg_row, const float* Y, int32_t ld_Y, int32_t NX,
                                 const int32_t* row_ptr, int64_t N, int32_t M, int32_t max_row, int32_t B, int32_t K,
@@ -1701,52 +1280,13 @@ extern "C" int face_density_bwd(const float* phi, int32_t ld_phi, const float* m
     RankIn G;
     if (!phi || !msg || !Y || !rank_in(G_ranks, atom_stride, x_stride, NX, G)) return FACE_ERR_ARG;
     hipStream_t st = (hipStream_t)stream;
-    // matrix cores: 20 monomials, B = 16, whole 16-channel blocks, 16-byte aligned rows
-    if (NX == 20 && B == 16 && K % 16 == 0 && K <= 64 && ld_phi % 4 == 0 && ld_msg % 4 == 0 && G.sa % 4 == 0 &&
-        G.sx % 4 == 0 && ((uintptr_t)phi & 15) == 0 && ((uintptr_t)msg & 15) == 0 && ((uintptr_t)G.p[0] & 15) == 0 &&
-        ((uintptr_t)G.p[1] & 15) == 0 && ((uintptr_t)G.p[2] & 15) == 0 && ((uintptr_t)G.p[3] & 15) == 0) {
-        // CSR rows of large systems: G staged in LDS per atom (read once), see density_bwd_lds_kernel
-        if (row_ptr && use_lds_bwd(N)) {
-#define FACE_DBL(KB_)                                                                                          \
-    hipLaunchKernelGGL((density_bwd_lds_kernel<KB_>), dim3((unsigned)N), dim3(kDbLWaves * kWave), 0, st, phi,   \
-                       ld_phi, msg, ld_msg, msg_row, Y, ld_Y, row_ptr, G, dphi, ld_dphi, dmsg, ld_dmsg, dY, ld_dY)
-            switch (K / 16) {
-                case 1: FACE_DBL(1); break;
-                case 2: FACE_DBL(2); break;
-                case 3: FACE_DBL(3); break;
-                default: FACE_DBL(4); break;
-            }
-#undef FACE_DBL
-            FACE_LAUNCH_CHECK();
-            return 0;
-        }
-        // small systems: split each atom's monomials over 4 waves (one atom per workgroup)
-        const bool split = N < (int64_t)device_cu_count() * 16;
-        const dim3 grid(split ? (unsigned)N : (unsigned)((N + kDbWaves - 1) / kDbWaves));
-        const dim3 block(split ? 4 * kWave : kDbWaves * kWave);
-#define FACE_DBM(KB_)                                                                                           \
-    do {                                                                                                        \
-        if (split && KB_ <= 2)                                                                                  \
-            hipLaunchKernelGGL((density_bwd_split_kernel<(KB_ <= 2 ? KB_ : 2)>), grid, block, 0, st, phi, ld_phi, \
-                               msg, ld_msg, msg_row, Y, ld_Y, row_ptr, M, G, dphi, ld_dphi, dmsg, ld_dmsg, dY,   \
-                               ld_dY);                                                                          \
-        else if (split)                                                                                         \
-            hipLaunchKernelGGL((density_bwd_mfma_kernel<KB_, 4>), grid, block, 0, st, phi, ld_phi, msg, ld_msg,  \
-                               msg_row, Y, ld_Y, row_ptr, N, M, G, dphi, ld_dphi, dmsg, ld_dmsg, dY, ld_dY);     \
-        else                                                                                                    \
-            hipLaunchKernelGGL((density_bwd_mfma_kernel<KB_, 1>), grid, block, 0, st, phi, ld_phi, msg, ld_msg,  \
-                               msg_row, Y, ld_Y, row_ptr, N, M, G, dphi, ld_dphi, dmsg, ld_dmsg, dY, ld_dY);     \
-    } while (0)
-        switch (K / 16) {
-            case 1: FACE_DBM(1); break;
-            case 2: FACE_DBM(2); break;
-            case 3: FACE_DBM(3); break;
-            default: FACE_DBM(4); break;
-        }
-#undef FACE_DBM
-        FACE_LAUNCH_CHECK();
-        return 0;
-    }
+    // matrix cores: 20 monomials, B = 16, whole 16-channel blocks, 16-byte aligned rows of the messages
+    // and the upstream gradient
+    if (NX == 20 && B == 16 && K % 16 == 0 && K <= 64 && ld_msg % 4 == 0 && G.sa % 4 == 0 && G.sx % 4 == 0 &&
+        ((uintptr_t)msg & 15) == 0 && ((uintptr_t)G.p[0] & 15) == 0 && ((uintptr_t)G.p[1] & 15) == 0 &&
+        ((uintptr_t)G.p[2] & 15) == 0 && ((uintptr_t)G.p[3] & 15) == 0)
+        return launch_density_bwd_limb(phi, ld_phi, msg, ld_msg, msg_row, Y, ld_Y, row_ptr, N, M, max_row, K, G, dphi,
+                                       ld_dphi, dmsg, ld_dmsg, dY, ld_dY, st);
     int ks = 8, glog = 2, nthr = 128;
     if (!plan_bwd(K, max_row, ks, glog, nthr)) return FACE_ERR_UNSUPPORTED;
     if (NX == 20)

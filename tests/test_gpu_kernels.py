@@ -1455,3 +1455,53 @@ def test_table_linears_match_torch(N, C, n):
     want = torch.autograd.grad((Vr * gv.double().cpu()).sum() + (Mr * gm.double().cpu()).sum(), (Vc, Mc))
     errs = [rel(Vb, Vr), rel(Mb, Mr)] + [rel(a, b) for a, b in zip(got, want)]
     assert max(errs) < 1e-5, errs
+
+
+@pytest.mark.parametrize("counts,K,huge", [
+    ([1, 0, 31, 32, 33, 5], 16, None), ([64, 65, 0, 2, 40], 32, None), ([96, 97, 130, 1, 64], 48, None),
+    ([70, 96, 33, 200, 0], 64, None), ([7, 30], 64, None), ([40, 3, 70], 32, "msg"), ([40, 3, 70], 32, "G"),
+    ([40, 3, 70], 32, "Y")])
+def test_factor_density_backward_row_lengths(counts, K, huge):
+    """Row lengths around the 32-edge tiles and the chunks of 32, 64 and 96 edges, gathered messages, against
+    fp64; one value past the largest bf16 (no finite limbs) leaves every other atom's results finite and
+    its own as plain fp32 gives them."""
+    from face_amd import _lib, ops
+    N, E, M = len(counts), sum(counts), max(counts)
+    say("factor density bwd", counts, K, huge)
+    torch.manual_seed(K + E)
+    row_ptr = torch.as_tensor(np.concatenate([[0], np.cumsum(counts)]).astype(np.int32), device=DEV)
+    col = torch.randint(0, N, (E,), dtype=torch.int32, device=DEV)
+    phi, Y = torch.randn(E, 21, device=DEV)[:, :16], torch.randn(E, 20, device=DEV)
+    msg = torch.randn(N, K, device=DEV)
+    G = [torch.randn(k, N, 16 * K, device=DEV) for k in ops.RANK_K]
+    if huge in ("msg", "Y"):                 # the other factors small: fp32 sums of the products stay in range
+        G = [g * 1e-3 for g in G]
+        phi *= 1e-3
+        if huge == "msg":
+            msg[1, 3] = 3.39e38
+            Y *= 1e-3
+        else:
+            Y[1, 4] = 3.4e38
+            msg *= 1e-3
+    if huge == "G":
+        G[2][1, 2, 5] = float("inf")
+    dphi, dmsg, dY = (torch.full((E, w), float("nan"), device=DEV) for w in (16, K, 20))
+    P = _lib.ptr
+    _lib.call("face_density_bwd", P(phi), 21, P(msg), K, P(col), P(Y), 20, 20, P(row_ptr), N, 0, M, 16, K,
+              *_lib.ranks_of_blocks(G), P(dphi), 16, P(dmsg), K, P(dY), 20, _lib.stream_of(phi))
+    rec = torch.repeat_interleave(torch.arange(N, device=DEV), torch.as_tensor(counts, device=DEV))
+    Gd = torch.cat(G, 0).permute(1, 0, 2).reshape(N, 20, 16, K).double()[rec]            # (E, 20, 16, K)
+    md, pd, Yd = msg.double()[col.long()], phi.double(), Y.double()
+    W = torch.einsum("exbk,ek->exb", Gd, md)
+    want = (torch.einsum("exb,ex->eb", W, Yd), torch.einsum("exbk,ex,eb->ek", Gd, Yd, pd),
+            torch.einsum("exb,eb->ex", W, pd))
+    for got, w in zip((dphi, dmsg, dY), want):
+        w32 = w.float()
+        assert torch.equal(torch.isnan(got), torch.isnan(w32))
+        inf = torch.isinf(w32)
+        assert torch.equal(got[inf], w32[inf])
+        ok = torch.isfinite(w32)
+        assert torch.isfinite(got[ok]).all()
+        # sums of at most 320 fp32 products: relative to each row's scale
+        scale = torch.where(ok, w32.abs(), torch.zeros_like(w32)).amax(1, keepdim=True).expand_as(w32)
+        assert ((got - w32).abs()[ok] <= 4e-6 * scale[ok]).all()
