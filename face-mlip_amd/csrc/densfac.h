@@ -5,6 +5,9 @@
 
 namespace face {
 
+int launch_density_fwd_limb(const float* phi, int ld_phi, const float* msg, int ld_msg, const int32_t* msg_row,
+                            const float* Y, int ld_Y, const int32_t* row_ptr, int64_t N, int M, int K, const RankOut& D,
+                            hipStream_t st);
 int launch_density_bwd_limb(const float* phi, int ld_phi, const float* msg, int ld_msg, const int32_t* msg_row,
                             const float* Y, int ld_Y, const int32_t* row_ptr, int64_t N, int M, int max_row, int K,
                             const RankIn& G, float* dphi, int ld_dphi, float* dmsg, int ld_dmsg, float* dY, int ld_dY,

@@ -1461,9 +1461,9 @@ def test_table_linears_match_torch(N, C, n):
     ([1, 0, 31, 32, 33, 5], 16, None), ([64, 65, 0, 2, 40], 32, None), ([96, 97, 130, 1, 64], 48, None),
     ([70, 96, 33, 200, 0], 64, None), ([7, 30], 64, None), ([40, 3, 70], 32, "msg"), ([40, 3, 70], 32, "G"),
     ([40, 3, 70], 32, "Y")])
-def test_factor_density_backward_row_lengths(counts, K, huge):
-    """Row lengths around the 32-edge tiles and the chunks of 32, 64 and 96 edges, gathered messages, against
-    fp64; one value past the largest bf16 (no finite limbs) leaves every other atom's results finite and
+def test_factor_density_row_lengths(counts, K, huge):
+    """Row lengths around the 16- and 32-edge tiles and the chunks of 32, 64 and 96 edges, gathered messages,
+    both directions against fp64; one value past the largest bf16 (no finite limbs) leaves every other atom's results finite and
     its own as plain fp32 gives them."""
     from face_amd import _lib, ops
     N, E, M = len(counts), sum(counts), max(counts)
@@ -1486,16 +1486,23 @@ def test_factor_density_backward_row_lengths(counts, K, huge):
     if huge == "G":
         G[2][1, 2, 5] = float("inf")
     dphi, dmsg, dY = (torch.full((E, w), float("nan"), device=DEV) for w in (16, K, 20))
+    D = [torch.full((k, N, 16 * K), float("nan"), device=DEV) for k in ops.RANK_K]
     P = _lib.ptr
     _lib.call("face_density_bwd", P(phi), 21, P(msg), K, P(col), P(Y), 20, 20, P(row_ptr), N, 0, M, 16, K,
               *_lib.ranks_of_blocks(G), P(dphi), 16, P(dmsg), K, P(dY), 20, _lib.stream_of(phi))
+    _lib.call("face_density_fwd", P(phi), 21, P(msg), K, P(col), P(Y), 20, 20, P(row_ptr), N, 0, 16, K,
+              *_lib.ranks_of_blocks(D), _lib.stream_of(phi))
     rec = torch.repeat_interleave(torch.arange(N, device=DEV), torch.as_tensor(counts, device=DEV))
     Gd = torch.cat(G, 0).permute(1, 0, 2).reshape(N, 20, 16, K).double()[rec]            # (E, 20, 16, K)
     md, pd, Yd = msg.double()[col.long()], phi.double(), Y.double()
     W = torch.einsum("exbk,ek->exb", Gd, md)
     want = (torch.einsum("exb,ex->eb", W, Yd), torch.einsum("exbk,ex,eb->ek", Gd, Yd, pd),
             torch.einsum("exb,eb->ex", W, pd))
-    for got, w in zip((dphi, dmsg, dY), want):
+    Dw = torch.zeros(N, 20, 16, K, dtype=torch.float64, device=DEV)
+    Dw.index_add_(0, rec, torch.einsum("ex,eb,ek->exbk", Yd, pd, md))
+    want += (Dw.reshape(N, -1),)
+    D = torch.cat(D, 0).permute(1, 0, 2).reshape(N, -1)
+    for got, w in zip((dphi, dmsg, dY, D), want):
         w32 = w.float()
         assert torch.equal(torch.isnan(got), torch.isnan(w32))
         inf = torch.isinf(w32)
