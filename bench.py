@@ -44,6 +44,7 @@ import torch  # noqa: E402
 METRIC = "atom-steps/s (E+F, fp32) at 864 & 24k atoms; density-kernel HBM GB/s"
 HBM_PEAK_GBS = 8000.0
 MFMA_PEAK_TFS = 157.3                   # MI355X dense fp32 MFMA
+SPLIT_PEAK_TFS = 2500.0 / 6             # fp32 products as six dense bf16 products of exact three-way splits
 CALLS_PER_ROUND = 5
 TAGS = {0: "mol64_c96", 1: "mol512_cp160", 2: "fcc864_c96", 3: "liquid24k_cp160", 4: "liquid100k_c256"}
 
@@ -62,7 +63,7 @@ KERNEL_FAMILY = {
     "edge_fwd": "edge_geom_fwd", "edge_bwd": "edge_geom_bwd", "force_scatter": "force_scatter",
     "gather_bwd": "gather_rows_bwd", "radial_fwd": "radial_fwd", "radial_bwd": "radial_bwd",
     "radial_head": "edge_linear_fwd", "edge_msg_fwd": "edge_linear_fwd", "edge_msg_bwd": "edge_linear_bwd",
-    "mix_fwd": "rows_gemm", "mix_bwd": "rows_gemm", "tmix_bwd": "rows_gemm", "mix_tmix_bwd": "rows_gemm",
+    "mix_fwd": "rows_gemm", "mix_tmix_fwd": "rows_gemm", "mix_bwd": "rows_gemm", "tmix_bwd": "rows_gemm", "mix_tmix_bwd": "rows_gemm",
     "proj_fwd": "rows_gemm",
     "proj_bwd": "rows_gemm", "readout_in": "rows_gemm", "readout_hid": "rows_gemm", "readout_out": "rows_gemm",
     "readout_in_bwd": "rows_gemm", "readout_hid_bwd": "rows_gemm", "readout_out_bwd": "rows_gemm",
@@ -73,9 +74,8 @@ KERNEL_FAMILY = {
 }
 # kernel family -> kernel functions of libface_hip.so it stands for (rocprofv3 names, namespace face)
 FAMILY_KERNELS = {
-    "density_fwd": ["density_fwd_row_kernel", "density_fwd_kernel"],
-    "density_bwd": ["density_bwd_split_kernel", "density_bwd_mfma_kernel", "density_bwd_lds_kernel",
-                    "density_bwd_kernel"],
+    "density_fwd": ["density_fwd_limb_kernel", "density_fwd_kernel"],
+    "density_bwd": ["density_bwd_limb_kernel", "density_bwd_kernel"],
     "density_mix_fwd": ["density_mix_fwd_kernel"], "density_mix_bwd": ["density_mix_bwd_kernel"],
     "cp_density_fwd": ["cp_density_fwd_wave_kernel", "cp_density_fwd_kernel"],
     "cp_density_bwd": ["cp_density_bwd_mfma_kernel", "cp_density_bwd_kernel"],
@@ -92,13 +92,17 @@ FAMILY_KERNELS = {
     "gather_rows_bwd": ["gather_rows_bwd_kernel"],
     "radial_fwd": ["radial_fwd_kernel"], "radial_bwd": ["radial_bwd_kernel"],
     "edge_linear_fwd": ["edge_linear_fwd_kernel"], "edge_linear_bwd": ["edge_linear_bwd_kernel"],
-    "rows_gemm": ["rows_gemm_kernel", "rows_gemm_kc_kernel"], "eq_gate_fwd": ["eq_gate_fwd_kernel"], "eq_gate_bwd": ["eq_gate_bwd_kernel"],
+    "rows_gemm": ["rows_gemm_kernel", "rows_gemm_direct_kernel", "split_weights_kernel"],
+    "eq_gate_fwd": ["eq_gate_fwd_kernel"], "eq_gate_bwd": ["eq_gate_bwd_kernel"],
     "layer_norm_fwd": ["layer_norm_fwd_kernel"], "layer_norm_bwd": ["layer_norm_bwd_kernel"],
     "spline_order": ["spline_zero_kernel", "spline_count_kernel", "spline_scan_kernel", "spline_place_kernel"],
     "radial_spline_fwd": ["radial_spline_fwd_kernel", "radial_spline_run_fwd_kernel"],
     "radial_spline_bwd": ["radial_spline_bwd_kernel", "radial_spline_run_bwd_kernel"],
 }
 TIMED = list(KERNEL_FAMILY)
+# families whose products run on the split (the per-edge linears too, but their launches are bound by bytes
+# and stay quoted against the fp32 instruction)
+SPLIT_FAMILIES = ("rows_gemm", "cp_radial_fwd", "density_fwd", "density_bwd")
 
 
 def log(*a):
@@ -207,7 +211,7 @@ def algorithmic_bytes(label, g, kw):
         return 4 * (20 * N * C + 48 * N * C + 9 * C * C)
     if label == "tmix_bwd":             # 9 N rows, C -> T
         return 4 * (9 * N * (C + T) + C * T)
-    if label == "mix_tmix_bwd":
+    if label in ("mix_tmix_fwd", "mix_tmix_bwd"):
         return algorithmic_bytes("mix_bwd", g, kw) + algorithmic_bytes("tmix_bwd", g, kw)
     if label in ("table_linear_fwd", "table_linear_bwd"):   # (3 + 6) N rows, C <-> 2 K_dir, two weights
         return 4 * (9 * N * (C + 2 * kw["K_dir"]) + 2 * C * 2 * kw["K_dir"])
@@ -262,7 +266,7 @@ def algorithmic_flops(label, g, kw):
         return 2 * 9 * N * C * kw["B"] * 2 * kw["K_dir"]
     if label in ("table_linear_fwd", "table_linear_bwd"):   # (3 + 6) N rows, C <-> nt K_dir
         return 2 * 9 * N * C * 2 * kw["K_dir"]
-    if label == "mix_tmix_bwd":         # both in one launch
+    if label in ("mix_tmix_fwd", "mix_tmix_bwd"):   # both in one launch
         return algorithmic_flops("mix_bwd", g, kw) + algorithmic_flops("tmix_bwd", g, kw)
     if label == "radial_head":
         return 2 * E * H * 4 * C
@@ -281,11 +285,12 @@ def algorithmic_flops(label, g, kw):
     # equivariant outputs, i.e. all passes but the last with eqmsg)
     gate = (kw.get("n_passes", 2) - 1) / kw.get("n_passes", 2) if kw.get("eqmsg") else 0.0
     if label == "readout_in":
-        return 2 * N * 10 * C * 2 * C + gate * 2 * N * 9 * C * 2 * C
+        # [inv | h]; the first pass's h columns come as a precomputed initial sum
+        return 2 * N * (10 - 1 / kw.get("n_passes", 2)) * C * 2 * C + gate * 2 * N * 9 * C * 2 * C
     if label in ("readout_hid", "readout_hid_bwd"):
         return 2 * N * 2 * C * 2 * C
     if label in ("readout_out", "readout_out_bwd"):
-        return 2 * N * 2 * C * (C + 16)
+        return 2 * N * 2 * C * C
     if label == "readout_in_bwd":
         return 2 * N * 2 * C * 10 * C + gate * 2 * N * 2 * C * 9 * C
     if label == "density_fwd20":
@@ -299,10 +304,15 @@ def algorithmic_flops(label, g, kw):
     return None
 
 
-def floor_us(byts, fl):
-    """(time floor in us, binding bound) of one launch: bytes at peak HBM, flops at the fp32 MFMA peak."""
+def mfma_peak(family):
+    """Peak rate of a kernel family's fp32 products: on split bf16 products or the fp32 instruction."""
+    return SPLIT_PEAK_TFS if family in SPLIT_FAMILIES else MFMA_PEAK_TFS
+
+
+def floor_us(byts, fl, family=None):
+    """(time floor in us, binding bound) of one launch: bytes at peak HBM, flops at the family's MFMA peak."""
     t_hbm = (byts or 0) / (HBM_PEAK_GBS * 1e9) * 1e6
-    t_mfma = (fl or 0) / (MFMA_PEAK_TFS * 1e12) * 1e6
+    t_mfma = (fl or 0) / (mfma_peak(family) * 1e12) * 1e6
     return (t_mfma, "mfma") if t_mfma > t_hbm else (t_hbm, "hbm")
 
 
@@ -341,7 +351,7 @@ def label_stats(timers, steps, g, kw):
         byts = algorithmic_bytes(label, g, kw)
         fl = algorithmic_flops(label, g, kw)
         ib = interface_bytes(label, g, kw)
-        fus, bound = floor_us(byts, fl)
+        fus, bound = floor_us(byts, fl, family_of(label))
         kern[label] = {"family": family_of(label), "launches_per_step": len(evs) / steps, "avg_us": avg_us,
                        "ms_per_step": float(np.sum(ms)) / steps, "alg_bytes": byts, "alg_flops": fl,
                        "GBps": (byts / (avg_us * 1e-6) / 1e9) if byts else None,
@@ -368,7 +378,7 @@ def family_stats(kern):
         f["bytes_per_step"] += n * (v["alg_bytes"] or 0)
         f["flops_per_step"] += n * (v["alg_flops"] or 0)
         if v["alg_bytes"] or v["alg_flops"]:
-            fus, bound = floor_us(v["alg_bytes"], v["alg_flops"])
+            fus, bound = floor_us(v["alg_bytes"], v["alg_flops"], v["family"])
             f["floor_ms_per_step"] += n * fus * 1e-3
             f["floor_" + bound] += n * fus * 1e-3
             f["known"] = True
@@ -392,7 +402,7 @@ def roofline_of(fam, tag):
     dom = max(known, key=lambda k: known[k]["ms_per_step"])
     v = known[dom]
     if v["bound"] == "mfma":
-        peak, unit = MFMA_PEAK_TFS, "TFLOP/s"
+        peak, unit = mfma_peak(dom), "TFLOP/s"
     else:
         peak, unit = HBM_PEAK_GBS, "GB/s"
     return {"kernel": dom, "kernels": v["kernels"], "labels": v["labels"], "bound": v["bound"],
@@ -988,7 +998,7 @@ def hot_path_kernels(r):
     """HBM fraction of the density kernels and of the force scatter (the kernels the target is
     quoted on): per family present, the fraction of 8 TB/s its algorithmic bytes reach, and for a
     family whose binding floor is its matrix work (the fused CP kernels, the factor density at
-    100k atoms) also its fraction of the fp32 MFMA peak. The force backward is also given as one
+    100k atoms) also its fraction of its products' MFMA peak. The force backward is also given as one
     unit, the edge backward (which writes every edge's dL/dvec into its reverse edge's slot) and
     the row scatter that completes it: their bytes over their time."""
     out = {}
@@ -1000,7 +1010,7 @@ def hot_path_kernels(r):
         out[fam_name] = {"us": _r(f["avg_us"]), "GBps": _r(gbs), "hbm_frac": _r(gbs / HBM_PEAK_GBS, 3)}
         if f.get("bound") == "mfma" and f.get("alg_flops_per_launch"):
             tfs = f["alg_flops_per_launch"] / (f["avg_us"] * 1e-6) / 1e12
-            out[fam_name]["mfma_frac"] = _r(tfs / MFMA_PEAK_TFS, 3)
+            out[fam_name]["mfma_frac"] = _r(tfs / mfma_peak(fam_name), 3)
     fe, fs = r["families"].get("edge_geom_bwd"), r["families"].get("force_scatter")
     if fe and fs and fe.get("alg_bytes_per_launch") and fs.get("alg_bytes_per_launch"):
         byts = fe["bytes_per_step"] + fs["bytes_per_step"]

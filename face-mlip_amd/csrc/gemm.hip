@@ -142,12 +142,11 @@ extern "C" int face_rows_linear_ws(const face_lin_problem* probs, int32_t n_prob
                                 int64_t period, void* work, int64_t work_bytes, void* stream) {
     if (!probs || n_probs < 1 || n_probs > kGemmMaxProbs) return FACE_ERR_ARG;
     int K = 16, n_widest = 16;
-    bool any_bias = false, any_ext = false, any_op = false;
+    bool any_ext = false, any_op = false;
     for (int i = 0; i < n_probs; ++i) {
         if (probs[i].k < 16 || probs[i].k % 16) return FACE_ERR_ARG;
         if (probs[i].k > K) K = probs[i].k;
         if (probs[i].n > n_widest) n_widest = probs[i].n;
-        if (probs[i].bias) any_bias = true;
         if (probs[i].x_op || probs[i].sum_row) any_op = true;
         if (probs[i].x_op || probs[i].sum_row || probs[i].x2 || probs[i].y0) any_ext = true;
     }
@@ -159,7 +158,7 @@ extern "C" int face_rows_linear_ws(const face_lin_problem* probs, int32_t n_prob
         return FACE_ERR_UNSUPPORTED;
     RowsCtx c{};
     GemmArgs& A = c.A;
-    A.n_probs = n_probs, A.w_kn = w_kn ? 1 : 0, A.any_bias = any_bias ? 1 : 0, A.xs = x_scale, A.ys = y_scale;
+    A.n_probs = n_probs, A.w_kn = w_kn ? 1 : 0, A.xs = x_scale, A.ys = y_scale;
     A.ld_s = ld_scale, A.n_groups = n_groups, A.group = scaled ? group : nullptr, A.period = period, A.kmax = K;
     for (int i = 0; i < n_probs; ++i) {
         const int st = fill_prob(probs[i], A.w_kn, scaled, x_scale, y_scale, ld_scale, A.p[i]);

@@ -1,4 +1,4 @@
-// Per-edge linear layers on the fp32 matrix cores (gfx950), for layers whose input is a
+// Per-edge linear layers on the matrix cores (gfx950; forward as split bf16 products), for layers whose input is a
 // per-edge feature row of K <= 64 values and whose output is a per-edge row of F values:
 //
 //   forward   Y[e] = X[e] W^T + b + T[idx[e]]                            (E, F)
@@ -20,7 +20,8 @@ namespace face {
 // D = W . X^T in 32 x 32 blocks as split bf16 products (edges.h): the weight blocks of the workgroup's
 // features sit in LDS as limbs, each wave splits the X rows of 32 edges once and walks the blocks, lane
 // e holding features 8 g + 4 (lane >> 5) + 0..3 of edge e, one float4 store each. Bound by the write of
-// Y; six blocks of 64 inputs (72 KB) leave room for two workgroups per CU.
+// Y; six blocks of 64 inputs (72 KB) leave room for two workgroups per CU (1.25 M edges, 64 -> 160 with
+// gathered table rows: 400 us as on fp32 instructions; the form is the one cp_radial_fwd shares).
 constexpr int kLinWaves = 4, kLinBlocks = 6;
 
 template <int KB, bool HAS_T>

@@ -82,7 +82,6 @@ struct GemmArgs {
     GemmProb p[kGemmMaxProbs];
     int n_probs, w_kn;
     const float *xs, *ys;
-    int any_bias;                          // some problem has a bias (side table present)
     int ld_s, n_groups;
     const int32_t* group;
     int64_t period;

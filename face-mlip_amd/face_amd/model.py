@@ -37,11 +37,8 @@ from .neighbors import graph_from_padded
 from .ops import Graph
 
 RANKS = [(0, 1), (1, 4), (4, 10), (10, 20)]   # monomial range of each rank (face/cartesian.py:18)
-# The readout chain on the row GEMM (ops.readout: 4 launches forward, 5 backward) instead of
-# LayerNorm + library GEMMs + elementwise SiLU / residual: measured slower at the benchmark widths
-# (24,000-atom C160 step 19.1 -> 21.4 ms, 864-atom C96 0.84 -> 0.96 ms: the whole-K weight
-# slices leave the N x 10C -> 2C input layer and its gradient under-occupied, and the small
-# 2C-wide layers pay a weight-slice staging per workgroup), so it is opt-in.
+# The readout with its LayerNorm as a launch of its own (ops.readout) instead of inside the node-algebra
+# kernels followed by ops.readout_mlp: it writes and reads the invariant row twice more, so it is opt-in.
 READOUT_ROW_GEMM = os.environ.get("FACE_READOUT_ROW_GEMM", "0") == "1"
 
 
@@ -422,8 +419,7 @@ class FactorBlock(nn.Module):
         else:
             feats, V, Ms = ops.node_features(ys[0], ys[1], ys[2], ys[3], *ab, self.eq_out, C, feats_buf)
         if not fused_ln and READOUT_ROW_GEMM and C % 16 == 0 and nf <= 2048:
-            # LayerNorm, the out MLP and the residual split on the row GEMM (four launches forward;
-            # opt-in: slower than the library GEMMs at the benchmark widths)
+            # LayerNorm, the out MLP and the residual split (four launches forward; opt-in)
             rw = self._readout_weights()
             e, h_new, gvm = ops.readout(feats, h, self.norm.weight.detach(), self.norm.bias.detach(), self.norm.eps,
                                         *rw)

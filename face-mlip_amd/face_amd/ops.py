@@ -412,8 +412,8 @@ class ReadoutMLP(torch.autograd.Function):
 
     Widths that are multiples of 16 run on the row-block kernels, SiLU and its derivative applied to
     the rows as they load: z0 and the gate row in one launch, then z1, the residual rows, the energy
-    row; backward in three launches (10,752 atoms, C = 160, forward and backward: 660 us on the
-    library's float32 products with the activations between them, 340 us here). Other widths, and
+    row; backward in three launches (10,752 atoms, C = 160, forward and backward: 667 us on the
+    library's float32 products with the activations between them, 405 us here). Other widths, and
     weights without 16-byte aligned rows, take the library products."""
 
     @staticmethod
@@ -870,12 +870,10 @@ def cp_density(R, env, msg, Y, graph, gathered=False):
 
 class CPRadialDensity(torch.autograd.Function):
     """CP pooling fed by the CP columns of the last radial layer: R = h2 W_cp^T + b_cp (E, 4C), then
-    A_l as in CPDensity (face/model.py:469-472, 496-502). With per-edge messages the forward computes
-    R on the matrix cores and pools it in the same launch (R is written once, for the backward, and
-    not read back: 1.85 ms against 2.03 ms for the two launches at 24,000 atoms, C = 160; 0.345
-    against 0.385 ms at 512 molecules); with node-table messages gathered through col, and for
-    shapes that launch cannot serve, R comes from the radial head and is pooled in a second launch
-    (1.89 ms against 2.03 ms fused there). The
+    A_l as in CPDensity (face/model.py:469-472, 496-502). The forward computes R on the matrix cores and
+    pools it in the same launch (R is written once, for the backward, and not read back: 1.36 / 1.26 ms
+    with per-edge / node-table messages at 24,000 atoms, C = 160); for shapes that launch cannot serve, R
+    comes from the radial head and is pooled in a second launch (1.96 ms there). The
     backward multiplies the pooling's dR by W_cp on the matrix cores inside the pooling kernel and
     returns d h2 (E, H) without writing dR. W_cp / b_cp receive no gradient (forces only)."""
 
@@ -1455,9 +1453,8 @@ class ScaledMix(torch.autograd.Function):
         C = wm[0].shape[0]
         dev = Af[0].device
         outs = [torch.empty(a.shape[0], N, C, device=dev) for a in Af]
-        # the transport sums are further input columns of ranks 1 and 2, with their own weights (24,000
-        # atoms, C = 160, 512 transport columns: 190 + 345 us for the library's products written first and
-        # accumulated onto, 390 us in the one launch)
+        # the transport sums are further input columns of ranks 1 and 2, with their own weights: their
+        # products are neither written first nor read back
         Ds = {1: D1, 2: D2}
         probs = []
         for l, a in enumerate(Af):
@@ -1468,7 +1465,8 @@ class ScaledMix(torch.autograd.Function):
                 probs.append(lin(x, wm[l], y, l * C, 1.0))
             else:
                 probs.append(lin(x, wm[l], y, l * C, x2=D, w2=None if D is None else wt[l - 1]))
-        rows_linear(probs, ys=s_tab, group=group, period=N, label="mix_fwd")
+        rows_linear(probs, ys=s_tab, group=group, period=N,
+                    label="mix_fwd" if D1 is None and D2 is None else "mix_tmix_fwd")
         ctx.save_for_backward(s_tab, group)
         ctx.wm, ctx.wt, ctx.has_D = wm, wt, (D1 is not None, D2 is not None)
         ctx.shapes = [a.shape for a in Af]

@@ -37,8 +37,8 @@ def _hip_runtime():
 
 
 def tune_library_gemms(results_file=None):
-    """Let PyTorch TunableOp pick the solutions of the GEMMs left to the libraries (readout MLP,
-    tmix forward, per-node linears): the first call of each shape times the fp32 hipBLASLt /
+    """Let PyTorch TunableOp pick the solutions of the GEMMs left to the libraries (per-node linears,
+    and the readout and transport mix of widths that are no multiples of 16): the first call of each shape times the fp32 hipBLASLt /
     rocBLAS solutions and keeps the fastest whose result matches the default one within 1e-5.
     Call before the first step (tuning runs eagerly, so before any graph capture). Process-wide;
     results go to results_file (default: a fresh temporary directory)."""
