@@ -164,3 +164,6 @@ def test_positions_of_any_strides(method):
     st = dict(pos=pos, Z=np.ones(150, int), cell=np.eye(3) * 9.0, pbc=True)
     check_graph([dict(st, pbc=np.ones(3, bool))], 4.0, method)
     check_graph([dict(st, pbc=np.ones(3, bool), pos=np.repeat(pos, 2, 0)[::2])], 4.0, method)
+    if method == "small":                                # several of them: their concatenation is column-major too
+        check_graph([dict(pos=rng.uniform(0, 6, (3, n)).T, Z=np.ones(n, int), cell=np.zeros((3, 3)),
+                          pbc=np.zeros(3, bool)) for n in (20, 1, 31)], 4.0, method)
