@@ -32,7 +32,7 @@ __global__ __launch_bounds__(kCrfWaves * kWave) __attribute__((amdgpu_waves_per_
     const float* __restrict__ Y, int ld_Y, const int32_t* __restrict__ row_ptr, int64_t N, int C, int nparts,
     RankOut A, float* __restrict__ R, int ld_R) {
     constexpr int H = 16 * HB;
-    extern __shared__ v8bf lds[];                     // 4 limb images (one per rank), then the waves' Y tiles
+    extern __shared__ v8bf lds[];                     // 4 limb images (one per rank), the biases, the waves' Y tiles
     const int tid = threadIdx.x, lane = tid & (kWave - 1), half = lane >> 5;
     const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
     // blocks b and b + 8 run on the same XCD: all parts of an edge share read its rows through one L2
@@ -52,8 +52,11 @@ __global__ __launch_bounds__(kCrfWaves * kWave) __attribute__((amdgpu_waves_per_
             const int ch = 32 * part + f;
             return ch < C ? w + (int64_t)(l * C + ch) * H : nullptr;
         });
+    float* const sb = reinterpret_cast<float*>(lds + 4 * kLimbImage<HB>);      // the part's 4 x 32 biases
+    for (int v = tid; v < 128; v += kCrfWaves * kWave)
+        sb[v] = b ? b[(v >> 5) * C + min(32 * part + (v & 31), C - 1)] : 0.f;
     big = __syncthreads_or(big);
-    float* const yt = reinterpret_cast<float*>(lds + 4 * kLimbImage<HB>) + wv * 32 * kCrfRow;
+    float* const yt = sb + 128 + wv * 32 * kCrfRow;
     const int64_t W = ngrp * kCrfWaves, gw = grp * kCrfWaves + wv;
     int64_t at = uniform64(wave_lower_bound(row_ptr, N, E * gw / W, lane));
     const int64_t a_end = gw + 1 == W ? N : uniform64(wave_lower_bound(row_ptr, N, E * (gw + 1) / W, lane));
@@ -87,11 +90,9 @@ __global__ __launch_bounds__(kCrfWaves * kWave) __attribute__((amdgpu_waves_per_
     }
     if (e_beg >= e_end) return;
     const uint32_t r_off = (uint32_t)(4 * half * ld_R + c) * 4u;
-    float sum[20], bias[4];
+    float sum[20];
 #pragma unroll
     for (int x = 0; x < 20; ++x) sum[x] = 0.f;
-#pragma unroll
-    for (int l = 0; l < 4; ++l) bias[l] = b ? b[l * C + cc] : 0.f;
     // a tile's h2 rows (A operand: lane = edge, 8 inputs per 16) and Y rows (lane = edge, 10 monomials
     // per half), loaded while the tile before it computes; edges past the share repeat its last one
     v4f hn[2 * HB];
@@ -113,8 +114,16 @@ __global__ __launch_bounds__(kCrfWaves * kWave) __attribute__((amdgpu_waves_per_
         xn = (half ? x_hi : x_lo)[e];
     };
     load_tile(e_beg);
-    for (int64_t t0 = e_beg; t0 < e_end; t0 += 32) {
-        const int n = (int)min((int64_t)32, e_end - t0);
+    // A tile whose Y rows hold a NaN or an infinity is walked once per atom segment, the rows of the other
+    // atoms' edges zero: zero times such a value is NaN, and only the products of other atoms' edges are
+    // zeroed below. first() is the first row of the current atom in the tile.
+    auto first = [&](int64_t t0) __attribute__((always_inline)) { return (int)max(rp(at) - t0, (int64_t)0); };
+    for (int64_t t0 = e_beg; t0 < e_end;) {
+        float yc = 0.f;
+#pragma unroll
+        for (int k = 0; k < 10; ++k) yc = fmaf(yn[k], 0.f, yc);
+        int n = (int)min((int64_t)32, e_end - t0);
+        if (__any(yc != yc)) n = (int)min(rp(at + 1) - t0, (int64_t)n);
         Split8 x[HB];
         float mx = 0.f;
 #pragma unroll
@@ -125,8 +134,9 @@ __global__ __launch_bounds__(kCrfWaves * kWave) __attribute__((amdgpu_waves_per_
         const bool plain = big || __any(mx > kLimbMax);
         {
             float* d = yt + (lane & 31) * kCrfRow + 12 * half;
+            const int w0 = first(t0);
 #pragma unroll
-            for (int k = 0; k < 10; ++k) d[k] = yn[k];
+            for (int k = 0; k < 10; ++k) d[k] = (lane & 31) >= w0 && (lane & 31) < n ? yn[k] : 0.f;
             yt[(lane & 31) * kCrfRow + 10 + half] = half || env ? xn : 1.f;
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -143,7 +153,8 @@ __global__ __launch_bounds__(kCrfWaves * kWave) __attribute__((amdgpu_waves_per_
 #pragma unroll
             for (int r = 0; r < 16; ++r) me[r] = mt[(int64_t)min(d_row(r) + 4 * half, n - 1) * ld_msg + cc];
         }
-        if (t0 + 32 < e_end) load_tile(t0 + 32);
+        const int64_t t1 = n == 32 || t0 + n == e_end ? t0 + 32 : t0;
+        if (t1 < e_end) load_tile(t1);
         int64_t nxt = at;
         // ranks L0 .. L0 + NL - 1 (monomials X0 .. X1 - 1): R, its rows out, the pooling
         auto ranks = [&](auto L0_, auto NL_) __attribute__((always_inline)) {
@@ -179,8 +190,9 @@ __global__ __launch_bounds__(kCrfWaves * kWave) __attribute__((amdgpu_waves_per_
             }
 #pragma unroll
             for (int l = 0; l < NL; ++l) {
+                const float bias = sb[32 * (L0 + l) + (lane & 31)];
 #pragma unroll
-                for (int r = 0; r < 16; ++r) acc[l][r] += bias[L0 + l];
+                for (int r = 0; r < 16; ++r) acc[l][r] += bias;
                 if (R && in_c) {
                     int64_t ld = ld_R;                // wave-uniform row addresses, formed here
                     asm volatile("" : "+s"(ld));
@@ -203,7 +215,7 @@ __global__ __launch_bounds__(kCrfWaves * kWave) __attribute__((amdgpu_waves_per_
             }
             // the tile's atom segments [lo, hi)
             int64_t a = at;
-            int lo = 0;
+            int lo = first(t0);
             while (true) {
                 const int64_t a_hi = rp(a + 1) - t0;
                 const int hi = (int)min(a_hi, (int64_t)n);
@@ -254,6 +266,7 @@ __global__ __launch_bounds__(kCrfWaves * kWave) __attribute__((amdgpu_waves_per_
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();              // the Y tile is overwritten next
         at = nxt;
+        t0 = n == 32 || t0 + n == e_end ? t0 + 32 : t0;
     }
 }
 
@@ -277,7 +290,7 @@ extern "C" int face_cp_radial_fwd(const float* h2, int32_t ld_h2, int32_t H, con
         (int64_t)ld_R * 16 >= ((int64_t)1 << 31))
         return FACE_ERR_UNSUPPORTED;
     const int nparts = (C + 31) / 32;
-    const size_t lds = (size_t)(4 * (H / 16) * 3 * kWave) * 16 + (size_t)kCrfWaves * 32 * kCrfRow * sizeof(float);
+    const size_t lds = (size_t)(4 * (H / 16) * 3 * kWave) * 16 + (size_t)(128 + kCrfWaves * 32 * kCrfRow) * sizeof(float);
     if ((int64_t)lds > device_max_lds()) return FACE_ERR_UNSUPPORTED;
     // two workgroups per CU (LDS); edge shares of at least 2 tiles per wave; a multiple of 8 groups, so
     // that blocks b and b + 8 (one XCD) hold the parts of one group

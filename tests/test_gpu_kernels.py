@@ -289,6 +289,52 @@ def test_cp_radial_fused_forward_without_edges():
     assert all((o == 0).all() for o in outs)
 
 
+@pytest.mark.parametrize("what", ["Y", "Yinf", "env", "msg", "h2"])
+@pytest.mark.parametrize("C,H,gathered", [(160, 64, True), (160, 64, False), (48, 16, True)])
+def test_cp_radial_fused_forward_contains_non_finite_edges(C, H, gathered, what):
+    """A NaN or an infinity on some edges (coincident atoms have NaN directions) stays with the receivers of
+    those edges: every other atom keeps its bits, though tiles of 32 edges span atoms, and a NaN in the
+    directions leaves the receiver's monomial of rank 0 alone."""
+    from face_amd import _lib, ops
+    say("cp radial fwd non-finite", C, H, gathered, what)
+    N = 300
+    counts = _ragged_counts(N, C + H)
+    E = int(sum(counts))
+    rec = np.repeat(np.arange(N), counts)
+    row_ptr = torch.as_tensor(np.concatenate([[0], np.cumsum(counts)]).astype(np.int32), device=DEV)
+    rng = np.random.default_rng(C)
+    col = torch.as_tensor(rng.integers(1, N, E).astype(np.int32), device=DEV)
+    torch.manual_seed(C + H)
+    t = {"h2": torch.randn(E, H, device=DEV), "env": torch.rand(E, device=DEV), "Y": torch.randn(E, 20, device=DEV),
+         "msg": torch.randn(N if gathered else E, C, device=DEV)}
+    W, b = torch.randn(4 * C, H, device=DEV) / H ** 0.5, torch.randn(4 * C, device=DEV)
+    bad = np.concatenate([[0, 7, 31, 32, E - 1], rng.integers(0, E, 12)])     # edges of tiles and of the list
+    if what == "msg" and gathered:
+        col[torch.as_tensor(bad, device=DEV)] = 0                             # the one bad table row
+
+    def run():
+        outs = [torch.full((k, N, C), 7.0, device=DEV) for k in ops.RANK_K]
+        P = _lib.ptr
+        _lib.call("face_cp_radial_fwd", P(t["h2"]), H, H, P(W), P(b), P(t["env"]), P(t["msg"]), C,
+                  P(col) if gathered else None, P(t["Y"]), 20, P(row_ptr), N, E, C, *_lib.ranks_of_blocks(outs), None,
+                  4 * C, _lib.stream_of(W))
+        return torch.cat(outs, 0)                                             # (20, N, C)
+
+    clean = run()
+    assert torch.isfinite(clean).all()
+    at = torch.as_tensor([0] if what == "msg" and gathered else bad, device=DEV)
+    if what[0] == "Y":
+        t["Y"][at, 1:] = float("nan") if what == "Y" else float("inf")
+    else:
+        t[what][at] = float("nan")
+    out = run()
+    hit = torch.zeros(N, dtype=torch.bool, device=DEV)
+    hit[torch.as_tensor(rec[bad], device=DEV)] = True
+    assert torch.equal(out[:, ~hit], clean[:, ~hit])
+    assert not torch.isfinite(out[1:, hit]).any()
+    assert torch.equal(out[0, hit], clean[0, hit]) if what[0] == "Y" else torch.isnan(out[0, hit]).all()
+
+
 # ----------------------------------------------------------------------------- gated outputs
 @pytest.mark.parametrize("N,C", [(1000, 160), (37, 96), (1, 4)])
 def test_eq_gate_matches_torch(N, C):
