@@ -106,8 +106,11 @@ static RowsShape rows_shape(const RowsCtx& c) {
     return {NW, NB, c.n_widest > 32 * NB, 0};
 }
 
-// Workspace: the limbs of every problem, 3 KB per 16 k x 32 columns, for an even number of 16-k steps.
-static int64_t work_blocks(const face_lin_problem& s) { return (int64_t)((s.k + 31) / 32 * 2) * ((s.n + 31) / 32); }
+// Workspace: the limbs of every problem, 3 KB per 16 k x 32 columns, for an even number of 16-k steps. A
+// problem of no rows has none (its pointers may be NULL).
+static int64_t work_blocks(const face_lin_problem& s) {
+    return s.m > 0 ? (int64_t)((s.k + 31) / 32 * 2) * ((s.n + 31) / 32) : 0;
+}
 static int64_t work_layout(const face_lin_problem* probs, int n_probs, GemmProb* p) {
     int64_t bytes = 0;
     for (int i = 0; i < n_probs; ++i) {
@@ -177,6 +180,7 @@ extern "C" int face_rows_linear_ws(const face_lin_problem* probs, int32_t n_prob
             blocks += work_blocks(probs[i]);
         }
         c.work = (char*)work;
+        if (blocks == 0) return 0;                               // no rows at all
         hipLaunchKernelGGL(split_weights_kernel, dim3((unsigned)blocks), dim3(kWave), 0, c.st, A, c.work);
         FACE_LAUNCH_CHECK();
     }

@@ -1142,6 +1142,27 @@ def test_rows_linear_edges_and_weights_split_ahead(m, n, k, w_kn, monkeypatch):
     assert torch.equal(outs[2], outs[3]) and torch.equal(outs[2], outs[4])
 
 
+@pytest.mark.parametrize("m", [0, 40])
+def test_rows_linear_split_ahead_beside_a_problem_of_no_rows(m):
+    """Weights split ahead where one problem has no rows and NULL operands, which are then never read
+    (and no rows at all: nothing is launched)."""
+    from face_amd import _lib
+    say("rows_linear split ahead, no rows", m)
+    torch.manual_seed(5)
+    k, n = 48, 64
+    x, w, y = torch.randn(40, k, device=DEV), torch.randn(n, k, device=DEV), torch.full((40, n), 7.0, device=DEV)
+    P = lambda rows, *p: _lib.LinProblem(p[0], k, rows, p[1], k, p[2], n, n, k, 0, 0.0, None, 0, k, 0, None, 0, None,
+                                         None, 0, 0, 0, None, 0, None, None)
+    arr = (_lib.LinProblem * 3)(P(0, None, None, None), P(m, x.data_ptr(), w.data_ptr(), y.data_ptr()),
+                                P(0, None, None, None))
+    need = 3 * 4 * 2 * 3072
+    work = torch.empty(need, dtype=torch.uint8, device=DEV)
+    _lib.call("face_rows_linear_ws", arr, 3, 0, None, None, 0, 0, None, 0, _lib.ptr(work), need, _lib.stream_of(y))
+    torch.cuda.synchronize()
+    ref = x.double() @ w.double().t().contiguous()
+    assert rel(y, ref) < 1e-5 if m else bool((y == 7.0).all())
+
+
 @pytest.mark.parametrize("ahead", [False, True])
 @pytest.mark.parametrize("where", ["x", "w"])
 def test_rows_linear_values_past_bf16(where, ahead):
