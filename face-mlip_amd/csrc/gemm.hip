@@ -73,7 +73,10 @@ static int launch_rows(const RowsCtx& c, RowsShape S) {
 // 8.9 against 16.4 us staged, 192 -> 192 5.2 against 7.5; 1,344 rows of 864 -> 192 (252 workgroups) 11.5
 // against 22, but 3,000 rows (564) 27 against 22. Two column blocks per wave where that brings a launch
 // of long K under the limit (4,000 rows of 512 -> 96: 13.3 against 16.6).
+// Row strides past kGemmMaxLd (at most 63 rows of them: an operand has fewer than 2^31 elements) take the
+// direct kernel at any number of problems; its addresses are 64 bits wide.
 static RowsShape rows_shape(const RowsCtx& c) {
+    if (c.far) return {4, 1, 0, 4};
     int NW = 4, NB = 2;
     for (int nb = 1; nb <= (c.K >= 384 ? 2 : 1) && !c.work; ++nb) {
         int64_t w = 0;
@@ -171,9 +174,12 @@ extern "C" int face_rows_linear_ws(const face_lin_problem* probs, int32_t n_prob
     c.probs = probs, c.n_probs = n_probs, c.K = K, c.n_widest = n_widest, c.max_lds = device_max_lds();
     c.n_cu = device_cu_count(), c.x_scale = x_scale != nullptr, c.y_scale = y_scale != nullptr, c.any_ext = any_ext;
     c.any_op = any_op;
+    for (int i = 0; i < n_probs; ++i)
+        for (const int64_t ld : {A.p[i].ld_x, A.p[i].ld_x2, A.p[i].ld_xz, A.p[i].ld_y, A.p[i].ld_y0})
+            c.far = c.far || ld > kGemmMaxLd;
     c.n_groups = n_groups, c.st = (hipStream_t)stream;
-    if (work) {
-        if (((uintptr_t)work & 255) || work_layout(probs, n_probs, A.p) > work_bytes) return FACE_ERR_ARG;
+    if (work && (((uintptr_t)work & 255) || work_layout(probs, n_probs, A.p) > work_bytes)) return FACE_ERR_ARG;
+    if (work && !c.far) {
         int64_t blocks = 0;
         for (int i = 0; i < n_probs; ++i) {
             A.p[i].first_block = blocks;

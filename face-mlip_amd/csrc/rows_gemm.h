@@ -32,6 +32,7 @@ constexpr int kGemmRows = 32;                   // rows per wave
 constexpr int kGemmK = 32;                      // k per staged chunk
 constexpr int kGemmMaxProbs = 8;                // problems per launch
 constexpr int kGemmMaxGroups = 64;              // scale-table rows (elements)
+constexpr int64_t kGemmMaxLd = (int64_t)1 << 25; // row stride of the staged kernel: 31 rows within 32 bits of bytes
 
 struct GemmProb {
     const float* x;
@@ -663,6 +664,7 @@ struct RowsCtx {
     const face_lin_problem* probs;
     int n_probs, K, n_widest, max_lds, n_cu, n_groups;
     bool x_scale, y_scale, any_ext, any_op;
+    bool far;                                    // a row stride past kGemmMaxLd
     char* work;                                  // workspace for split weights, or null
     hipStream_t st;
 };
@@ -670,7 +672,7 @@ struct RowsCtx {
 // One launch of a shape; FACE_ERR_UNSUPPORTED, before anything is launched, if there is no such kernel.
 template <int XM>
 static int launch_rows_xm(const RowsCtx& c, RowsShape S) {
-    if (S.NB < 1 || S.NB > 16 || (S.KW && c.work)) return FACE_ERR_UNSUPPORTED;
+    if (S.NB < 1 || S.NB > 16 || (S.KW && c.work) || (!S.KW && c.far)) return FACE_ERR_UNSUPPORTED;
     GemmArgs A = c.A;
     A.xcd_order = S.xcd;
     A.work = c.work;

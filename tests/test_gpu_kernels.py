@@ -1142,6 +1142,37 @@ def test_rows_linear_edges_and_weights_split_ahead(m, n, k, w_kn, monkeypatch):
     assert torch.equal(outs[2], outs[3]) and torch.equal(outs[2], outs[4])
 
 
+@pytest.mark.parametrize("w_kn", [False, True])
+def test_rows_linear_rows_far_apart(w_kn):
+    """Seven rows 2^28 elements apart (just below the 2^31 elements an operand may span), where 32 bits do
+    not hold a row's byte offset: every operand that has a row stride, plain and with transforms, with and
+    without a workspace for the split weights."""
+    from face_amd import ops
+    say("rows_linear far rows", w_kn)
+    torch.manual_seed(6)
+    m, ld, k1, k2, n = 7, 1 << 28, 48, 16, 80
+    buf = torch.empty(6 * ld + 4096, device=DEV)
+    far = lambda at, w: buf.as_strided((m, w), (ld, 1), at)
+    x, x2, xz, y0, y = far(0, k1), far(512, k2), far(1024, k1), far(1536, n), far(2048, n)
+    for t in (x, x2, xz, y0):
+        t.copy_(torch.randn(t.shape, device=DEV))
+    w = torch.randn(k1 + k2, n, device=DEV) if w_kn else torch.randn(n, k1 + k2, device=DEV)
+    d = lambda t: t.double().cpu()
+    wd = d(w) if w_kn else d(w).T
+    w1 = w[:k1] if w_kn else w[:, :k1]
+    for ahead in (False, True):
+        y.fill_(7.0)
+        _rows_launch(x, w1, y, w_kn, ahead)
+        assert rel(y, d(x) @ wd[:k1]) < 1e-5
+    for op in (0, 2):
+        y.fill_(7.0)
+        ops.rows_linear([ops.lin(x, w, y, x2=x2, x_op=op, xz=xz if op else None, y0=y0, beta=0.5)], w_kn=w_kn)
+        z, xi = d(xz), d(x)
+        s = torch.sigmoid(z)
+        xi = xi * s * (1 + z * (1 - s)) if op else xi
+        assert rel(y, 0.5 * d(y0) + torch.cat([xi, d(x2)], 1) @ wd) < 1e-5
+
+
 @pytest.mark.parametrize("m", [0, 40])
 def test_rows_linear_split_ahead_beside_a_problem_of_no_rows(m):
     """Weights split ahead where one problem has no rows and NULL operands, which are then never read
