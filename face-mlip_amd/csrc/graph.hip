@@ -299,9 +299,11 @@ __global__ __launch_bounds__(kNbrWaves * kWave) void nbr_cell_kernel(
                         double shv[3];
                         ok = !(i == j && s0 == 0 && s1 == 0 && s2 == 0) &&
                              pair_within(pos, i, j, cell, s0, s1, s2, rc, shv);
-                        k = pair_key(j, s0, s1, s2);
-                        if (ok && key && (s0 < -512 || s0 > 511 || s1 < -512 || s1 > 511 || s2 < -512 || s2 > 511))
-                            atomicAdd(overflow, 1);
+                        if (ok && key) {               // past the key's range the atom's index stays whole
+                            const int c0 = min(max(s0, -512), 511), c1 = min(max(s1, -512), 511), c2 = min(max(s2, -512), 511);
+                            k = pair_key(j, c0, c1, c2);
+                            if (s0 != c0 || s1 != c1 || s2 != c2) atomicAdd(overflow, 1);
+                        }
                     }
                     const uint64_t acc = __ballot(ok);
                     if (key && ok) {
@@ -315,7 +317,8 @@ __global__ __launch_bounds__(kNbrWaves * kWave) void nbr_cell_kernel(
             }
         }
     if (counts && lane == 0) counts[i] = n;
-    if (!key || n > cap) return;
+    if (!key) return;
+    n = min(n, cap);                                 // a row that overflowed (counted above) keeps its first cap pairs
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");       // the other lanes' keys
     auto place = [&](auto at) {
         for (int p = lane; p < n; p += kWave) {
@@ -356,7 +359,8 @@ __global__ __launch_bounds__(kNbrWaves * kWave) void nbr_rev_kernel(const int32_
     for (int64_t e = row_ptr[i] + (threadIdx.x & (kWave - 1)); e < row_ptr[i + 1]; e += kWave) {
         const int64_t j = col[e];
         const int t0 = -S[e * 3], t1 = -S[e * 3 + 1], t2 = -S[e * 3 + 2];
-        int64_t lo = row_ptr[j], hi = row_ptr[j + 1];   // rows are sorted by (col, S)
+        const bool in = j >= 0 && j < N;                 // no atom in a row that was not filled: missing below
+        int64_t lo = in ? row_ptr[j] : 0, hi = in ? row_ptr[j + 1] : 0;   // rows are sorted by (col, S)
         int64_t found = -1;
         while (lo < hi) {
             const int64_t mid = (lo + hi) >> 1;

@@ -167,3 +167,60 @@ def test_positions_of_any_strides(method):
     if method == "small":                                # several of them: their concatenation is column-major too
         check_graph([dict(pos=rng.uniform(0, 6, (3, n)).T, Z=np.ones(n, int), cell=np.zeros((3, 3)),
                           pbc=np.zeros(3, bool)) for n in (20, 1, 31)], 4.0, method)
+
+
+def test_overflowing_rows_hold_valid_pairs():
+    """A row whose space is too small, and images past the sort key's range, count as overflows; every row
+    of the cell list then still holds pairs of existing atoms (a short row its first ones), and the reverse
+    map answers for a list with indexes that are no atoms, without following them."""
+    from face_amd import _lib, neighbors
+    say("overflowing rows")
+    rng = np.random.default_rng(2)
+    N, L, rc = 400, 16.0, 4.5
+    st = {"pos": rng.uniform(0, L, (N, 3)), "Z": np.ones(N, int), "cell": np.eye(3) * L, "pbc": np.ones(3, bool)}
+    g = neighbors.build_graph([st], rc, method="cell")
+    counts = (g.row_ptr[1:] - g.row_ptr[:-1]).cpu().numpy()
+    i32 = dict(dtype=torch.int32, device="cuda")
+    P, strm = _lib.ptr, _lib.stream_of(g.col)
+
+    def fill(pos, row_ptr):
+        nbh = neighbors._grid(st["cell"], rc)
+        nb = (_lib.I32 * 6)(*nbh)
+        pos = torch.as_tensor(pos, dtype=torch.float64, device="cuda")
+        cell = torch.as_tensor(st["cell"].reshape(9), dtype=torch.float64, device="cuda")
+        inv = torch.as_tensor(np.linalg.inv(st["cell"]).reshape(9), dtype=torch.float64, device="cuda")
+        nbins = nbh[0] * nbh[1] * nbh[2]
+        bin_of, wrap, cnt, start, slots, atoms = (torch.empty(s, **i32) for s in (N, (N, 3), nbins, nbins + 1, nbins, N))
+        _lib.call("face_nbr_bin", P(pos), N, P(inv), nb, P(bin_of), P(wrap), P(cnt), P(start), P(slots), P(atoms), strm)
+        E = int(row_ptr[-1])
+        key = torch.empty(E, dtype=torch.int64, device="cuda")
+        col, S = torch.full((E,), 1 << 30, **i32), torch.empty(E, 3, **i32)
+        shift, over = torch.empty(E, 3, device="cuda"), torch.zeros(1, **i32)
+        rp = torch.as_tensor(row_ptr.astype(np.int32), device="cuda")
+        _lib.call("face_nbr_fill", P(pos), N, None, None, P(cell), None, None, rc, nb, P(bin_of), P(wrap), P(start),
+                  P(atoms), P(rp), P(key), P(col), P(S), P(shift), P(over), strm)
+        return rp, col, S, int(over)
+
+    # one row five pairs short
+    short = counts.copy()
+    short[7] -= 5
+    rp, col, S, over = fill(st["pos"], np.concatenate([[0], np.cumsum(short)]))
+    assert over == 5
+    full = [set(zip(c.tolist(), map(tuple, s.tolist()))) for c, s in
+            ((g.col[g.row_ptr[i]:g.row_ptr[i + 1]].cpu(), g.S[g.row_ptr[i]:g.row_ptr[i + 1]].cpu()) for i in range(N))]
+    rph = rp.cpu().numpy()
+    for i in range(N):
+        got = list(zip(col[rph[i]:rph[i + 1]].tolist(), map(tuple, S[rph[i]:rph[i + 1]].tolist())))
+        assert set(got) <= full[i] and len(set(got)) == short[i], i
+    # atom 3 lies 600 cells away: its images do not fit the key
+    far = st["pos"].copy()
+    far[3, 0] += 600 * L
+    rp, col, S, over = fill(far, np.concatenate([[0], np.cumsum(counts)]))
+    assert over > 0 and int(col.min()) >= 0 and int(col.max()) < N
+    # indexes that are no atoms
+    col = g.col.clone()
+    bad = torch.tensor([0, 100, g.E - 1], device="cuda")
+    col[bad] = torch.tensor([-5, N, 1 << 30], **i32)
+    rev, missing = torch.empty(g.E, **i32), torch.zeros(1, **i32)
+    _lib.call("face_nbr_rev", P(g.row_ptr), P(col), P(g.S), N, P(rev), P(missing), strm)
+    assert int(missing) >= 3 and torch.equal(rev[bad].long(), bad)
