@@ -396,9 +396,17 @@ def dir_transport(Vb, Mb, phi, Y, graph, Kd, transport):
 
 def _rows16(*ts):
     """Whether every tensor (None skipped) is a float32 device matrix or vector whose rows the row-block
-    kernels take as they are: unit column stride, 16-byte aligned rows."""
+    kernels take as they are: unit column stride, 16-byte aligned rows one after the other."""
     return all(t is None or (t.is_cuda and t.dtype == torch.float32 and t.stride(-1) == 1 and t.data_ptr() % 16 == 0
-                             and (t.dim() == 1 or t.stride(0) % 4 == 0)) for t in ts)
+                             and (t.dim() == 1 or (t.stride(0) % 4 == 0 and t.stride(0) >= t.shape[1]))) for t in ts)
+
+
+def _gemm_rows(x):
+    """x itself when the row-block kernels take it as an operand: float rows of unit stride, 16-byte aligned,
+    one after the other (an expanded gradient repeats one row); else a dense copy."""
+    ok = (x.dtype == torch.float32 and x.stride(1) == 1 and x.stride(0) % 4 == 0 and x.stride(0) >= x.shape[1]
+          and x.data_ptr() % 16 == 0)
+    return x if ok else x.float().clone(memory_format=torch.contiguous_format)
 
 
 class ReadoutMLP(torch.autograd.Function):
@@ -428,10 +436,10 @@ class ReadoutMLP(torch.autograd.Function):
                     and _rows16(W0a, W0b, b0, W1, b1, W2, Wg, bg) and inv.dtype == torch.float32
                     and h.dtype == torch.float32 and inv.is_cuda)
         if ctx.rows:
-            inv_, h_ = _aligned_rows(inv), _aligned_rows(h)
+            inv_, h_ = _gemm_rows(inv), _gemm_rows(h)
             z0 = torch.empty(N, H1, device=dev)
             if hb is not None:                            # b0 + h W0b^T precomputed (h a constant)
-                probs = [lin(inv_, W0a, z0, beta=1.0, y0=_aligned_rows(hb))]
+                probs = [lin(inv_, W0a, z0, beta=1.0, y0=_gemm_rows(hb))]
             else:
                 probs = [lin(inv_, W0a, z0, x2=h_, w2=W0b, bias=b0)]
             gvm = None
@@ -487,12 +495,12 @@ class ReadoutMLP(torch.autograd.Function):
                 rows_linear([lin(W2[:1].expand(N, -1), W1, da0, x_op=2, xz=z1, sum_row=ge_)], w_kn=True,
                             label="readout_hid_bwd")
             else:
-                gh_ = _aligned_rows(gh)
+                gh_ = _gemm_rows(gh)
                 da1 = torch.empty_like(z1)
                 rows_linear([lin(gh_, W2[1:], da1, bias=W2[0], bias_row=ge_)], w_kn=True, label="readout_out_bwd")
                 rows_linear([lin(da1, W1, da0, x_op=2, xz=z1)], w_kn=True, label="readout_hid_bwd")
             dinv = torch.empty(N, W0a.shape[1], device=dev)
-            probs = [lin(da0, W0a, dinv, x_op=2, xz=z0, x2=_aligned_rows(ggvm) if gate else None,
+            probs = [lin(da0, W0a, dinv, x_op=2, xz=z0, x2=_gemm_rows(ggvm) if gate else None,
                          w2=Wg if gate else None)]
             dh = None
             if need_h:

@@ -1263,6 +1263,50 @@ def test_readout_mlp_matches_torch(N, C, last, gate, const_h):
         assert rel(got[1], want[1]) < 5e-6
 
 
+def _readout_case(N, C, seed=0):
+    """Random operands of ops.readout_mlp with the gate: (inv, h, weights)."""
+    torch.manual_seed(seed)
+    r = lambda *s: torch.randn(*s, device=DEV) / s[-1] ** 0.5
+    ws = [r(2 * C, 9 * C), r(2 * C, C), r(2 * C), r(2 * C, 2 * C), r(2 * C), r(C + 1, 2 * C), r(C + 1), r(2 * C, 9 * C),
+          r(2 * C)]
+    return torch.randn(N, 9 * C, device=DEV), torch.randn(N, C, device=DEV), ws
+
+
+@pytest.mark.parametrize("N", [1, 70])
+def test_readout_mlp_takes_broadcast_rows(N):
+    """Expanded operands and upstream gradients (row stride 0, as a sum over atoms gives; strides of
+    one-row tensors; transposed ones) give the results of their dense copies."""
+    from face_amd import ops
+    say("readout_mlp broadcast", N)
+    C = 32
+    inv, h, ws = _readout_case(N, C)
+    row = lambda w: torch.randn(1, w, device=DEV).expand(N, w)
+    odd = lambda w: torch.randn(w, N, device=DEV).t()
+    hb = row(2 * C)
+
+    def run(inv, h, hb, ups):
+        i, x = inv.detach().requires_grad_(True), h.detach().requires_grad_(True)
+        outs = ops.readout_mlp(i, x, *ws, False, hb)
+        return list(outs) + list(torch.autograd.grad(outs, [i, x], ups))
+
+    for give_hb in (False, True):
+        for ins in ((row(9 * C), row(C)), (odd(9 * C), odd(C)), (inv, h)):
+            for ups in ([row(1), row(C), row(2 * C)], [odd(1), odd(C), odd(2 * C)]):
+                got = run(*ins, hb if give_hb else None, ups)
+                want = run(*(t.clone(memory_format=torch.contiguous_format) for t in ins), hb.clone(
+                    memory_format=torch.contiguous_format) if give_hb else None,
+                    [u.clone(memory_format=torch.contiguous_format) for u in ups])
+                assert all(torch.equal(a, b) for a, b in zip(got, want))
+    # a loss over sums of the outputs, as a user writes it
+    i, x = inv.requires_grad_(True), h.requires_grad_(True)
+    v = torch.randn(C, device=DEV)
+    outs = ops.readout_mlp(i, x, *ws, False)
+    got = torch.autograd.grad(outs[0].sum() + (outs[1].sum(0) * v).sum() + outs[2].sum(), [i, x])
+    outs = ops.readout_mlp(i, x, *ws, False)
+    want = torch.autograd.grad(outs, [i, x], [torch.ones(N, 1, device=DEV), v.repeat(N, 1), torch.ones(N, 2 * C, device=DEV)])
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 @pytest.mark.parametrize("side", ["xs", "ys"])
 def test_rows_linear_scale_tables_larger_than_lds(side):
     """64 groups whose scale rows do not fit in LDS beside the weights: read from memory instead, the
@@ -1411,6 +1455,25 @@ def test_scaled_mix_forward_backward(transport, Cin, merge, monkeypatch):
     errs = [rel(a, b) for a, b in zip(A, A2)] + [rel(a, b) for a, b in zip(gr, gr2)]
     say("   errs", errs)
     assert max(errs) < 1e-5, errs
+
+
+def test_scaled_mix_takes_broadcast_transport_sums():
+    """Transport sums and weights whose rows are one row repeated (stride 0) give the results of their dense
+    copies (to the rounding of two float32 routes)."""
+    from face_amd import ops
+    say("scaled mix broadcast")
+    torch.manual_seed(8)
+    N, C, Dw = 45, 32, 64
+    grp = torch.zeros(N, device=DEV, dtype=torch.int32)
+    s_tab = torch.rand(1, 4 * C, device=DEV) + 0.5
+    Af = [torch.randn(k, N, C, device=DEV) for k in (1, 3, 6, 10)]
+    wm = [torch.randn(C, C, device=DEV) / C ** 0.5 for _ in range(4)]
+    D = [torch.randn(1, 1, Dw, device=DEV).expand(k, N, Dw) for k in (3, 6)]
+    wt = [torch.randn(C, Dw, device=DEV) / 8, torch.randn(1, Dw, device=DEV).expand(C, Dw)]
+    dense = lambda ts: [t.clone(memory_format=torch.contiguous_format) for t in ts]
+    got = ops.scaled_mix(s_tab, grp, wm, wt, *D, Af)
+    want = ops.scaled_mix(s_tab, grp, wm, dense(wt), *dense(D), Af)
+    assert all(rel(a, b) < 1e-5 for a, b in zip(got, want))
 
 
 @pytest.mark.parametrize("n_sets,C,in_row", [(1, 160, False), (2, 160, False), (2, 96, False), (3, 32, False),
