@@ -394,18 +394,23 @@ def dir_transport(Vb, Mb, phi, Y, graph, Kd, transport):
     return DirTransport.apply(Vb, Mb, phi, Y, graph, Kd, transport)
 
 
+GEMM_SPAN = 1 << 31                 # elements an operand of face_rows_linear spans at most (rows x stride), exclusive
+
+
 def _rows16(*ts):
     """Whether every tensor (None skipped) is a float32 device matrix or vector whose rows the row-block
-    kernels take as they are: unit column stride, 16-byte aligned rows one after the other."""
+    kernels take as they are: unit column stride, 16-byte aligned rows one after the other, fewer than
+    GEMM_SPAN elements."""
     return all(t is None or (t.is_cuda and t.dtype == torch.float32 and t.stride(-1) == 1 and t.data_ptr() % 16 == 0
-                             and (t.dim() == 1 or (t.stride(0) % 4 == 0 and t.stride(0) >= t.shape[1]))) for t in ts)
+                             and (t.dim() == 1 or (t.stride(0) % 4 == 0 and t.stride(0) >= t.shape[1]
+                                                   and t.shape[0] * t.stride(0) < GEMM_SPAN))) for t in ts)
 
 
 def _gemm_rows(x):
     """x itself when the row-block kernels take it as an operand: float rows of unit stride, 16-byte aligned,
-    one after the other (an expanded gradient repeats one row); else a dense copy."""
+    one after the other (an expanded gradient repeats one row), not too far apart; else a dense copy."""
     ok = (x.dtype == torch.float32 and x.stride(1) == 1 and x.stride(0) % 4 == 0 and x.stride(0) >= x.shape[1]
-          and x.data_ptr() % 16 == 0)
+          and x.shape[0] * x.stride(0) < GEMM_SPAN and x.data_ptr() % 16 == 0)
     return x if ok else x.float().clone(memory_format=torch.contiguous_format)
 
 
@@ -421,8 +426,8 @@ class ReadoutMLP(torch.autograd.Function):
     Widths that are multiples of 16 run on the row-block kernels, SiLU and its derivative applied to
     the rows as they load: z0 and the gate row in one launch, then z1, the residual rows, the energy
     row; backward in three launches (10,752 atoms, C = 160, forward and backward: 667 us on the
-    library's float32 products with the activations between them, 405 us here). Other widths, and
-    weights without 16-byte aligned rows, take the library products."""
+    library's float32 products with the activations between them, 405 us here). Other widths,
+    weights without 16-byte aligned rows and rows past GEMM_SPAN elements take the library products."""
 
     @staticmethod
     def forward(ctx, inv, h, W0a, W0b, b0, W1, b1, W2, b2, Wg, bg, last, hb):
@@ -430,7 +435,8 @@ class ReadoutMLP(torch.autograd.Function):
         ctx.w = (W0a, W0b, W1, W2, Wg)
         C, H1, H2 = W0b.shape[1], W0a.shape[0], W1.shape[0]
         N, dev = inv.shape[0], inv.device
-        ctx.rows = (N > 0 and all(v % 16 == 0 for v in (C, H1, H2, W0a.shape[1])) and W2.shape[0] == C + 1
+        widest = max(C, H1, H2, W0a.shape[1], 0 if Wg is None else Wg.shape[0])
+        ctx.rows = (0 < N * widest < GEMM_SPAN and all(v % 16 == 0 for v in (C, H1, H2, W0a.shape[1])) and W2.shape[0] == C + 1
                     and (Wg is None or (Wg.shape[0] % 16 == 0 and bg is not None))
                     and all(b is not None for b in (b0, b1, b2))
                     and _rows16(W0a, W0b, b0, W1, b1, W2, Wg, bg) and inv.dtype == torch.float32

@@ -1457,6 +1457,44 @@ def test_scaled_mix_forward_backward(transport, Cin, merge, monkeypatch):
     assert max(errs) < 1e-5, errs
 
 
+def test_readout_and_mix_past_the_span_of_a_row_block(monkeypatch):
+    """Operands of 2^31 elements and more (eight rows 2^28 apart), which the row-block kernels refuse, and,
+    with the limit lowered, as many rows: the results of small dense operands, bit for bit where the
+    operands are copied, to the rounding of two float32 routes where the library products take over."""
+    from face_amd import ops
+    say("readout and mix past the span")
+    N, C, Dw, ld = 8, 32, 64, 1 << 28
+    inv, h, ws = _readout_case(N, C)
+    buf = torch.empty(7 * ld + 8192, device=DEV)
+
+    def far(t, at):
+        v = buf.as_strided(t.shape, (ld, 1), at)
+        return v.copy_(t)
+
+    def readout(inv, h, ups):
+        i, x = inv.detach().requires_grad_(True), h.detach().requires_grad_(True)
+        outs = ops.readout_mlp(i, x, *ws, False)
+        return [o.detach() for o in outs] + list(torch.autograd.grad(outs, [i, x], ups))
+
+    ups = [torch.randn(N, w, device=DEV) for w in (1, C, 2 * C)]
+    want = readout(inv, h, ups)
+    got = readout(far(inv, 0), far(h, 1024), [ups[0], far(ups[1], 2048), far(ups[2], 3072)])
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    grp = torch.zeros(N, device=DEV, dtype=torch.int32)
+    s_tab = torch.rand(1, 4 * C, device=DEV) + 0.5
+    Af = [torch.randn(k, N, C, device=DEV) for k in (1, 3, 6, 10)]
+    wm = [torch.randn(C, C, device=DEV) / C ** 0.5 for _ in range(4)]
+    D1, D2 = torch.randn(3, N, Dw, device=DEV), torch.randn(6, N, Dw, device=DEV)
+    wt = [torch.randn(C, Dw, device=DEV) / 8 for _ in range(2)]
+    want_mix = ops.scaled_mix(s_tab, grp, wm, wt, D1, D2, Af)
+    spread = torch.empty(23 * (1 << 27) + Dw, device=DEV)
+    Df = spread.as_strided(D1.shape, (8 << 27, 1 << 27, 1), 0).copy_(D1)      # 24 rows 2^27 elements apart
+    got_mix = ops.scaled_mix(s_tab, grp, wm, wt, Df, D2, Af)
+    monkeypatch.setattr(ops, "GEMM_SPAN", N * 9 * C)                          # the readout's widest rows reach it
+    got = readout(inv, h, ups)
+    assert all(rel(a, b) < 1e-5 for a, b in zip(got + list(got_mix), want + list(want_mix)))
+
+
 def test_scaled_mix_takes_broadcast_transport_sums():
     """Transport sums and weights whose rows are one row repeated (stride 0) give the results of their dense
     copies (to the rounding of two float32 routes)."""
