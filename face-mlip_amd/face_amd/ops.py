@@ -493,7 +493,7 @@ class ReadoutMLP(torch.autograd.Function):
         if not ctx.last and gh is None:
             gh = z0.new_zeros(N, C)
         gate = ggvm is not None and Wg is not None
-        if ctx.rows:
+        if ctx.rows and not torch.is_grad_enabled():      # create_graph: torch's own, which refuse a second one
             dev = z0.device
             ge_ = ge.float().contiguous().view(-1)
             da0 = torch.empty_like(z0)

@@ -1457,6 +1457,23 @@ def test_scaled_mix_forward_backward(transport, Cin, merge, monkeypatch):
     assert max(errs) < 1e-5, errs
 
 
+@pytest.mark.parametrize("last", [False, True])
+def test_readout_mlp_refuses_a_second_derivative(last):
+    """The input gradients have no derivative of their own: asked for with create_graph they are refused when
+    differentiated, alone or in a sum with something that has one, never dropped from it."""
+    from face_amd import ops
+    say("readout_mlp double backward", last)
+    inv, h, ws = _readout_case(50, 32)
+    inv.requires_grad_(True)
+    outs = [o for o in ops.readout_mlp(inv, h, *ws, last) if o is not None]
+    ups = [torch.randn_like(o).requires_grad_(True) for o in outs]
+    want = torch.autograd.grad(outs, inv, [u.detach() for u in ups], retain_graph=True)[0]
+    d_inv = torch.autograd.grad(outs, inv, ups, create_graph=True)[0]
+    assert rel(d_inv, want) < 1e-5
+    with pytest.raises(RuntimeError, match="not implemented"):
+        torch.autograd.grad(d_inv.sum() + sum((u * u).sum() for u in ups), ups)
+
+
 def test_readout_and_mix_past_the_span_of_a_row_block(monkeypatch):
     """Operands of 2^31 elements and more (eight rows 2^28 apart), which the row-block kernels refuse, and,
     with the limit lowered, as many rows: the results of small dense operands, bit for bit where the
