@@ -219,7 +219,7 @@ __global__ __launch_bounds__(256) void silu_dot_kernel(const float* __restrict__
     for (int c = 4 * lane; c < k; c += 4 * kWave) {
         const v4f a = ld4(x + r * ld_x + c), f = ld4(w + c);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s = fmaf(a[i] * gemm_sigmoid(a[i]), f[i], s);
+        for (int i = 0; i < 4; ++i) s = fmaf(gemm_op(a[i], 0.f, 1), f[i], s);
     }
     s = group_sum(s, kWave);
     if (lane == 0) y[r] = s + (b ? *b : 0.f);

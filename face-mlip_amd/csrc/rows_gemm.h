@@ -60,15 +60,28 @@ struct GemmProb {
     int64_t w_off;                         // its split weights in the workspace (bytes)
 };
 
-// silu and its derivative with the hardware exp2 and reciprocal (about 1 ulp each)
-__device__ __forceinline__ float gemm_sigmoid(float x) {
-    return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.44269504088896341f * x));
+// Logistic function (and one minus it) with the hardware exp2 and reciprocal, each corrected to first order:
+// e = exp(-x) from the rounded exponent t and what its rounding and that of log2(e) left over, 1 / (1 + e) by
+// one Newton step. Uncorrected, x < 0 came out 0.3 to 0.8 ulp too large on average (silu: mean -0.30 ulp,
+// rms 0.90). |x| is cut at 80, where exp(-|x|) is 2e-35 and all intermediate values are finite.
+__device__ __forceinline__ float gemm_sigmoid(float x, float& rest) {
+    constexpr float kL = 0x1.715476p+0f, kLow = 0x1.4ae0cp-26f;           // log2(e) = kL + kLow
+    const float a = __builtin_amdgcn_fmed3f(x, -80.f, 80.f), t = -kL * a;
+    const float lo = fmaf(-kLow, a, fmaf(-kL, a, -t));
+    float e = __builtin_amdgcn_exp2f(t);
+    e = fmaf(e, 0.693147181f * lo, e);
+    const float d = 1.f + e;
+    float r = __builtin_amdgcn_rcpf(d);
+    r = fmaf(fmaf(-d, r, 1.f), r, r);
+    rest = e * r;
+    return r;
 }
 __device__ __forceinline__ float gemm_op(float x, float z, int op) {
-    if (op == 1) return x * gemm_sigmoid(x);
+    float rest;
+    if (op == 1) return x * gemm_sigmoid(x, rest);
     if (op == 2) {                                                     // x * d silu(z) / dz
-        const float sg = gemm_sigmoid(z);
-        return x * (sg * (1.f + z * (1.f - sg)));
+        const float sg = gemm_sigmoid(z, rest);
+        return x * (sg * fmaf(z, rest, 1.f));
     }
     return x;
 }

@@ -1263,6 +1263,34 @@ def test_readout_mlp_matches_torch(N, C, last, gate, const_h):
         assert rel(got[1], want[1]) < 5e-6
 
 
+@pytest.mark.parametrize("lo,hi", [(-20.0, -6.0), (-6.0, -1.0), (-1.0, 0.0), (0.0, 1.0), (1.0, 20.0)])
+def test_silu_on_load_is_rounded_without_bias(lo, hi):
+    """silu and the silu derivative as the row kernels form them (identity weights: the products are exact)
+    and as the energy row does, in ulps of the fp64 values: the hardware exponential's ulp and at most six
+    roundings to nearest (0.29 rms each), so an rms below 1 and a mean within 0.1 (raw exp2 and reciprocal:
+    rms 1 to 5 and mean 0.3 to 0.8 for x < 0; 1 - sigmoid for the slope: rms 2.8 for x > 1)."""
+    from face_amd import _lib, ops
+    say("silu on load", lo, hi)
+    torch.manual_seed(9)
+    m, k = 4096, 64
+    z = torch.rand(m, k, device=DEV) * (hi - lo) + lo
+    one, eye = torch.ones(m, k, device=DEV), torch.eye(k, device=DEV)
+    y1, y2, e = torch.empty(m, k, device=DEV), torch.empty(m, k, device=DEV), torch.empty(m, device=DEV)
+    ops.rows_linear([ops.lin(z, eye, y1, x_op=1)])
+    ops.rows_linear([ops.lin(one, eye, y2, x_op=2, xz=z)])
+    _lib.call("face_silu_dot", _lib.ptr(z), k, m, k, _lib.ptr(eye[3].contiguous()), None, _lib.ptr(e), _lib.stream_of(e))
+    zd = z.double()
+    s = torch.sigmoid(zd)
+    for what, got, ref in (("silu", y1, zd * s), ("energy row", e, (zd * s)[:, 3]), ("slope", y2, s * (1 + zd * (1 - s)))):
+        ok = ref.abs() > (0.2 if what == "slope" else 0)             # away from the slope's zero at -1.278
+        if not ok.any():
+            continue
+        err = ((got.double() - ref) / 2.0 ** (torch.floor(torch.log2(ref.abs())) - 23))[ok]
+        say(f"   {what} mean {err.mean():+.3f} rms {err.pow(2).mean().sqrt():.3f}")
+        assert err.pow(2).mean().sqrt() < 1.0
+        assert err.mean().abs() < 0.1
+
+
 def _readout_case(N, C, seed=0):
     """Random operands of ops.readout_mlp with the gate: (inv, h, weights)."""
     torch.manual_seed(seed)
