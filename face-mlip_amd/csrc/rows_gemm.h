@@ -299,36 +299,37 @@ __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(
     const uint32_t yo = 4 * (uint32_t)(4 * hf * (int)ld_y + j);
     const bool full = m0 + kGemmRows <= M;
     auto row_ok = [&](int r) __attribute__((always_inline)) { return m0 + 8 * (r >> 2) + (r & 3) + 4 * hf < M; };
-    // accumulators start at beta y0, else zero
-    v16f acc[NB];
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[nb][r] = 0.f;
+    // beta y0 of a column block. A sum onto y starts there, its loads under the first x rows'; the forms with
+    // an initial sum of their own (a residual, larger than what is added to it) add it after the products,
+    // which then round at their own size (readout, d h: 3.5e-7 with the residual first, 0.7e-7).
     const float beta = P.beta;
-    if (beta != 0.f) {
+    auto initial = [&](int nb, v16f& v) __attribute__((always_inline)) {
         const float* y0 = P.y0 ? P.y0 : P.y;
         const int64_t ld0 = P.y0 ? P.ld_y0 : ld_y;
         const float* y0b = y0 + m0 * ld0 + n0;
         const uint32_t o0 = 4 * (uint32_t)(4 * hf * (int)ld0 + j);
         const int n_y0 = min(P.n_y0 - n0, ns);
+        if (full && 32 * nb + 32 <= n_y0) {                   // uniform
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-            if (full && 32 * nb + 32 <= n_y0) {               // uniform
+            for (int r = 0; r < 16; ++r) v[r] = beta * *at_off(y0b + (8 * (r >> 2) + (r & 3)) * ld0 + 32 * nb, o0);
+        } else if (32 * nb < n_y0 && m0 < M) {
+            const int64_t c = min(32 * nb + j, n_y0 - 1);
 #pragma unroll
-                for (int r = 0; r < 16; ++r) acc[nb][r] = *at_off(y0b + (8 * (r >> 2) + (r & 3)) * ld0 + 32 * nb, o0);
-            } else if (32 * nb < n_y0 && m0 < M) {
-                const int64_t c = min(32 * nb + j, n_y0 - 1);
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {                // at the nearest valid place, zero outside
-                    const int64_t rr = min(m0 + 8 * (r >> 2) + (r & 3) + 4 * hf, M - 1);
-                    const float v = y0[rr * ld0 + n0 + c];
-                    acc[nb][r] = (32 * nb + j < n_y0 && row_ok(r)) ? v : 0.f;
-                }
+            for (int r = 0; r < 16; ++r) {                    // at the nearest valid place, zero outside
+                const int64_t rr = min(m0 + 8 * (r >> 2) + (r & 3) + 4 * hf, M - 1);
+                const float x = y0[rr * ld0 + n0 + c];
+                v[r] = (32 * nb + j < n_y0 && row_ok(r)) ? beta * x : 0.f;
             }
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[nb][r] *= beta;
         }
+    };
+    v16f acc[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[nb][r] = 0.f;
+    if (!XO && beta != 0.f) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) initial(nb, acc[nb]);
     }
     __syncthreads();
     const int nchunk = (K + kGemmK - 1) / kGemmK;
@@ -406,7 +407,18 @@ __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(
         for (int i = 0; i < kGemmRows; ++i) plain_row<XM>(A, P, m0 + i, n0, ns, lane);
         return;
     }
-    // epilogue: bias and y scale, then stores of 128 bytes per row
+    // epilogue: initial sum, bias and y scale, then stores of 128 bytes per row
+    if (XO && beta != 0.f) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            v16f v;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) v[r] = 0.f;
+            initial(nb, v);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[nb][r] += v[r];
+        }
+    }
     if (XF && P.sum_row) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -536,8 +548,8 @@ __global__ __launch_bounds__(4 * kWave, 2) void rows_gemm_direct_kernel(GemmArgs
     const float* y0 = P.y0 ? P.y0 : P.y;
     const int64_t ld_y = P.ld_y, ld0 = P.y0 ? P.ld_y0 : ld_y;
     auto out_row = [&](int r) __attribute__((always_inline)) { return m0 + 8 * (r >> 2) + (r & 3) + 4 * hf; };
-    if (beta != 0.f && kp == 0) {
-        const int n_y0 = min(P.n_y0 - n0, ns);
+    const int n_y0 = min(P.n_y0 - n0, ns);
+    if (!XO && beta != 0.f && kp == 0) {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             if (32 * nb >= n_y0) break;
@@ -600,6 +612,18 @@ __global__ __launch_bounds__(4 * kWave, 2) void rows_gemm_direct_kernel(GemmArgs
         for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
             for (int i = 0; i < NR; ++i) v[nb][i] = acc[nb][i];
+    }
+    if (XO && beta != 0.f) {                                  // after the products, as in the staged kernel
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            if (32 * nb >= n_y0) break;
+            const int64_t c = n0 + min(32 * nb + j, n_y0 - 1);
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                const float x = y0[min(out_row(rb + i), M - 1) * ld0 + c];
+                v[nb][i] += (32 * nb + j < n_y0 && out_row(rb + i) < M) ? beta * x : 0.f;
+            }
+        }
     }
     float chk = 0.f;
 #pragma unroll

@@ -1263,6 +1263,26 @@ def test_readout_mlp_matches_torch(N, C, last, gate, const_h):
         assert rel(got[1], want[1]) < 5e-6
 
 
+@pytest.mark.parametrize("op", [0, 1])
+@pytest.mark.parametrize("m", [40, 20000, 170000])
+def test_rows_linear_adds_a_residual_once(m, op):
+    """An initial sum of its own (y0, a thousand times the products) is added to the finished products: one
+    rounding of the result and the products' own error (below 2^-21 |x| |w|), in the direct kernel, the staged one
+    and the one with the weights split ahead; not a rounding at the residual's size per instruction."""
+    from face_amd import ops
+    say("rows_linear residual", m, op)
+    torch.manual_seed(m)
+    k, n = 320, 160
+    x, w = torch.randn(m, k, device=DEV), torch.randn(n, k, device=DEV) / k ** 0.5
+    y0, y = 1000 * torch.randn(m, n, device=DEV), torch.empty(m, n, device=DEV)
+    ops.rows_linear([ops.lin(x, w, y, x_op=op, y0=y0, beta=0.5)])
+    xd = torch.nn.functional.silu(x.double()) if op else x.double()
+    wd = w.double().t().contiguous()
+    ref = 0.5 * y0.double() + xd @ wd
+    bound = 2.0 ** -24 * ref.abs() + 2.0 ** -21 * (xd.abs() @ wd.abs())
+    assert bool(((y.double() - ref).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("lo,hi", [(-20.0, -6.0), (-6.0, -1.0), (-1.0, 0.0), (0.0, 1.0), (1.0, 20.0)])
 def test_silu_on_load_is_rounded_without_bias(lo, hi):
     """silu and the silu derivative as the row kernels form them (identity weights: the products are exact)
