@@ -1,5 +1,6 @@
 // face_rows_linear: argument checks, launch shapes and the plain input mode of the row-block linear
 // layers (rows_gemm.h).
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -15,6 +16,33 @@ static bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 }  // namespace face
 
 using namespace face;
+
+// The chunks of negated weights of a sum over K (rows_gemm.h): of the starts in the first half, the one that
+// comes nearest to half of the drift between the turns.
+static void turn_chunks(GemmProb& p, bool onto_y) {
+    constexpr int kMax = 128;
+    const int nk = p.k / 16, nc = (nk + 1) / 2;
+    p.turn0 = p.turn1 = nc;
+    if (nc < 2) return;
+    if (nc > kMax) {
+        p.turn0 = nc / 5, p.turn1 = p.turn0 + nc / 2;
+        return;
+    }
+    float sum[kMax + 1];                                       // drift of the first c chunks
+    sum[0] = 0.f;
+    for (int c = 0, st = 0; c < nc; ++c) {
+        float d = 0.f;
+        for (; st < nk && st < 2 * c + 2; ++st) d += onto_y ? 1.f : (st == 0 ? 6.5f : std::sqrt((float)(st + 1)));
+        sum[c + 1] = sum[c] + d;
+    }
+    float best = 1e30f;
+    for (int a = 1, b = 1; a <= (nc + 1) / 2; ++a) {
+        auto off = [&](int e) { return std::fabs(2.f * (sum[e] - sum[a]) - sum[nc]); };
+        b = std::max(a, b);
+        while (b < nc && off(b + 1) <= off(b)) ++b;
+        if (off(b) < 0.999f * best) best = off(b), p.turn0 = a, p.turn1 = b;
+    }
+}
 
 // Validate problem s and fill p (everything but the tiling); 0 or a FACE_ERR_* status.
 static int fill_prob(const face_lin_problem& s, int w_kn, bool scaled, const float* x_scale, const float* y_scale,
@@ -171,6 +199,7 @@ extern "C" int face_rows_linear_ws(const face_lin_problem* probs, int32_t n_prob
         if (st) return st;
     }
     if (x_scale && any_ext) return FACE_ERR_UNSUPPORTED;                 // x scale with split / op / y0
+    for (int i = 0; i < n_probs; ++i) turn_chunks(A.p[i], A.p[i].beta != 0.f && !any_ext);
     c.probs = probs, c.n_probs = n_probs, c.K = K, c.n_widest = n_widest, c.max_lds = device_max_lds();
     c.n_cu = device_cu_count(), c.x_scale = x_scale != nullptr, c.y_scale = y_scale != nullptr, c.any_ext = any_ext;
     c.any_op = any_op;

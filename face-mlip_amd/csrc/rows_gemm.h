@@ -58,7 +58,21 @@ struct GemmProb {
     int n_y0;
     int64_t first_block;                   // first work item of this problem
     int64_t w_off;                         // its split weights in the workspace (bytes)
+    int turn0, turn1;                      // chunks of negated weights (see flip_sign)
 };
+
+// The matrix instruction cuts each addend, aligned to the largest of the sum, below 2^-8 of an ulp towards
+// minus infinity, so a long sum drifts: its mean error over random operands was -1.1e-8 of the results' rms at
+// K = 160 and -2.7e-8 at 512, the same sign in every output, which a sum over atoms collects (fp32
+// instructions: none). Chunks [turn0, turn1) of 32 k therefore enter with negated weights into accumulators
+// whose sign is turned before and after, so that two parts of the sum drift in opposite directions. A step of
+// 16 k drifts as the accumulators grow, by the square root of its number, the first one 6.5 times the unit (its
+// last product is larger than the sum so far), and all alike where the sum starts at y: turn_chunks (gemm.hip)
+// puts half of the whole between the turns. What is left is about 1e-9 from K = 80 on, 3e-9 at 64, 5e-9 at 48;
+// one chunk keeps its 7e-9.
+__device__ __forceinline__ v4f flip_sign(v4f v, uint32_t sign) {
+    return __builtin_bit_cast(v4f, __builtin_bit_cast(v4u, v) ^ sign);
+}
 
 // Logistic function (and one minus it) with the hardware exp2 and reciprocal, each corrected to first order:
 // e = exp(-x) from the rounded exponent t and what its rounding and that of log2(e) left over, 1 / (1 + e) by
@@ -182,6 +196,7 @@ __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(
     const int n0 = (local - tile * slices) * NSB;
     const int ns = min(NSB, N - n0);                          // a multiple of 16
     const int ncb = (N + 31) >> 5;                            // 32-column blocks
+    const int turn0 = P.turn0, turn1 = P.turn1;
     const int64_t M = P.m, m0 = ((int64_t)tile * NW + wv) * kGemmRows;
     const int64_t mb = min(m0, M - 1);                        // first row read (waves past m: the last row)
     const int jr = (int)min((int64_t)j, M - 1 - mb);          // this lane's input row - mb
@@ -255,7 +270,7 @@ __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(
             }
         }
     };
-    auto store_w = [&](int buf, const v4f (&bw)[WU]) __attribute__((always_inline)) {
+    auto store_w = [&](int c, int buf, const v4f (&bw)[WU]) __attribute__((always_inline)) {
         if (PS) {
 #pragma unroll
             for (int u = 0; u < WU; ++u)
@@ -265,7 +280,8 @@ __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(
             for (int u = 0; u < WI; ++u) {
                 int col, kg;
                 item(u, col, kg);
-                const Split8 w = split8(bw[2 * u], bw[2 * u + 1]);
+                const uint32_t sg = c >= turn0 && c < turn1 ? 0x80000000u : 0u;     // uniform
+                const Split8 w = split8(flip_sign(bw[2 * u], sg), flip_sign(bw[2 * u + 1], sg));
                 v8bf* d = reinterpret_cast<v8bf*>(smem + buf * BUF + ((kg >> 1) * NB + (col >> 5)) * 3072) + (kg & 1) * 32 +
                           (col & 31);
                 d[0] = w.h;
@@ -291,7 +307,7 @@ __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(
             sxs[g * A.kmax + k] = A.xs[(int64_t)g * A.ld_s + P.s_off + k];
         }
     }
-    store_w(0, bw);
+    store_w(0, 0, bw);
     // output element (row 8 (r >> 2) + 4 hf + (r & 3), column 32 nb + j) of the wave: a uniform base per
     // (r, nb) and one byte offset per lane
     const int64_t ld_y = P.ld_y;
@@ -334,66 +350,76 @@ __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(
     __syncthreads();
     const int nchunk = (K + kGemmK - 1) / kGemmK;
 #pragma unroll 1
-    for (int c = 0; c < nchunk; ++c) {
-        const int buf = c & 1, cn = min(c + 1, nchunk - 1);
-        load_w(cn, bw);
-        Split8 xq[2];
+    for (int c = 0, part = 0; part < 3; ++part) {
+        const int end = part == 0 ? turn0 : (part == 1 ? turn1 : nchunk);
+#pragma unroll 1
+        for (; c < end; ++c) {
+            const int buf = c & 1, cn = min(c + 1, nchunk - 1);
+            load_w(cn, bw);
+            Split8 xq[2];
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            const int k0 = min(kGemmK * c + 16 * s, K - 16);
-            v4f a = xn[2 * s], b = xn[2 * s + 1];
-            if (XS) {
-                if (A.side_lds) {
-                    a *= lds4_at(sxs, grp * A.kmax + k0 + 8 * hf);
-                    b *= lds4_at(sxs, grp * A.kmax + k0 + 8 * hf + 4);
-                } else {
-                    const float* t = A.xs + (int64_t)grp * A.ld_s + P.s_off + k0 + 8 * hf;
-                    a *= ld4(t);
-                    b *= ld4(t + 4);
+            for (int s = 0; s < 2; ++s) {
+                const int k0 = min(kGemmK * c + 16 * s, K - 16);
+                v4f a = xn[2 * s], b = xn[2 * s + 1];
+                if (XS) {
+                    if (A.side_lds) {
+                        a *= lds4_at(sxs, grp * A.kmax + k0 + 8 * hf);
+                        b *= lds4_at(sxs, grp * A.kmax + k0 + 8 * hf + 4);
+                    } else {
+                        const float* t = A.xs + (int64_t)grp * A.ld_s + P.s_off + k0 + 8 * hf;
+                        a *= ld4(t);
+                        b *= ld4(t + 4);
+                    }
+                }
+                if (XF && x_op && k0 < k1) {
+                    a = gemm_op4(a, zn[2 * s], x_op);
+                    b = gemm_op4(b, zn[2 * s + 1], x_op);
+                }
+                xq[s] = split8(a, b);
+            }
+            load_x(cn, xn, zn);
+            __builtin_amdgcn_sched_barrier(0);                    // the loads ahead are issued before the products
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                if (s && kGemmK * c + 16 >= K) break;
+                const v8bf* wf = reinterpret_cast<const v8bf*>(smem + buf * BUF + s * NB * 3072) + lane;
+                const Split8& x = xq[s];
+                // the limbs of the next column block are read ahead; the smallest products first
+                v8bf w[3];
+#pragma unroll
+                for (int q = 0; q < 3; ++q) w[q] = wf[q * 64];
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) {
+                    v8bf wn[3];
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) wn[q] = nb + 1 < NB ? wf[(nb + 1) * 192 + q * 64] : w[q];
+                    acc[nb] = mfma_32x32x16(x.l, w[0], acc[nb]);
+                    acc[nb] = mfma_32x32x16(x.h, w[2], acc[nb]);
+                    acc[nb] = mfma_32x32x16(x.m, w[1], acc[nb]);
+                    acc[nb] = mfma_32x32x16(x.m, w[0], acc[nb]);
+                    acc[nb] = mfma_32x32x16(x.h, w[1], acc[nb]);
+                    acc[nb] = mfma_32x32x16(x.h, w[0], acc[nb]);
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) w[q] = wn[q];
+                }
+                // issue order: the reads of blocks 0 and 1, then per block its products and the reads of the
+                // block after the next one
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) {
+                    if (nb == 0) __builtin_amdgcn_sched_group_barrier(0x100, NB > 1 ? 6 : 3, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
+                    if (nb + 2 < NB) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
                 }
             }
-            if (XF && x_op && k0 < k1) {
-                a = gemm_op4(a, zn[2 * s], x_op);
-                b = gemm_op4(b, zn[2 * s + 1], x_op);
-            }
-            xq[s] = split8(a, b);
+            store_w(cn, buf ^ 1, bw);
+            __syncthreads();
         }
-        load_x(cn, xn, zn);
-        __builtin_amdgcn_sched_barrier(0);                    // the loads ahead are issued before the products
+        if (part < 2) {
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            if (s && kGemmK * c + 16 >= K) break;
-            const v8bf* wf = reinterpret_cast<const v8bf*>(smem + buf * BUF + s * NB * 3072) + lane;
-            const Split8& x = xq[s];
-            // the limbs of the next column block are read ahead; the smallest products first
-            v8bf w[3];
+            for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-            for (int q = 0; q < 3; ++q) w[q] = wf[q * 64];
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                v8bf wn[3];
-#pragma unroll
-                for (int q = 0; q < 3; ++q) wn[q] = nb + 1 < NB ? wf[(nb + 1) * 192 + q * 64] : w[q];
-                acc[nb] = mfma_32x32x16(x.l, w[0], acc[nb]);
-                acc[nb] = mfma_32x32x16(x.h, w[2], acc[nb]);
-                acc[nb] = mfma_32x32x16(x.m, w[1], acc[nb]);
-                acc[nb] = mfma_32x32x16(x.m, w[0], acc[nb]);
-                acc[nb] = mfma_32x32x16(x.h, w[1], acc[nb]);
-                acc[nb] = mfma_32x32x16(x.h, w[0], acc[nb]);
-#pragma unroll
-                for (int q = 0; q < 3; ++q) w[q] = wn[q];
-            }
-            // issue order: the reads of blocks 0 and 1, then per block its products and the reads of the
-            // block after the next one
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                if (nb == 0) __builtin_amdgcn_sched_group_barrier(0x100, NB > 1 ? 6 : 3, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
-                if (nb + 2 < NB) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
-            }
+                for (int r = 0; r < 16; ++r) acc[nb][r] = -acc[nb][r];
         }
-        store_w(buf ^ 1, bw);
-        __syncthreads();
     }
     // Operands that round to a bf16 infinity have a NaN limb, which every product they enter carries into
     // the sums: a wave with a sum that is not finite forms its rows again in plain fp32 products.
@@ -536,6 +562,7 @@ __global__ __launch_bounds__(4 * kWave, 2) void rows_gemm_direct_kernel(GemmArgs
         }
     };
     const int s0 = nk * kp / KW, s1 = nk * (kp + 1) / KW;
+    const uint32_t sg = kp == 1 || kp == 2 ? 0x80000000u : 0u;   // the middle parts drift the other way (see flip_sign)
     Step b[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) load(s0 + d, b[d]);
@@ -571,7 +598,7 @@ __global__ __launch_bounds__(4 * kWave, 2) void rows_gemm_direct_kernel(GemmArgs
                 c.x[0] = gemm_op4(c.x[0], c.z[0], x_op);
                 c.x[1] = gemm_op4(c.x[1], c.z[1], x_op);
             }
-            const Split8 x = split8(c.x[0], c.x[1]);
+            const Split8 x = split8(flip_sign(c.x[0], sg), flip_sign(c.x[1], sg));
             Split8 w[NB];
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) w[nb] = split8(c.w[nb][0], c.w[nb][1]);
@@ -605,7 +632,10 @@ __global__ __launch_bounds__(4 * kWave, 2) void rows_gemm_direct_kernel(GemmArgs
             for (int i = 0; i < NR; ++i) {
                 v[nb][i] = ssum[(nb * 16 + rb + i) * kWave + lane];
 #pragma unroll
-                for (int k = 1; k < KW; ++k) v[nb][i] += ssum[((k * NB + nb) * 16 + rb + i) * kWave + lane];
+                for (int k = 1; k < KW; ++k) {
+                    const float p = ssum[((k * NB + nb) * 16 + rb + i) * kWave + lane];
+                    v[nb][i] += k == 1 || k == 2 ? -p : p;
+                }
             }
     } else {
 #pragma unroll
@@ -682,7 +712,8 @@ __global__ __launch_bounds__(kWave) inline void split_weights_kernel(GemmArgs A,
             b = ld4(p + 4);
         }
     }
-    const Split8 w = split8(a, b);
+    const uint32_t sg = (step >> 1) >= P.turn0 && (step >> 1) < P.turn1 ? 0x80000000u : 0u;
+    const Split8 w = split8(flip_sign(a, sg), flip_sign(b, sg));
     v8bf* d = reinterpret_cast<v8bf*>(work + P.w_off + local * 3072) + lane;
     d[0] = w.h;
     d[64] = w.m;

@@ -1263,6 +1263,30 @@ def test_readout_mlp_matches_torch(N, C, last, gate, const_h):
         assert rel(got[1], want[1]) < 5e-6
 
 
+@pytest.mark.parametrize("w_kn", [False, True])
+@pytest.mark.parametrize("route", ["direct", "staged", "ahead"])
+@pytest.mark.parametrize("k", [32, 48, 64, 96, 160, 320, 512, 1440])
+def test_rows_linear_sums_do_not_drift(k, route, w_kn):
+    """The mean error of many random sums, whose instructions all cut towards minus infinity: -0.7e-8
+    (k = 64) to -2.7e-8 (512) and -7.7e-8 (1440) of the results' rms when nothing turns their sign. With the
+    turns the drifts of single 16-k steps (1 to 6e-9 each) cancel but for about one step's, 2e-9; below k = 80
+    for what the first chunk of 32 has over the others, 5e-9, and a chunk alone keeps its 7e-9."""
+    torch.manual_seed(k)
+    m, n, reps = (40, 160, 200) if route == "direct" else (8192, 160, 1)
+    w = (torch.randn(k, n, device=DEV) if w_kn else torch.randn(n, k, device=DEV)) / k ** 0.5
+    wd = w.double() if w_kn else w.double().t().contiguous()
+    err, ref = [], []
+    for _ in range(reps):
+        x, y = torch.randn(m, k, device=DEV), torch.empty(m, n, device=DEV)
+        _rows_launch(x, w, y, w_kn, route == "ahead")
+        ref.append(x.double() @ wd)
+        err.append(y.double() - ref[-1])
+    err, rms = torch.cat(err), torch.cat(ref).pow(2).mean().sqrt()
+    mean, se = (err.mean() / rms).item(), (err.std() / rms / err.numel() ** 0.5).item()
+    say(f"rows_linear drift k {k} {route} kn {w_kn} mean {mean:+.2e} se {se:.1e} rms {(err.pow(2).mean().sqrt() / rms).item():.2e}")
+    assert abs(mean) < (2e-9 if k >= 80 else 5.5e-9 if k > 32 else 8e-9)
+
+
 @pytest.mark.parametrize("op", [0, 1])
 @pytest.mark.parametrize("m", [40, 20000, 170000])
 def test_rows_linear_adds_a_residual_once(m, op):
