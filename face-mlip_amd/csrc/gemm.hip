@@ -104,13 +104,13 @@ static int launch_rows(const RowsCtx& c, RowsShape S) {
 // Row strides past kGemmMaxLd (at most 63 rows of them: an operand has fewer than 2^31 elements) take the
 // direct kernel at any number of problems; its addresses are 64 bits wide.
 static RowsShape rows_shape(const RowsCtx& c) {
-    if (c.far) return {4, 1, 0, 4};
+    if (c.far) return {kDirectWaves, 1, 0, true};
     int NW = 4, NB = 2;
     for (int nb = 1; nb <= (c.K >= 384 ? 2 : 1) && !c.work; ++nb) {
         int64_t w = 0;
         for (int k = 0; k < c.n_probs; ++k)
             w += (c.probs[k].m + kGemmRows - 1) / kGemmRows * ((c.probs[k].n + 32 * nb - 1) / (32 * nb));
-        if (w <= c.n_cu) return {4, nb, 0, 4};
+        if (w <= c.n_cu) return {kDirectWaves, nb, 0, true};
     }
     static constexpr int kSplitAhead[] = {8, 6, 5, 4, 3, 2}, kInKernel[] = {5, 4, 3, 2, 1};
     double best = 1e300;
@@ -134,7 +134,7 @@ static RowsShape rows_shape(const RowsCtx& c) {
             w8 += (c.probs[k].m + kGemmRows * 8 - 1) / (kGemmRows * 8) * ((c.probs[k].n + 32 * NB - 1) / (32 * NB));
         if (w8 >= 2 * c.n_cu) NW = 8;
     }
-    return {NW, NB, c.n_widest > 32 * NB, 0};
+    return {NW, NB, c.n_widest > 32 * NB, false};
 }
 
 // Workspace: the limbs of every problem, 3 KB per 16 k x 32 columns, for an even number of 16-k steps. A
@@ -219,13 +219,13 @@ extern "C" int face_rows_linear_ws(const face_lin_problem* probs, int32_t n_prob
         hipLaunchKernelGGL(split_weights_kernel, dim3((unsigned)blocks), dim3(kWave), 0, c.st, A, c.work);
         FACE_LAUNCH_CHECK();
     }
-    // FACE_GEMM_SHAPE="nw,n_sl,xcd" forces one launch shape (nw < 0: the direct kernel, KW = -nw), for tests that compare every shape's
-    // results (split ahead where there is such a kernel); FACE_ERR_UNSUPPORTED if there is none
+    // FACE_GEMM_SHAPE="nw,n_sl,xcd" forces one launch shape (nw = -4: the direct kernel), for tests that compare every
+    // shape's results (split ahead where there is such a kernel); FACE_ERR_UNSUPPORTED if there is none
     if (const char* fs = getenv("FACE_GEMM_SHAPE")) {
         int nw = 0, ns = 0, xcd = 0;
         if (sscanf(fs, "%d,%d,%d", &nw, &ns, &xcd) == 3 && ns > 0) {
             const int nb = ((n_widest + ns - 1) / ns + 31) / 32;
-            const RowsShape S = nw < 0 ? RowsShape{4, nb, 0, -nw} : RowsShape{nw, nb, xcd ? 1 : 0, 0};
+            const RowsShape S{nw < 0 ? kDirectWaves : nw, nb, xcd ? 1 : 0, nw < 0};
             const int rc = launch_rows(c, S);
             if (rc != FACE_ERR_UNSUPPORTED || !c.work) return rc;
             c.work = nullptr;                    // no such kernel for weights split ahead

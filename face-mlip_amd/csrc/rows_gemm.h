@@ -495,18 +495,19 @@ __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(
 
 // Small launches: no staging. Each wave loads its columns' weights straight into its B operands (lane
 // j + 32 h: 8 consecutive k of column j), splits them itself and runs D steps of 16 k ahead, without LDS
-// or barriers in the loop; KW of the four waves of a workgroup share a 32-row tile, each a contiguous
+// or barriers in the loop; the four waves of a workgroup share a 32-row tile, each a contiguous
 // part of K, and add their sums through LDS in wave order. What bounds these launches is the chain of a
 // wave -- split, products that wait for each other, 0.4 us per 16 k with one wave per SIMD -- times the
 // length of K, not the products or the memory: a quarter of K per wave takes 21 rows of 864 -> 192 from 22 us
 // (staged) to 9.1, and 1,344 rows from 22 to 11.5.
-template <int NB, int KW, int XM>
-__global__ __launch_bounds__(4 * kWave, 2) void rows_gemm_direct_kernel(GemmArgs A) {
+constexpr int kDirectWaves = 4;
+template <int NB, int XM>
+__global__ __launch_bounds__(kDirectWaves * kWave, 2) void rows_gemm_direct_kernel(GemmArgs A) {
     constexpr bool XS = XM == 1, XO = XM >= 2, XF = XM == 3;
-    constexpr int NSB = 32 * NB, RT = 4 / KW, D = NB >= 3 ? 2 : 3, NR = 16 / KW;
-    __shared__ float ssum[KW > 1 ? KW * NB * 16 * kWave : 1];
+    constexpr int NSB = 32 * NB, D = 3, KW = kDirectWaves, NR = 16 / KW;
+    __shared__ float ssum[KW * NB * 16 * kWave];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), j = lane & 31, hf = lane >> 5;
-    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave), kp = wv % KW, it = blockIdx.x;
+    const int kp = __builtin_amdgcn_readfirstlane(tid / kWave), it = blockIdx.x;
     int pi = 0;
 #pragma unroll 1
     for (int k = 1; k < A.n_probs; ++k)
@@ -515,7 +516,7 @@ __global__ __launch_bounds__(4 * kWave, 2) void rows_gemm_direct_kernel(GemmArgs
     const int slices = P.slices, local = it - (int)P.first_block, tile = local / slices;
     const int K = P.k, N = P.n, k1 = P.k1, x_op = XF ? P.x_op : 0, nk = K >> 4;
     const int n0 = (local - tile * slices) * NSB, ns = min(NSB, N - n0);
-    const int64_t M = P.m, m0 = ((int64_t)tile * RT + wv / KW) * kGemmRows;
+    const int64_t M = P.m, m0 = (int64_t)tile * kGemmRows;
     const int64_t row = min(m0 + j, M - 1);
     const float *xr = P.x + row * P.ld_x + 8 * hf, *x2r = P.x2 + row * P.ld_x2 + 8 * hf;
     const float* xzr = P.xz + row * P.ld_xz + 8 * hf;
@@ -618,31 +619,24 @@ __global__ __launch_bounds__(4 * kWave, 2) void rows_gemm_direct_kernel(GemmArgs
         }
     }
     // the NR accumulator registers this wave finishes, of rows out_row(NR kp + i)
-    const int rb = NR * (KW > 1 ? kp : 0);
+    const int rb = NR * kp;
     float v[NB][NR];
-    if (KW > 1) {
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
+    for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) ssum[((kp * NB + nb) * 16 + r) * kWave + lane] = acc[nb][r];
-        __syncthreads();
+        for (int r = 0; r < 16; ++r) ssum[((kp * NB + nb) * 16 + r) * kWave + lane] = acc[nb][r];
+    __syncthreads();
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
+    for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-            for (int i = 0; i < NR; ++i) {
-                v[nb][i] = ssum[(nb * 16 + rb + i) * kWave + lane];
+        for (int i = 0; i < NR; ++i) {
+            v[nb][i] = ssum[(nb * 16 + rb + i) * kWave + lane];
 #pragma unroll
-                for (int k = 1; k < KW; ++k) {
-                    const float p = ssum[((k * NB + nb) * 16 + rb + i) * kWave + lane];
-                    v[nb][i] += k == 1 || k == 2 ? -p : p;
-                }
+            for (int k = 1; k < KW; ++k) {
+                const float p = ssum[((k * NB + nb) * 16 + rb + i) * kWave + lane];
+                v[nb][i] += k == 1 || k == 2 ? -p : p;
             }
-    } else {
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-            for (int i = 0; i < NR; ++i) v[nb][i] = acc[nb][i];
-    }
+        }
     if (XO && beta != 0.f) {                                  // after the products, as in the staged kernel
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
@@ -720,10 +714,10 @@ __global__ __launch_bounds__(kWave) inline void split_weights_kernel(GemmArgs A,
     d[128] = w.l;
 }
 
-// Launch shape: NB column blocks of 32 per wave; NW waves of the staged kernel (KW = 0) or KW waves per
-// row tile of the direct one.
+// Launch shape: NB column blocks of 32 per wave, NW waves per workgroup; direct: the direct kernel (four waves).
 struct RowsShape {
-    int NW, NB, xcd, KW;
+    int NW, NB, xcd;
+    bool direct;
 };
 
 // Everything a launch needs but its shape.
@@ -740,11 +734,11 @@ struct RowsCtx {
 // One launch of a shape; FACE_ERR_UNSUPPORTED, before anything is launched, if there is no such kernel.
 template <int XM>
 static int launch_rows_xm(const RowsCtx& c, RowsShape S) {
-    if (S.NB < 1 || S.NB > 16 || (S.KW && c.work) || (!S.KW && c.far)) return FACE_ERR_UNSUPPORTED;
+    if (S.NB < 1 || S.NB > 16 || (S.direct && c.work) || (!S.direct && c.far)) return FACE_ERR_UNSUPPORTED;
     GemmArgs A = c.A;
     A.xcd_order = S.xcd;
     A.work = c.work;
-    const int waves = S.KW ? 4 : S.NW, rows = kGemmRows * (S.KW ? 4 / S.KW : S.NW);
+    const int waves = S.direct ? kDirectWaves : S.NW, rows = S.direct ? kGemmRows : kGemmRows * S.NW;
     int64_t blocks = 0;
     for (int i = 0; i < c.n_probs; ++i) {
         const face_lin_problem& s = c.probs[i];
@@ -756,7 +750,7 @@ static int launch_rows_xm(const RowsCtx& c, RowsShape S) {
     if (blocks == 0) return 0;
     if (blocks > INT32_MAX) return FACE_ERR_UNSUPPORTED;
     size_t lds = 0;
-    if (!S.KW) {
+    if (!S.direct) {
         const int64_t side = (c.y_scale ? (int64_t)c.n_groups * 32 * S.NB : 0) + (c.x_scale ? (int64_t)c.n_groups * c.K : 0);
         A.side_lds = gemm_lds(S.NB, S.NW, side) <= (size_t)c.max_lds;
         lds = gemm_lds(S.NB, S.NW, A.side_lds ? side : 0);
@@ -769,12 +763,9 @@ static int launch_rows_xm(const RowsCtx& c, RowsShape S) {
         FACE_LAUNCH_CHECK();
         return 0;
     };
-    if (S.KW) {
-        switch (S.KW * 16 + S.NB) {
-            case 65: return go(rows_gemm_direct_kernel<1, 4, XM>);
-            case 66: return go(rows_gemm_direct_kernel<2, 4, XM>);
-            default: return FACE_ERR_UNSUPPORTED;
-        }
+    if (S.direct) {
+        if (S.NB > 2) return FACE_ERR_UNSUPPORTED;
+        return S.NB == 1 ? go(rows_gemm_direct_kernel<1, XM>) : go(rows_gemm_direct_kernel<2, XM>);
     }
     const int NW = S.NW;
     if (c.work) {
