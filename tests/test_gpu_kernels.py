@@ -91,18 +91,15 @@ def _pad(x_edge, counts, M):
     return out * valid.reshape(N, M, *([1] * (x_edge.dim() - 1))).to(x_edge.dtype)
 
 
-@pytest.mark.parametrize("nx,gathered,B,K,lds", [(20, False, 16, 32, None), (20, True, 16, 32, None),
-                                                 (4, True, 16, 144, None), (20, False, 8, 16, None),
-                                                 (4, True, 8, 36, None), (20, False, 16, 64, "1"),
-                                                 (20, True, 16, 32, "1"), (20, False, 16, 48, "1")])
-def test_csr_density_ragged_rows(nx, gathered, B, K, lds, monkeypatch):
-    """Factor density forward / backward on ragged CSR rows (a 70-edge hub row, isolated atoms)
-    against the oracle; lds = "1" forces the backward that stages each atom's G in LDS (the route
-    of large systems)."""
+@pytest.mark.parametrize("nx,gathered,B,K", [(20, False, 16, 32), (20, True, 16, 32), (4, True, 16, 144), (20, False, 8, 16),
+                                             (4, True, 8, 36), (20, False, 16, 64), (20, False, 16, 48),
+                                             (20, True, 16, 80)])
+def test_csr_density_ragged_rows(nx, gathered, B, K):
+    """Factor density forward / backward on ragged CSR rows (a 53-edge hub row, isolated atoms)
+    against the oracle: the split-product kernels (20 monomials, B = 16, K up to 64) and the general
+    ones (other B, K and the 4-monomial set)."""
     from face_amd import ops
-    if lds is not None:
-        monkeypatch.setenv("FACE_DENSITY_BWD_LDS", lds)
-    say("csr density", nx, gathered, B, K, lds)
+    say("csr density", nx, gathered, B, K)
     g = _G(57, 500, 2)
     counts = g.counts
     E = sum(counts)
@@ -930,19 +927,18 @@ def _lin_ref(x, w, w_kn, y0, beta, bias, xs, ys, grp, period, s_off):
     return y
 
 
-@pytest.mark.parametrize("case,kc", [("single", None), ("ranks_proj", None), ("ranks_scaled", None),
-                                     ("kn_xscale", None), ("k512", None), ("empty", None), ("k1024", None),
-                                     ("ranks_proj", "1"), ("ranks_scaled", "1"), ("kn_xscale", "1"),
-                                     ("k512", "1"), ("empty", "1")])
-def test_rows_linear_matches_torch(case, kc, monkeypatch):
+@pytest.mark.parametrize("case,shape", [("single", None), ("ranks_proj", None), ("ranks_scaled", None),
+                                        ("kn_xscale", None), ("k512", None), ("empty", None), ("k1024", None),
+                                        ("single", "-4"), ("ranks_proj", "-4"), ("ranks_scaled", "-4"), ("kn_xscale", "-4"),
+                                        ("k512", "8"), ("empty", "8")])
+def test_rows_linear_matches_torch(case, shape, monkeypatch):
     """y = (beta y + (x * xs) w^T + bias) * ys over up to four problems per launch (mix / tmix /
     proj with the elem_scale factor and their input gradients) vs torch fp64: ragged row counts,
     weight column slices (ld_w > k), (k, n) weights, K = 512 and 1024, sliced outputs (n = 480), an
-    empty problem beside full ones. kc = "1" forces the K-chunked kernel (the route of long K)."""
+    empty problem beside full ones. shape forces the kernel the size would not choose: "-4" the direct
+    one, "8" the staged one in workgroups of eight waves."""
     from face_amd import ops
-    if kc is not None:
-        monkeypatch.setenv("FACE_ROWS_GEMM_KC", kc)
-    say("rows_linear", case, kc)
+    say("rows_linear", case, shape)
     torch.manual_seed(len(case))
     N, C = 1000, 160
     grp = torch.randint(0, 3, (N,), device=DEV, dtype=torch.int32)
@@ -986,20 +982,21 @@ def test_rows_linear_matches_torch(case, kc, monkeypatch):
                  (torch.randn(77, C, device=DEV), torch.randn(C, C, device=DEV), torch.empty(77, C, device=DEV), 0, 0.0)]
     for (x, w, y, s, b) in probs:
         refs.append(_lin_ref(x, w, w_kn, y, b, bias, xs, ys, grp if (xs is not None or ys is not None) else None, N, s))
+    if shape is not None:
+        monkeypatch.setenv("FACE_GEMM_SHAPE", f"{shape},{-(-max(p[2].shape[1] for p in probs) // 32)},0")
     ops.rows_linear(probs, w_kn=w_kn, bias=bias, xs=xs, ys=ys, group=grp, period=N)
     errs = [rel(p[2], r) if r.numel() else 0.0 for p, r in zip(probs, refs)]
     say("   errs", errs)
     assert max(errs) < 1e-5, errs
 
 
-def test_rows_linear_launch_shapes_give_bitwise_equal_rows(monkeypatch):
-    """face_rows_linear times launch shapes (waves per workgroup, column slices) on the first call of
-    a problem signature and keeps the fastest. Every shape must give the same bits: the 864-atom
-    factor mix backward (17,280 rows of 96 -> 512 columns, (k, n) weight, input scale; the shape
-    the timing changes there) against its first 2,000 rows as a separate call (another signature,
-    timed again) and against 17,279 rows with the timing off (the rules' shape), plus torch fp64."""
+def test_rows_linear_rows_do_not_depend_on_their_number():
+    """Launches past one workgroup per CU take the staged kernel, whose sums are the same sequence for any
+    number of rows, whatever launch shape the size chooses: the 864-atom factor mix backward (17,280
+    rows of 96 -> 512 columns, (k, n) weight, input scale) against its first 2,000 rows and against 17,279 of
+    them, plus torch fp64."""
     from face_amd import ops
-    say("rows_linear launch shapes")
+    say("rows_linear number of rows")
     torch.manual_seed(11)
     N, C, BK = 864, 96, 512
     tab = torch.rand(1, 4 * C, device=DEV) + 0.5
@@ -1014,37 +1011,27 @@ def test_rows_linear_launch_shapes_give_bitwise_equal_rows(monkeypatch):
         torch.cuda.synchronize()
         return ys
 
-    full = run(10 * N)                                   # timed shapes
-    part = run(2000)                                     # another signature, timed separately
-    monkeypatch.setenv("FACE_GEMM_TUNE", "0")
-    rule = run(10 * N - 1)                               # the rules' shape
+    full, part, most = run(10 * N), run(2000), run(10 * N - 1)
     for l, (x, w) in enumerate(zip(xs, ws)):
         ref = (x.double() * tab.double()[0, l * C:(l + 1) * C]) @ w.double()
         assert (full[l].double() - ref).abs().max() <= 1e-5 * ref.abs().max()
         assert torch.equal(part[l], full[l][:part[l].shape[0]])
-        assert torch.equal(rule[l], full[l][:rule[l].shape[0]])
+        assert torch.equal(most[l], full[l][:most[l].shape[0]])
 
 
-def _gemm_shapes(n_widest, ns_max=160):
-    """Every (waves per workgroup, column slices) pair face_rows_linear's shape timing tries."""
-    out = []
-    for nw in (16, 8, 4):
-        seen = set()
-        for ns in range(16, ns_max + 1, 16):
-            k = -(-n_widest // ns)
-            if k <= 32 and k not in seen:
-                seen.add(k)
-                out.append((nw, k))
-    return out
+def _gemm_shapes(n_widest):
+    """Every (waves per workgroup, column slices) pair that gives another launch of the staged kernel: slices
+    of 1 to 8 blocks of 32 columns."""
+    return [(nw, ns) for nw in (8, 4) for ns in sorted({-(-n_widest // (32 * nb)) for nb in range(1, 9)})]
 
 
 @pytest.mark.parametrize("case", ["fcc864_mix_bwd", "liquid24k_mix_fwd"])
 def test_rows_linear_every_launch_shape_gives_bitwise_equal_rows(case, monkeypatch):
-    """Every launch shape the timing may pick (4, 8, 16 waves per workgroup x every slice count x
-    plain / XCD-aware item order, forced through FACE_GEMM_SHAPE) gives the same bits as the rules'
-    shape: the 864-atom factor mix backward ((k, n) weight 96 -> 512, input scale: one item per
-    workgroup) and the 24,000-atom CP mix forward (480,000 rows of 160 -> 160 over four ranks,
-    (n, k) weights, output scale: more tiles than resident workgroups, so the persistent runs)."""
+    """Every launch shape of the staged kernel (4 or 8 waves per workgroup, every slice width, plain and
+    XCD-aware item order, forced through FACE_GEMM_SHAPE) gives the same bits as the rules' shape: the
+    864-atom factor mix backward ((k, n) weight 96 -> 512, input scale, split in the kernel) and the
+    24,000-atom CP mix forward (480,000 rows of 160 -> 160 over four ranks, (n, k) weights split ahead where
+    the shape has such a kernel, output scale)."""
     from face_amd import ops
     say("rows_linear every shape", case)
     torch.manual_seed(13)
@@ -1068,7 +1055,6 @@ def test_rows_linear_every_launch_shape_gives_bitwise_equal_rows(case, monkeypat
         torch.cuda.synchronize()
         return ys
 
-    monkeypatch.setenv("FACE_GEMM_TUNE", "0")
     rule = run()
     for l, (x, w) in enumerate(zip(xs, ws)):
         g = grp.long().repeat(x.shape[0] // N)
@@ -1083,7 +1069,7 @@ def test_rows_linear_every_launch_shape_gives_bitwise_equal_rows(case, monkeypat
             monkeypatch.setenv("FACE_GEMM_SHAPE", f"{nw},{n_sl},{xcd}")
             try:
                 out = run()
-            except RuntimeError as err:                  # a shape whose slice does not fit LDS
+            except RuntimeError as err:                  # a slice width without a kernel
                 assert "(code -2)" in str(err), err
                 refused += 1
                 continue
@@ -1091,7 +1077,7 @@ def test_rows_linear_every_launch_shape_gives_bitwise_equal_rows(case, monkeypat
                 assert torch.equal(a, b), (nw, n_sl, xcd)
             ran += 1
     say(f"   {ran} shapes bitwise equal to the rules' shape, {refused} refused")
-    assert ran >= 24
+    assert ran == 16, (ran, refused)
 
 
 def _rows_launch(x, w, y, w_kn, ahead, beta=0.0, xs=None, ys=None, grp=None, s_off=0):
@@ -1194,19 +1180,21 @@ def test_rows_linear_split_ahead_beside_a_problem_of_no_rows(m):
     assert rel(y, ref) < 1e-5 if m else bool((y == 7.0).all())
 
 
-@pytest.mark.parametrize("ahead", [False, True])
+@pytest.mark.parametrize("route", ["direct", "staged", "ahead"])
 @pytest.mark.parametrize("where", ["x", "w"])
-def test_rows_linear_values_past_bf16(where, ahead):
+def test_rows_linear_values_past_bf16(where, route, monkeypatch):
     """Operands that round to a bf16 infinity (3.4e38), infinities and NaN: the results are those of
     plain float32 products, and those of other 32-row tiles keep their bits."""
-    say("rows_linear past bf16", where, ahead)
+    say("rows_linear past bf16", where, route)
+    ahead = route == "ahead"
+    monkeypatch.setenv("FACE_GEMM_SHAPE", "-4,3,0" if route == "direct" else "4,1,0")
     torch.manual_seed(3)
     m, n, k = 200, 96, 64
     x, w = torch.randn(m, k, device=DEV), torch.randn(n, k, device=DEV)
     w[:, 1] = w[:, 1].abs() + 0.5                                    # a definite sign against the infinity
     plain = torch.empty(m, n, device=DEV)
     _rows_launch(x, w, plain, False, ahead)
-    big = x.clone() if where == "x" else w.clone()              # three column blocks: the direct kernel
+    big = x.clone() if where == "x" else w.clone()
     big[5, 0], big[70, 1], big[70, 2], big[80, 3] = 3.4e38, float("inf"), 1e30, float("nan")
     small = w if where == "x" else x
     small[:, 0] = small[:, 0].clamp(-0.5, 0.5)                       # 3.4e38 * 0.5 stays finite
@@ -1396,18 +1384,18 @@ def test_rows_linear_scale_tables_larger_than_lds(side):
     assert rel(y, ref) < 1e-5
 
 
-@pytest.mark.parametrize("kc", [None, "1"])
+@pytest.mark.parametrize("shape", [None, "-4,2,0", "8,1,1"])
 @pytest.mark.parametrize("w_kn", [False, True])
-def test_rows_linear_split_input_transforms_and_initial_sum(w_kn, kc, monkeypatch):
+def test_rows_linear_split_input_transforms_and_initial_sum(w_kn, shape, monkeypatch):
     """The readout forms of face_rows_linear vs torch fp64: input columns from two tensors
     ([x | x2], the split at k1), silu(x) and x * silu'(xz) applied to the x columns as they load,
     a bias per problem, and the sum started at beta * y0 over the first n_y0 columns of another
     tensor (a residual); four problems of different K in one launch, ragged rows, strided views.
-    kc = "1" forces the K-chunked kernel."""
+    shape forces the direct kernel and the staged one in workgroups of eight waves."""
     from face_amd import ops
-    if kc is not None:
-        monkeypatch.setenv("FACE_ROWS_GEMM_KC", kc)
-    say("rows_linear split/ops", w_kn, kc)
+    if shape is not None:
+        monkeypatch.setenv("FACE_GEMM_SHAPE", shape)
+    say("rows_linear split/ops", w_kn, shape)
     torch.manual_seed(7)
     m = 1203
     silu = lambda t: t * torch.sigmoid(t)
