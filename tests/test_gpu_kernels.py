@@ -332,6 +332,70 @@ def test_cp_radial_fused_forward_contains_non_finite_edges(C, H, gathered, what)
     assert torch.equal(out[0, hit], clean[0, hit]) if what[0] == "Y" else torch.isnan(out[0, hit]).all()
 
 
+@pytest.mark.parametrize("where", ["x", "w"])
+@pytest.mark.parametrize("C,H,gathered", [(160, 64, True), (48, 16, False), (16, 48, True)])
+def test_edge_products_of_values_past_bf16(C, H, gathered, where):
+    """Inputs or weights between the largest bf16 and the largest float32, and an infinity, take the plain float32
+    products of the CP pooling forward and of the per-edge linear: last tiles of 21 edges, 16-channel tails, rows of
+    several tiles. Bounds: one rounding (2^-24 of the sum of magnitudes) per term of the dot product and, for A, per
+    edge of the row, plus four for the factors of a term."""
+    from face_amd import _lib
+    say("edge products past bf16", C, H, gathered, where)
+    N = 300
+    counts = _ragged_counts(N, C + H)
+    counts[60] += (21 - sum(counts)) % 32
+    E, rec = int(sum(counts)), np.repeat(np.arange(N), counts)
+    assert E % 32 == 21
+    row_ptr = torch.as_tensor(np.concatenate([[0], np.cumsum(counts)]).astype(np.int32), device=DEV)
+    col = torch.as_tensor(np.random.default_rng(C).integers(0, N, E).astype(np.int32), device=DEV)
+    torch.manual_seed(C + H)
+    h2, W, b = torch.randn(E, H, device=DEV), torch.randn(4 * C, H, device=DEV) / H ** 0.5, torch.randn(4 * C, device=DEV)
+    env, Y = torch.rand(E, device=DEV), 2 * torch.rand(E, 20, device=DEV) - 1
+    msg = 2 * torch.rand(N if gathered else E, C, device=DEV) - 1
+    tab = torch.randn(N, 4 * C, device=DEV)
+    big, inf = 3.395e38, E // 2
+    if where == "x":
+        W[:, 1] = W[:, 1].clamp(-0.25, 0.25)
+        W[:, 2] = W[:, 2].abs() + 0.1                                 # a definite sign against the infinity
+        h2[[0, 33, E - 1], 1] = big
+        h2[inf, 2] = float("inf")
+    else:
+        h2[:, 1] = 0.002 * h2[:, 1].clamp(-1, 1)                      # sums over a row of edges stay finite
+        W[[0, 2 * C + 17 % C, 4 * C - 1], 1] = big
+    P, st = _lib.ptr, _lib.stream_of(h2)
+    outs = [torch.full((k, N, C), float("nan"), device=DEV) for k in (1, 3, 6, 10)]
+    R, L = torch.full((E, 4 * C), 7.0, device=DEV), torch.full((E, 4 * C), 7.0, device=DEV)
+    _lib.call("face_cp_radial_fwd", P(h2), H, H, P(W), P(b), P(env), P(msg), C, P(col) if gathered else None, P(Y), 20,
+              P(row_ptr), N, E, C, *_lib.ranks_of_blocks(outs), P(R), 4 * C, st)
+    _lib.call("face_edge_linear_fwd", P(h2), H, E, H, P(W), P(b), 4 * C, P(tab), 4 * C, P(col), P(L), 4 * C, st)
+    torch.cuda.synchronize()
+    edges = torch.ones(E, dtype=torch.bool, device=DEV)
+    if where == "x":
+        edges[inf] = False
+        assert bool((R[inf] == float("inf")).all()) and bool((L[inf] == float("inf")).all())
+    u = 2.0 ** -24
+    ref = h2.double() @ W.double().t().contiguous() + b.double()
+    mag = h2.double().abs() @ W.double().abs().t().contiguous() + b.double().abs()
+    assert bool(((R.double() - ref).abs() <= (H + 1) * u * mag)[edges].all())
+    t = tab.double()[col.long()]
+    assert bool(((L.double() - ref - t).abs() <= (H + 2) * u * (mag + t.abs()))[edges].all())
+    atoms = torch.ones(N, dtype=torch.bool, device=DEV)
+    if where == "x":
+        atoms[int(rec[inf])] = False
+        assert not bool(torch.isfinite(outs[0][0, int(rec[inf])]).any())
+        ref[inf], mag[inf] = 0.0, 0.0
+    m = (msg[col.long()] if gathered else msg).double() * env.double()[:, None]
+    at = torch.as_tensor(rec, device=DEV)
+    x0 = 0
+    for l, k in enumerate((1, 3, 6, 10)):
+        for x in range(k):
+            y = Y[:, x0 + x].double()[:, None]
+            want = torch.zeros(N, C, dtype=torch.float64, device=DEV).index_add_(0, at, y * m * ref[:, l * C:(l + 1) * C])
+            size = torch.zeros_like(want).index_add_(0, at, (y * m).abs() * mag[:, l * C:(l + 1) * C])
+            assert bool(((outs[l][x].double() - want).abs() <= (H + max(counts) + 4) * u * size)[atoms].all()), (l, x)
+        x0 += k
+
+
 # ----------------------------------------------------------------------------- gated outputs
 @pytest.mark.parametrize("N,C", [(1000, 160), (37, 96), (1, 4)])
 def test_eq_gate_matches_torch(N, C):
