@@ -66,14 +66,15 @@ __device__ __forceinline__ v4f mfma_16x16x4(float a, float b, v4f c) {
 }
 
 // fp32 products on the bf16 matrix cores. x = h + m + l with h = bf16(x), m = bf16(x - h),
-// l = bf16(x - h - m), each rounded to nearest: the three limbs hold 24 bits of x, and
-// x w = xh wh + (xh wm + xm wh) + (xm wm + xh wl + xl wh) up to 2^-25 of |x w| at most, below one fp32
-// rounding. Six v_mfma_f32_32x32x16_bf16 do the work of sixteen 16x16x4 fp32 products of the same
+// l = bf16(x - h - m), each rounded to nearest: the three limbs hold the 24 bits of x, and
+// x w = xh wh + (xh wm + xm wh) + (xm wm + xh wl + xl wh) up to the three products left out, together below
+// 2^-24 of |x w|, half an ulp of fp32 (1.98 2^-25 at x = w = 0x1.00ff8p0; of random pairs one in 700 passes
+// 2^-25). Six v_mfma_f32_32x32x16_bf16 do the work of sixteen 16x16x4 fp32 products of the same
 // shape in 192 cycles instead of 512 (register-only loops: 1300-1580 / 6 = 217-263 against 110-137
 // TFLOP/s), and with fp32 accumulation over fewer, longer dot products their sums are closer to
 // 64 bits (relative error of a K = 160 / 512 / 1024 sum 1.7e-7 / 3.4e-7 / 4.9e-7 against 2.2e-7 /
-// 4.0e-7 / 5.8e-7). Values past the largest bf16 (and infinities)
-// have a NaN limb.
+// 4.0e-7 / 5.8e-7). Both ends of the range: values past the largest bf16 (and infinities) have a NaN limb;
+// below |x| = 2^-110 the low limb ends at bf16's smallest subnormal, and x is held to 2^-134 only.
 // Operand layouts (wave64): A[i][k], k = 8 (lane >> 5) + e in element e of lane i + 32 (k >> 3);
 // B[k][j] likewise by j; D[8 (r >> 2) + 4 (lane >> 5) + (r & 3)][lane & 31] in register r.
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));

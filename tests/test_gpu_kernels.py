@@ -1280,6 +1280,21 @@ def test_rows_linear_values_past_bf16(where, route, monkeypatch):
     assert (out[5].double() - ref[5]).abs().max() <= 1e-6 * ref[5].abs().max()
 
 
+@pytest.mark.parametrize("route", ["direct", "staged"])
+@pytest.mark.parametrize("e", [-100, -109, -112, -120])
+def test_rows_linear_smallest_values(e, route, monkeypatch):
+    """Values near the end of the float32 range (identity weights: the sum of the three limbs): exact down to
+    2^-110, held to 2^-134 below."""
+    monkeypatch.setenv("FACE_GEMM_SHAPE", "-4,1,0" if route == "direct" else "4,1,0")
+    torch.manual_seed(2)
+    x = (1 + torch.rand(64, 32, device=DEV)) * 2.0 ** e
+    y = torch.empty(64, 32, device=DEV)
+    _rows_launch(x, torch.eye(32, device=DEV), y, False, False)
+    err = (y.double() - x.double()).abs().max().item()
+    say("rows_linear smallest values", e, route, err * 2.0 ** 134)
+    assert err <= (0 if e >= -110 else 2.0 ** -134)
+
+
 @pytest.mark.parametrize("last,gate,const_h", [(False, True, False), (False, False, True), (True, False, False),
                                                (True, True, False)])
 @pytest.mark.parametrize("N,C", [(1, 16), (33, 48), (700, 160), (40, 24)])
