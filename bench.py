@@ -215,6 +215,22 @@ def algorithmic_bytes(label, g, kw):
         return algorithmic_bytes("mix_bwd", g, kw) + algorithmic_bytes("tmix_bwd", g, kw)
     if label in ("table_linear_fwd", "table_linear_bwd"):   # (3 + 6) N rows, C <-> 2 K_dir, two weights
         return 4 * (9 * N * (C + 2 * kw["K_dir"]) + 2 * C * 2 * kw["K_dir"])
+    # readout layers, averaged over the P passes like their flops below: the gate row in all passes but the
+    # last, the first pass's h as a precomputed initial sum and without a gradient
+    P = kw.get("n_passes", 2)
+    gate = (P - 1) / P if kw.get("eqmsg") else 0.0
+    if label == "readout_in":           # inv, h (or the initial sum) in; z0, gate row out
+        return 4 * (N * C * (9 + (P - 1) / P + 2 / P + 2 + 2 * gate) + 2 * C * C * (9 + (P - 1) / P + 9 * gate))
+    if label == "readout_hid":
+        return 4 * (4 * N * C + 4 * C * C)
+    if label == "readout_hid_bwd":      # upstream (one row for all in the last pass), z1 in
+        return 4 * (N * C * (6 - 2 / P) + 4 * C * C)
+    if label == "readout_out":          # z1, h in; h_new out
+        return 4 * (4 * N * C + 2 * C * C)
+    if label == "readout_out_bwd":      # upstream rows and their energy column in
+        return 4 * (N * (3 * C + 1) + 2 * C * C)
+    if label == "readout_in_bwd":       # da0, z0, the gate row's gradient, the residual's in; d inv, d h out
+        return 4 * (N * C * (4 + 2 * gate + 9 + (P - 1) / P + max(P - 2, 0) / P) + 2 * C * C * (9 + (P - 1) / P + 9 * gate))
     if label == "ln_fwd":               # row of 9C in and out (+ mean, rstd)
         return 4 * (2 * 9 * C + 2) * N
     if label == "ln_bwd":
@@ -600,9 +616,9 @@ def pmc_probe(k, steps=2, copy_floats=1 << 28):
     sts, kw, el, desc = systems.workload(k)
     g = build_graph(sts, kw["rc"])
     m = model_for(kw, el)
-    # one step first, so that the row GEMM's launch shapes are timed and cached; then a marker
-    # launch (the gather form of the force scatter, which the model does not use) whose dispatch
-    # separates that step's (and the shape timing's) dispatches from the recorded steps'
+    # one step first, which fills the model's caches of constant rows; then a marker launch (the gather
+    # form of the force scatter, which the model does not use) whose dispatch separates that step's
+    # dispatches from the recorded steps'
     m(g.with_pos(g.pos.clone()))["forces"]
     trace_mark()
     # a marker after every library call: the dispatches between two markers are one call's
@@ -711,7 +727,7 @@ def pmc_summary(fetch_dir, write_dir, probe_log, out_path):
                    f"> $OUT/pmc_{C}_w{k}.log\n")
     out.append(f"python bench.py --pmc-summary $OUT/pmc_FETCH_SIZE_w{k} $OUT/pmc_WRITE_SIZE_w{k} "
                f"$OUT/pmc_FETCH_SIZE_w{k}.log {out_path}\n```\n\n")
-    out.append("`bench.py --pmc-probe` runs one eager E+F step (the row GEMM's launch shapes are timed there) "
+    out.append("`bench.py --pmc-probe` runs one eager E+F step (which fills the model's caches of constant rows) "
                "and a marker launch, then 2 recorded eager E+F steps with a marker launch after every library "
                "call, then three device-to-device copies of 1 GiB; only dispatches after the first marker are "
                "counted. Its JSON line lists the library calls of the recorded steps in launch order: the "
@@ -785,9 +801,8 @@ def sq_summary(out_path, title, probe_args, *dirs):
     import collections
     import csv
     import glob
-    # rows keyed by call label for the kernels that serve labels (each pass is its own process, whose
-    # row GEMM may pick other launch shapes, i.e. other kernel instances, for the same call), else by
-    # kernel; each pass's probe JSON line (the .log beside its directory) gives the call order
+    # rows keyed by call label for the kernels that serve labels (a call may launch several kernel instances),
+    # else by kernel; each pass's probe JSON line (the .log beside its directory) gives the call order
     data = collections.defaultdict(lambda: collections.defaultdict(list))
     for d in dirs:
         f = sorted(glob.glob(os.path.join(d, "**", "*counter_collection.csv"), recursive=True))
