@@ -17,7 +17,7 @@ namespace face {
 // kernels in rounding only; R is bitwise the edge_linear_fwd product.
 // R goes out through non-temporal stores (read next by the backward, milliseconds later).
 // Bound by two waves per SIMD (256 registers) and the stores: 24,000 atoms, 1.25 M edges, C = 160, H = 64:
-// 1.36 ms with per-edge messages and 1.26 with table messages (fp32 instructions with the pooling on them:
+// 1.29 ms with per-edge messages and 1.26 with table messages (fp32 instructions with the pooling on them:
 // 1.87, and 1.14 + 0.82 ms for head and pooling), 0.90 without R; in timing-only variants the products
 // and the pooling take 0.34 ms each, the message loads 0.07. What moved it: no spilled address and no branch
 // around an optional operand's load (each wait includes the stores of R in flight). Measured and not

@@ -425,8 +425,8 @@ class ReadoutMLP(torch.autograd.Function):
 
     Widths that are multiples of 16 run on the row-block kernels, SiLU and its derivative applied to
     the rows as they load: z0 and the gate row in one launch, then z1, the residual rows, the energy
-    row; backward in three launches (10,752 atoms, C = 160, forward and backward: 667 us on the
-    library's float32 products with the activations between them, 405 us here). Other widths,
+    row; backward in three launches (10,752 atoms, C = 160, forward and backward: 657 us on the
+    library's float32 products with the activations between them, 416 us here). Other widths,
     weights without 16-byte aligned rows and rows past GEMM_SPAN elements take the library products."""
 
     @staticmethod
@@ -885,7 +885,7 @@ def cp_density(R, env, msg, Y, graph, gathered=False):
 class CPRadialDensity(torch.autograd.Function):
     """CP pooling fed by the CP columns of the last radial layer: R = h2 W_cp^T + b_cp (E, 4C), then
     A_l as in CPDensity (face/model.py:469-472, 496-502). The forward computes R on the matrix cores and
-    pools it in the same launch (R is written once, for the backward, and not read back: 1.36 / 1.26 ms
+    pools it in the same launch (R is written once, for the backward, and not read back: 1.29 / 1.26 ms
     with per-edge / node-table messages at 24,000 atoms, C = 160); for shapes that launch cannot serve, R
     comes from the radial head and is pooled in a second launch (1.96 ms there). The
     backward multiplies the pooling's dR by W_cp on the matrix cores inside the pooling kernel and
@@ -1449,8 +1449,9 @@ def rows_linear(probs, w_kn=False, bias=None, xs=None, ys=None, group=None, peri
          ptr(work), need, _lib.stream_of(ref), label=label)
 
 
-# mix and transport-mix backward in one launch up to this many atoms (launch-bound sizes; at
-# 24,000 atoms the six-problem launch measured 646 us against 238 + 354 us for the two)
+# mix and transport-mix backward in one launch up to this many atoms (launch-bound sizes; mix and projections of
+# C = 160, both directions, two launches against one: 523 and 492 us at 4,096 atoms, 606 and 605 at 6,000, 1157 and
+# 1157 at 12,000, 2232 and 2265 at 24,000)
 MIX_MERGE_MAX_ATOMS = 4096
 
 
