@@ -430,17 +430,29 @@ class ReadoutMLP(torch.autograd.Function):
     weights without 16-byte aligned rows and rows past GEMM_SPAN elements take the library products."""
 
     @staticmethod
+    def takes_rows(inv, h, W0a, W0b, b0, W1, b1, W2, b2, Wg, bg, hb):
+        """Whether the row-block kernels, which take shapes, types and places on trust, serve these operands.
+        All others go to the library products, which broadcast what can be and refuse the rest."""
+        N, n_inv, H1, H2, C = inv.shape[0], W0a.shape[1], W0a.shape[0], W1.shape[0], W0b.shape[1]
+        want = [(inv, (N, n_inv)), (h, (N, C)), (W0b, (H1, C)), (b0, (H1,)), (W1, (H2, H1)), (b1, (H2,)), (W2, (C + 1, H2)),
+                (b2, (C + 1,))]
+        if Wg is not None:
+            want += [(Wg, (Wg.shape[0], n_inv)), (bg, (Wg.shape[0],))]
+        if hb is not None:
+            want.append((hb, (N, H1)))
+        if any(t is None or t.shape != sh or t.dtype != torch.float32 or t.device != inv.device for t, sh in want):
+            return False
+        widths = [C, H1, H2, n_inv] + ([] if Wg is None else [Wg.shape[0]])
+        return (0 < N * max(widths) < GEMM_SPAN and all(v % 16 == 0 for v in widths)
+                and _rows16(W0a, W0b, b0, W1, b1, W2, Wg, bg))
+
+    @staticmethod
     def forward(ctx, inv, h, W0a, W0b, b0, W1, b1, W2, b2, Wg, bg, last, hb):
         ctx.last = last
         ctx.w = (W0a, W0b, W1, W2, Wg)
         C, H1, H2 = W0b.shape[1], W0a.shape[0], W1.shape[0]
         N, dev = inv.shape[0], inv.device
-        widest = max(C, H1, H2, W0a.shape[1], 0 if Wg is None else Wg.shape[0])
-        ctx.rows = (0 < N * widest < GEMM_SPAN and all(v % 16 == 0 for v in (C, H1, H2, W0a.shape[1])) and W2.shape[0] == C + 1
-                    and (Wg is None or (Wg.shape[0] % 16 == 0 and bg is not None))
-                    and all(b is not None for b in (b0, b1, b2))
-                    and _rows16(W0a, W0b, b0, W1, b1, W2, Wg, bg) and inv.dtype == torch.float32
-                    and h.dtype == torch.float32 and inv.is_cuda)
+        ctx.rows = ReadoutMLP.takes_rows(inv, h, W0a, W0b, b0, W1, b1, W2, b2, Wg, bg, hb)
         if ctx.rows:
             inv_, h_ = _gemm_rows(inv), _gemm_rows(h)
             z0 = torch.empty(N, H1, device=dev)

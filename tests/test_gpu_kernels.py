@@ -1446,6 +1446,34 @@ def test_readout_mlp_takes_broadcast_rows(N):
     assert all(torch.equal(a, b) for a, b in zip(got, want))
 
 
+def test_readout_mlp_refuses_or_broadcasts_other_shapes():
+    """Operands whose shape, type or place is not the row-block kernels': refused where the library products
+    refuse them (a row of other width, a weight of other shape, another type, host memory), and broadcast where
+    these broadcast (a bias of one value, one row for all atoms)."""
+    from face_amd import ops
+    say("readout_mlp shapes")
+    C, N = 32, 70
+    inv, h, ws = _readout_case(N, C)
+    hb = torch.randn(1, 2 * C, device=DEV)
+    swap = lambda k, t: ws[:k] + [t] + ws[k + 1:]
+    refused = [(inv[:, :8 * C], h, ws, None), (torch.randn(N, 10 * C, device=DEV), h, ws, None), (inv, h[:, :16], ws, None),
+               (inv, h[:64], ws, None), (inv, h.cpu(), ws, None), (inv, h.double(), ws, None),
+               (inv, h, ws, hb.expand(N, -1).double()), (inv, h, ws, hb.expand(N, -1).cpu())]
+    refused += [(inv, h, swap(k, ws[k][..., :16]), None) for k in (1, 2, 3, 4, 5, 6, 7, 8)]        # of the weights and biases
+    refused += [(inv, h, swap(k, ws[k].cpu()), None) for k in range(9)]
+    for i, (x, y, w, b) in enumerate(refused):
+        assert not ops.ReadoutMLP.takes_rows(x, y, *w, b), i
+        with pytest.raises(RuntimeError):
+            ops.readout_mlp(x, y, *w, False, b)
+    assert ops.ReadoutMLP.takes_rows(inv, h, *ws, None)
+    for k in (2, 4, 8):                                                # b0, b1, bg of one value
+        one = torch.full((1,), 0.3, device=DEV)
+        got, want = ops.readout_mlp(inv, h, *swap(k, one), False), ops.readout_mlp(inv, h, *swap(k, one.repeat(2 * C)), False)
+        assert all(rel(a, b) < 5e-6 for a, b in zip(got, want))
+    got, want = ops.readout_mlp(inv, h, *ws, False, hb), ops.readout_mlp(inv, h, *ws, False, hb.repeat(N, 1))
+    assert all(rel(a, b) < 5e-6 for a, b in zip(got, want))
+
+
 @pytest.mark.parametrize("side", ["xs", "ys"])
 def test_rows_linear_scale_tables_larger_than_lds(side):
     """64 groups whose scale rows do not fit in LDS beside the weights: read from memory instead, the
