@@ -1481,13 +1481,17 @@ class ScaledMix(torch.autograd.Function):
         dev = Af[0].device
         outs = [torch.empty(a.shape[0], N, C, device=dev) for a in Af]
         # the transport sums are further input columns of ranks 1 and 2, with their own weights: their
-        # products are neither written first nor read back
+        # products are neither written first nor read back (operands that are not exactly what the kernels take:
+        # written first, by the library, which refuses the wrong ones)
         Ds = {1: D1, 2: D2}
         probs = []
         for l, a in enumerate(Af):
             x, y, D = a.reshape(-1, a.shape[-1]), outs[l].view(-1, C), Ds.get(l)
             D = None if D is None else D.reshape(-1, D.shape[-1])
-            if D is not None and not (D.shape[1] % 16 == 0 and _rows16(D, wt[l - 1])):
+            if D is not None and wt[l - 1].shape[0] != C:
+                raise RuntimeError(f"scaled_mix: transport weight of {wt[l - 1].shape[0]} rows for {C} channels")
+            if D is not None and not (D.shape[1] % 16 == 0 and wt[l - 1].shape[1] == D.shape[1]
+                                      and D.device == wt[l - 1].device == x.device and _rows16(D, wt[l - 1])):
                 torch.mm(D, wt[l - 1].t(), out=y)
                 probs.append(lin(x, wm[l], y, l * C, 1.0))
             else:

@@ -1624,6 +1624,23 @@ def test_scaled_mix_forward_backward(transport, Cin, merge, monkeypatch):
     assert max(errs) < 1e-5, errs
 
 
+@pytest.mark.parametrize("wrong", ["width", "weight", "weight_rows", "host", "host_weight", "type"])
+def test_scaled_mix_refuses_other_transport_operands(wrong):
+    """Transport sums or weights that do not fit the mix (width, shape, host memory, type) are refused."""
+    from face_amd import ops
+    say("scaled mix wrong transport operands", wrong)
+    N, C, Dw = 40, 32, 64
+    grp = torch.zeros(N, device=DEV, dtype=torch.int32)
+    s_tab = torch.rand(1, 4 * C, device=DEV)
+    Af = [torch.randn(k, N, C, device=DEV) for k in (1, 3, 6, 10)]
+    wm = [torch.randn(C, C, device=DEV) for _ in range(4)]
+    D, w = torch.randn(3, N, Dw, device=DEV), torch.randn(C, Dw, device=DEV)
+    D = {"width": D[..., :48], "host": D.cpu(), "type": D.double()}.get(wrong, D)
+    w = {"weight": w[:, :32], "weight_rows": w[:16], "host_weight": w.cpu()}.get(wrong, w)
+    with pytest.raises(RuntimeError):
+        ops.scaled_mix(s_tab, grp, wm, [w, None], D, None, Af)
+
+
 @pytest.mark.parametrize("last", [False, True])
 def test_readout_mlp_refuses_a_second_derivative(last):
     """The input gradients have no derivative of their own: asked for with create_graph they are refused when
