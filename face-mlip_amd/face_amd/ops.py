@@ -440,7 +440,10 @@ class ReadoutMLP(torch.autograd.Function):
             want += [(Wg, (Wg.shape[0], n_inv)), (bg, (Wg.shape[0],))]
         if hb is not None:
             want.append((hb, (N, H1)))
-        if any(t is None or t.shape != sh or t.dtype != torch.float32 or t.device != inv.device for t, sh in want):
+        dev = inv.get_device()
+        if any(t is None or t.shape != sh or t.get_device() != dev for t, sh in want):
+            return False
+        if any(t is not None and t.dtype != torch.float32 for t in (inv, h, hb)):
             return False
         widths = [C, H1, H2, n_inv] + ([] if Wg is None else [Wg.shape[0]])
         return (0 < N * max(widths) < GEMM_SPAN and all(v % 16 == 0 for v in widths)
