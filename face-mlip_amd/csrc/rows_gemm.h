@@ -422,16 +422,27 @@ __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(
         }
     }
     // Operands that round to a bf16 infinity have a NaN limb, which every product they enter carries into
-    // the sums: a wave with a sum that is not finite forms its rows again in plain fp32 products.
+    // the sums: a row with a sum that is not finite is formed again in plain fp32 products (and not stored
+    // below); the others of the wave keep theirs.
     float chk = 0.f;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) chk = fmaf(acc[nb][r], 0.f, chk);
+    uint32_t redo = 0;                                        // rows of the tile, uniform
     if (__any(chk != chk)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            float c = 0.f;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) c = fmaf(acc[nb][r], 0.f, c);
+            const uint64_t b = __ballot(c != c);
+            const int row = 8 * (r >> 2) + (r & 3);
+            redo |= ((uint32_t)b ? 1u : 0u) << row | ((b >> 32) ? 1u : 0u) << (row + 4);
+        }
 #pragma unroll 1
-        for (int i = 0; i < kGemmRows; ++i) plain_row<XM>(A, P, m0 + i, n0, ns, lane);
-        return;
+        for (int i = 0; i < kGemmRows; ++i)
+            if (redo >> i & 1) plain_row<XM>(A, P, m0 + i, n0, ns, lane);
     }
     // epilogue: initial sum, bias and y scale, then stores of 128 bytes per row
     if (XO && beta != 0.f) {
@@ -482,13 +493,14 @@ __global__ __launch_bounds__(NW * kWave, NB <= 2 ? 3 : 2) void rows_gemm_kernel(
     }
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-        if (full && 32 * nb + 32 <= ns) {                     // uniform
+        if (full && !redo && 32 * nb + 32 <= ns) {            // uniform
 #pragma unroll
             for (int r = 0; r < 16; ++r) *at_off(yb + (8 * (r >> 2) + (r & 3)) * ld_y + 32 * nb, yo) = acc[nb][r];
         } else {
 #pragma unroll
             for (int r = 0; r < 16; ++r)
-                if (32 * nb + j < ns && row_ok(r)) *at_off(yb + (8 * (r >> 2) + (r & 3)) * ld_y + 32 * nb, yo) = acc[nb][r];
+                if (32 * nb + j < ns && row_ok(r) && !(redo >> (8 * (r >> 2) + (r & 3) + 4 * hf) & 1))
+                    *at_off(yb + (8 * (r >> 2) + (r & 3)) * ld_y + 32 * nb, yo) = acc[nb][r];
         }
     }
 }
@@ -649,16 +661,20 @@ __global__ __launch_bounds__(kDirectWaves * kWave, 2) void rows_gemm_direct_kern
             }
         }
     }
-    float chk = 0.f;
+    uint32_t redo = 0;                                        // rows formed again, as in the staged kernel: bits i, i + 16
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
+    for (int i = 0; i < NR; ++i) {
+        float c = 0.f;
 #pragma unroll
-        for (int i = 0; i < NR; ++i) chk = fmaf(v[nb][i], 0.f, chk);
-    if (__any(chk != chk)) {
+        for (int nb = 0; nb < NB; ++nb) c = fmaf(v[nb][i], 0.f, c);
+        const uint64_t b = __ballot(c != c);
+        redo |= ((uint32_t)b ? 1u : 0u) << i | ((b >> 32) ? 1u : 0u) << (i + 16);
+    }
+    if (redo) {
 #pragma unroll 1
         for (int i = 0; i < 2 * NR; ++i)
-            plain_row<XM>(A, P, m0 + 8 * ((rb + (i >> 1)) >> 2) + ((rb + (i >> 1)) & 3) + 4 * (i & 1), n0, ns, lane);
-        return;
+            if (redo >> ((i >> 1) + 16 * (i & 1)) & 1)
+                plain_row<XM>(A, P, m0 + 8 * ((rb + (i >> 1)) >> 2) + ((rb + (i >> 1)) & 3) + 4 * (i & 1), n0, ns, lane);
     }
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
@@ -672,7 +688,7 @@ __global__ __launch_bounds__(kDirectWaves * kWave, 2) void rows_gemm_direct_kern
             if (XF && P.sum_row) o *= sr;
             if (P.bias) o = fmaf(f, P.bias[n0 + c], o);
             if (A.ys) o *= t[c];
-            if (32 * nb + j < ns && r < M) P.y[r * ld_y + n0 + c] = o;
+            if (32 * nb + j < ns && r < M && !(redo >> (i + 16 * hf) & 1)) P.y[r * ld_y + n0 + c] = o;
         }
     }
 }

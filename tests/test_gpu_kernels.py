@@ -1248,7 +1248,7 @@ def test_rows_linear_split_ahead_beside_a_problem_of_no_rows(m):
 @pytest.mark.parametrize("where", ["x", "w"])
 def test_rows_linear_values_past_bf16(where, route, monkeypatch):
     """Operands that round to a bf16 infinity (3.4e38), infinities and NaN: the results are those of
-    plain float32 products, and those of other 32-row tiles keep their bits."""
+    plain float32 products, and all other rows, of the same 32-row tile too, keep their bits."""
     say("rows_linear past bf16", where, route)
     ahead = route == "ahead"
     monkeypatch.setenv("FACE_GEMM_SHAPE", "-4,3,0" if route == "direct" else "4,1,0")
@@ -1273,7 +1273,7 @@ def test_rows_linear_values_past_bf16(where, route, monkeypatch):
     touched = torch.zeros(out.shape[0], dtype=torch.bool, device=DEV)
     touched[[5, 70, 80]] = True
     if where == "x":
-        assert torch.equal(out[32:64], plain[32:64]) and torch.equal(out[96:], plain[96:])
+        assert torch.equal(out[~touched], plain[~touched])
     rest = ref[~touched]
     assert (out[~touched].double() - rest).abs().max() <= 1e-5 * rest.abs().max()
     assert bool((out[70] == float("inf")).all()) and bool(torch.isnan(out[80]).all())

@@ -520,3 +520,29 @@ def test_workload4_ragged_box_matches_oracle():
     Eo, Fo = _oracle_EF(sts, kw, el)
     dE, dF = check(o["energy"].detach().cpu(), o["forces"].detach().cpu(), Eo, Fo)
     say(f"  dE/E {dE:.2e}  max|dF|/rms {dF:.2e}")
+
+
+@pytest.mark.parametrize("cp", [True, False])
+@pytest.mark.parametrize("n_passes", [1, 2])
+@pytest.mark.parametrize("where", [0, 3, 5])
+def test_broken_structure_leaves_the_others_of_its_batch(cp, n_passes, where):
+    """A structure with two coincident atoms (NaN directions) has a NaN energy; the others of its batch, whose
+    edges and rows share tiles with it, keep theirs: 1e-6 and 1e-5 for sums whose order follows their place
+    in a tile."""
+    from face_amd import systems
+    from face_amd.neighbors import build_graph
+    say("broken structure", cp, n_passes, where)
+    good = systems.molecules(6, np.random.default_rng(3))
+    bad = dict(good[where], pos=np.array(good[where]["pos"]))
+    bad["pos"][4] = bad["pos"][3]
+    kw = dict(systems.FLAGSHIP, C=64, B=16, K=32, rc=4.5, cp=cp, n_passes=n_passes)
+    m = product_model(kw, [1, 6, 8])
+    n = np.cumsum([0] + [len(s["pos"]) for s in good])
+    want = m(build_graph(good, kw["rc"]))
+    got = m(build_graph(good[:where] + [bad] + good[where + 1:], kw["rc"]))
+    assert torch.isnan(got["energy"][where])
+    rms = want["forces"].pow(2).mean().sqrt()
+    for k in range(6):
+        if k != where:
+            assert abs(got["energy"][k] - want["energy"][k]) <= 1e-6 * abs(want["energy"][k])
+            assert ((got["forces"] - want["forces"])[n[k]:n[k + 1]].abs() <= 1e-5 * rms).all()
